@@ -136,11 +136,11 @@ constexpr int NT = 512;
 constexpr int NGRP = NT / 16;     // 32 groups
 constexpr int RK = 8;             // knots per group
 constexpr int KNOTS = NGRP * RK;  // 256
-constexpr int MAXI = 8;
+constexpr int MAXI = 8;  // instances per bin (act is read as two 16-byte words)
 
 // A block slot: rotated row element n of lane i at ((n >> 1) * 16 + i) * 2 +
 // (n & 1), read as 8 x 64-bit words (each 16-lane read covers the 32 banks
-// once); lanes 14, 15 read zeros (never written).
+// once); lanes 14, 15 hold zeros.
 constexpr int SLOT = 256;
 
 struct SplitShared {
@@ -148,12 +148,12 @@ struct SplitShared {
   float K1[NGRP * SLOT];     // rows of L^_{8g+1}^T
   float K2[NGRP * SLOT];     // rows of L^_{8g+2}^T
   float K8[NGRP * SLOT];     // rows of L^_{8g+8}^T
-  float zb[NGRP * 2 * 16];   // staged vector element of each group's first and last knot
+  float zb[NGRP * 2 * 16 + 16];  // staged vector element of each group's first and last knot, then zeros
   float red[2][MAXI][NGRP];  // dot-product partials: one per group, by instance and group
-  uint32_t nlive;            // instances of the bin still iterating
+  uint32_t act[MAXI];        // by instance of the bin: 1 while it iterates
 };
-constexpr uint32_t SPLIT_CLEAR4 = (uint32_t)(offsetof(SplitShared, nlive) / 16);
-static_assert(offsetof(SplitShared, nlive) % 16 == 0, "slots, zb and red are cleared as one float4 range");
+constexpr uint32_t SPLIT_CLEAR4 = (uint32_t)(sizeof(SplitShared) / 16);
+static_assert(sizeof(SplitShared) % 16 == 0 && offsetof(SplitShared, act) % 16 == 0, "cleared and read as 16-byte words");
 
 __device__ __forceinline__ void write_slot(float *Sl, uint32_t i, const float (&M)[16]) {
   float2 *s2 = reinterpret_cast<float2 *>(Sl) + i;
@@ -171,6 +171,10 @@ __device__ __forceinline__ void read_slot(float (&M)[16], const float *Sl, uint3
   }
 }
 
+// a condition that has the same value in every lane of the wave, in a scalar
+// register (a branch on it leaves EXEC alone)
+__device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
+
 // total of the 16 lanes of each row, in every lane of the row (fixed order;
 // each step adds two values in either order, so the lanes agree bitwise)
 __device__ __forceinline__ float row_total(float v) {
@@ -181,32 +185,44 @@ __device__ __forceinline__ float row_total(float v) {
   return v;
 }
 
-__device__ __forceinline__ float ror1(float v) { return dpp_f<0x121>(v); }
-
 // (M_k^T x_k)_i for three blocks with rotated rows M_k: sum_n ror_n(m_n),
 // m_n = M[(16 - n) & 15] x, in Horner form m_0 + ror_1(m_1 + ror_1(m_2 + ...
 // + ror_1(m_15))): 16 products and 15 row_ror:1 additions per block, the
-// three chains interleaved
+// three chains interleaved.  A DPP instruction needs two wait states after
+// the VALU write of what it reads; per step the three products come first,
+// then the three additions, so the distances are there without an s_nop
+// (the compiler's order, product and addition of one chain back to back,
+// put one ahead of each of the 45 additions: 8.3 clocks an instruction of a
+// lone wave against 4.7).
+#define MPC_HSTEP(m0, m1, m2)                                                                           \
+  "v_mul_f32 %3, %" #m0 ", %6\n"                                                                        \
+  "v_mul_f32 %4, %" #m1 ", %7\n"                                                                        \
+  "v_mul_f32 %5, %" #m2 ", %8\n"                                                                        \
+  "v_add_f32_dpp %0, %0, %3 row_ror:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"                        \
+  "v_add_f32_dpp %1, %1, %4 row_ror:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"                        \
+  "v_add_f32_dpp %2, %2, %5 row_ror:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define MPC_HORNER3(k0, k1, k2)                                                                         \
+  asm(MPC_HSTEP(9, 10, 11) MPC_HSTEP(12, 13, 14) MPC_HSTEP(15, 16, 17)                                  \
+      : "+v"(a0), "+v"(a1), "+v"(a2), "=&v"(t0), "=&v"(t1), "=&v"(t2)                                   \
+      : "v"(x0), "v"(x1), "v"(x2), "v"(M0[k0]), "v"(M1[k0]), "v"(M2[k0]), "v"(M0[k1]), "v"(M1[k1]),     \
+        "v"(M2[k1]), "v"(M0[k2]), "v"(M1[k2]), "v"(M2[k2]))
 __device__ __forceinline__ void rot_mtv3(const float (&M0)[16], float x0, const float (&M1)[16], float x1,
                                          const float (&M2)[16], float x2, float &c0, float &c1, float &c2) {
-  // separate products: a fused multiply-add would take the rotated sum as
-  // its addend, which DPP cannot supply (it rotates the first source only)
-#pragma clang fp contract(off)
-  float a0 = M0[1] * x0, a1 = M1[1] * x1, a2 = M2[1] * x2;
-#pragma unroll
-  for (int n = 14; n >= 0; --n) {
-    const int k = (16 - n) & 15;
-    a0 = ror1(a0) + M0[k] * x0;
-    a1 = ror1(a1) + M1[k] * x1;
-    a2 = ror1(a2) + M2[k] * x2;
-  }
+  float a0 = M0[1] * x0, a1 = M1[1] * x1, a2 = M2[1] * x2, t0, t1, t2;
+  MPC_HORNER3(2, 3, 4);
+  MPC_HORNER3(5, 6, 7);
+  MPC_HORNER3(8, 9, 10);
+  MPC_HORNER3(11, 12, 13);
+  MPC_HORNER3(14, 15, 0);
   c0 = a0;
   c1 = a1;
   c2 = a2;
 }
+#undef MPC_HORNER3
+#undef MPC_HSTEP
 
 // Four / five interleaved accumulations a_k += sum_{n=1..15} M_k[n] * ror_n(x_k),
-// three terms per asm statement; one s_nop 4 ahead of the first (the wait
+// three terms per asm statement; an s_nop ahead of the first (the two wait
 // states between a VALU write of x_k and its DPP read)
 #define MPC_TERM(n, acc, x, m) \
   "v_fmac_f32_dpp %" #acc ", %" #x ", %" #m " row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
@@ -219,7 +235,7 @@ __device__ __forceinline__ void rot_mtv3(const float (&M0)[16], float x0, const 
 __device__ __forceinline__ void rot_fma15x4(float &a, float xa, const float (&Ma)[16], float &b, float xb,
                                             const float (&Mb)[16], float &c, float xc, const float (&Mc)[16],
                                             float &e, float xe, const float (&Me)[16]) {
-  MPC_B4("s_nop 4\n", 1, 2, 3);
+  MPC_B4("s_nop 1\n", 1, 2, 3);
   MPC_B4("", 4, 5, 6);
   MPC_B4("", 7, 8, 9);
   MPC_B4("", 10, 11, 12);
@@ -239,7 +255,7 @@ __device__ __forceinline__ void rot_fma15x5(float &a, float xa, const float (&Ma
                                             const float (&Mb)[16], float &c, float xc, const float (&Mc)[16],
                                             float &e, float xe, const float (&Me)[16], float &f, float xf,
                                             const float (&Mf)[16]) {
-  MPC_B5("s_nop 4\n", 1, 2, 3);
+  MPC_B5("s_nop 1\n", 1, 2, 3);
   MPC_B5("", 4, 5, 6);
   MPC_B5("", 7, 8, 9);
   MPC_B5("", 10, 11, 12);
@@ -249,16 +265,43 @@ __device__ __forceinline__ void rot_fma15x5(float &a, float xa, const float (&Ma
 #undef MPC_T5
 #undef MPC_TERM
 
-// rotated rows of the column-major 14 x 14 block Lh (T = true: of its
-// transpose); zeros where has is false and in lanes 14, 15
-template <bool T = false>
-__device__ __forceinline__ void load_lrows(float (&Lr)[16], bool has, uint32_t i, uint32_t d,
-                                           const float *__restrict__ Lh) {
-  const bool row = has && i < (uint32_t)NX;
+// base[off], with a 32-bit byte offset from a uniform base (one address
+// register; an instance's rows are at most 256 * 2352 bytes)
+__device__ __forceinline__ float at(const float *__restrict__ base, uint32_t off) {
+  return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + 4u * off);
+}
+
+// element offsets of the rotated rows of a block of row b0
+__device__ __forceinline__ void block_offsets(uint32_t (&off)[16], uint32_t b0, uint32_t i, uint32_t d) {
 #pragma unroll
   for (int n = 0; n < 16; ++n) {
     const uint32_t j = (i + (uint32_t)n * d) & 15u;
-    Lr[n] = row && j < (uint32_t)NX ? Lh[T ? j + NX * i : i + NX * j] : 0.f;
+    off[n] = S_STRIDE * b0 + i + (j < (uint32_t)NX ? NX * j : 0u);
+  }
+}
+
+// Rotated rows of a column-major 14 x 14 block (its element (i, src(i, n)) at
+// base + off[n], i = the lane), zeros where ok is false; one branch for the
+// block's 16 reads, none between them.
+__device__ __forceinline__ void load_lrows(float (&Lr)[16], bool ok, uint32_t i, uint32_t d, const float *__restrict__ base,
+                                           const uint32_t (&off)[16]) {
+#pragma unroll
+  for (int n = 0; n < 16; ++n) Lr[n] = 0.f;
+  if (ok) {
+#pragma unroll
+    for (int n = 0; n < 16; ++n) Lr[n] = at(base, off[n]);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) Lr[n] = ((i + (uint32_t)n * d) & 15u) < (uint32_t)NX ? Lr[n] : 0.f;
+  }
+}
+
+// the slot of the block's transpose from its rotated rows: the element of
+// lane i, rotation n is the one of lane src(i, n), rotation -n, there
+__device__ __forceinline__ void write_slot_t(float *Sl, uint32_t i, uint32_t d, const float (&M)[16]) {
+#pragma unroll
+  for (int n = 0; n < 16; ++n) {
+    const uint32_t m = (16u - (uint32_t)n) & 15u, c = (i + (uint32_t)n * d) & 15u;
+    Sl[((m >> 1) * 16u + c) * 2u + (m & 1u)] = M[n];
   }
 }
 
@@ -271,19 +314,21 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   SplitShared &sh = *reinterpret_cast<SplitShared *>(smem_raw);
   const uint32_t tid = threadIdx.x, bin = blockIdx.x;
   const uint32_t g = tid >> 4, i = tid & 15u;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t d = ror_step(tid);
   {
     float4 *z4 = reinterpret_cast<float4 *>(smem_raw);
     for (uint32_t idx = tid; idx < SPLIT_CLEAR4; idx += NT) z4[idx] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tid == 0) sh.nlive = 0u;
   }
-  // my instance in this bin (items: {inst, first group, groups, -})
+  // the wave's instance in this bin (items: {inst, first group, groups, -};
+  // an instance owns whole waves, so everything about it is uniform over the
+  // wave and stays in scalar registers)
   const uint32_t i0 = bin_off[bin], ni = bin_off[bin + 1] - i0;
   int slot = -1;
   uint32_t inst = 0, g0 = 0;
   for (uint32_t jx = 0; jx < ni; ++jx) {
     const uint4 it = items[i0 + jx];
-    if (g >= it.y && g < it.y + it.z) {
+    if (4u * w >= it.y && 4u * w < it.y + it.z) {
       slot = (int)jx;
       inst = it.x;
       g0 = it.y;
@@ -292,77 +337,103 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   const bool mine = slot >= 0;
   const uint32_t N = mine ? inst_len(b, inst) : 0u;
   const uint32_t K0 = mine ? inst_first(b, inst) : 0u;
-  const bool live = mine && !(status && !(status[inst] & ST_ACTIVE));
+  const bool live = uniform(mine && !(status && !(status[inst] & ST_ACTIVE)));
   const uint32_t cap = pcg_cap(max_iter, N);
   const uint32_t lg = g - g0;
-  const bool leader = lg == 0 && i == 0 && mine;  // the instance's first lane
   const bool lane_ok = i < (uint32_t)NX;
   __syncthreads();  // LDS cleared
 
   // ---- load: lambda^ = W^-1 lambda by back substitution (W upper
-  // triangular; each solved element broadcast to the group by DPP, every
-  // lane active) and gamma^, then the blocks (fewer values live at once)
+  // triangular) and gamma^, then the blocks (fewer values live at once).
+  // The reads of a wave that has no instance, or of knots past its end, go
+  // to a valid row (clamped) and are replaced by zeros.
   const uint32_t b0 = lg * RK;
-  float lam[RK], r[RK], p[RK], y[RK], gh[RK];  // z = -r is not stored
+  const float *Pw = Ps + (size_t)S_STRIDE * K0;  // the instance's rows
+  const uint32_t klast = N ? N - 1u : 0u, il = lane_ok ? i : 0u;
+  auto knot = [&](uint32_t t) { return b0 + t < klast ? b0 + t : klast; };
+  float lam[RK], r[RK], p[RK], y[RK];  // z = -r is not stored; r starts as gamma^
+  bool any = false;
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
-    const uint32_t bk = b0 + (uint32_t)t;
-    const bool has = live && bk < N && lane_ok;
-    const float *Wr = Ps + (size_t)S_STRIDE * (K0 + (has ? bk : 0u)) + NXX;
-    float wrow[NX];
+    const bool has = live && b0 + (uint32_t)t < N && lane_ok;
+    const float l = lambda[(size_t)NX * (K0 + knot(t)) + il], h = ghat[(size_t)NX * (K0 + knot(t)) + il];
+    lam[t] = has ? l : 0.f;
+    r[t] = has ? h : 0.f;
+    any = any || lam[t] != 0.f;
+  }
+  // A start from lambda = 0 has lambda^ = 0.  Otherwise the group's eight
+  // back substitutions run in lockstep: in step k lane t of the row takes
+  // knot t's pivot quotient (from lane k of that knot, by DPP), so one
+  // division serves all eight, and each goes back to its row by DPP.
+  if (__builtin_amdgcn_ballot_w64(any) != 0) {
+    float wr[RK][NX], den[NX];
+    const uint32_t td = i & (RK - 1);
 #pragma unroll
-    for (int c = 0; c < NX; ++c) wrow[c] = has ? Wr[i + NX * c] : 0.f;
-    float acc = has ? lambda[(size_t)NX * (K0 + bk) + i] : 0.f;
-    float lh = 0.f;
+    for (int k = 0; k < NX; ++k) {
+      const float v = at(Pw, S_STRIDE * knot(td) + NXX + k + NX * k);
+      den[k] = live ? v : 1.f;
+    }
+#pragma unroll
+    for (int t = 0; t < RK; ++t)
+#pragma unroll
+      for (int c = 0; c < NX; ++c) wr[t][c] = at(Pw, S_STRIDE * knot(t) + NXX + il + NX * c);
+    float lh[RK];
+#pragma unroll
+    for (int t = 0; t < RK; ++t) lh[t] = 0.f;
 #pragma unroll
     for (int k = NX - 1; k >= 0; --k) {
-      const float xk = bcast_dyn16<true>(acc / wrow[k], k);
-      lh = (int)i == k ? xk : lh;
-      asm volatile("" : "+v"(lh));  // select now, not after the last step
-      acc -= wrow[k] * xk;
-    }
-    lam[t] = has ? lh : 0.f;
-    gh[t] = has ? ghat[(size_t)NX * (K0 + bk) + i] : 0.f;
-  }
-  float *R0g = sh.R0 + g * SLOT, *K1g = sh.K1 + g * SLOT, *K2g = sh.K2 + g * SLOT, *K8g = sh.K8 + g * SLOT;
-  auto blk = [&](uint32_t t, bool &has) {
-    const uint32_t bk = b0 + t;
-    has = live && bk < N && bk > 0;  // L^_0 = 0
-    return Ps + (size_t)S_STRIDE * (K0 + (has ? bk : 0u));
-  };
-  {
-    const uint32_t ts[4] = {0u, 1u, 2u, (uint32_t)RK};
-    float *dst[4] = {R0g, K1g, K2g, K8g};
+      float num = 0.f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      bool has;
-      const float *Pr = blk(ts[u], has);
-      float Ls[16];
-      if (u == 0)
-        load_lrows(Ls, has, i, d, Pr);
-      else
-        load_lrows<true>(Ls, has, i, d, Pr);
-      if (lane_ok) write_slot(dst[u], i, Ls);
-      asm volatile("" ::: "memory");  // store now: Ls need not stay live across the other loads
+      for (int t = 0; t < RK; ++t) {
+        const float v = bcast_dyn16<true>(lam[t], k);
+        num = td == (uint32_t)t ? v : num;
+      }
+      const float quo = num / den[k];
+#pragma unroll
+      for (int t = 0; t < RK; ++t) {
+        const float xk = bcast_dyn16<true>(quo, t);
+        lh[t] = (int)i == k ? xk : lh[t];
+        lam[t] -= wr[t][k] * xk;
+      }
+      pin(lh);
+      pin(lam);
     }
+#pragma unroll
+    for (int t = 0; t < RK; ++t) lam[t] = live && b0 + (uint32_t)t < N && lane_ok ? lh[t] : 0.f;
   }
+  asm volatile("" ::: "memory");  // the block reads below stay behind the rows of W
+  float *R0g = sh.R0 + g * SLOT, *K1g = sh.K1 + g * SLOT, *K2g = sh.K2 + g * SLOT, *K8g = sh.K8 + g * SLOT;
+  auto ok = [&](uint32_t t) { return live && lane_ok && b0 + t < N && b0 + t > 0; };  // L^_0 = 0
+  uint32_t roff[16];
+  block_offsets(roff, b0, i, d);
+  // Only rows are read (a group's 16 reads of a block touch its 784 bytes
+  // once each; reading the transposes by lanes 56 bytes apart took 36 k
+  // clocks of address processing for a full workgroup); the transposes are
+  // written from them, through the slot of L^_0 where they end in registers.
   float Lr[RK - 1][16];  // Lr[t - 1]: rows of L^_t, t = 1 .. 7
   float Kr[2][16];       // Kr[t - 3]: rows of L^_t^T, t = 3, 4
 #pragma unroll
-  for (int t = 1; t < RK; ++t) {
-    bool has;
-    const float *Pr = blk((uint32_t)t, has);
-    load_lrows(Lr[t - 1], has, i, d, Pr);
-  }
+  for (int t = 1; t < RK; ++t) load_lrows(Lr[t - 1], ok(t), i, d, Pw + S_STRIDE * t, roff);
+  write_slot_t(K1g, i, d, Lr[0]);
+  write_slot_t(K2g, i, d, Lr[1]);
 #pragma unroll
   for (int t = 3; t < 5; ++t) {
-    bool has;
-    const float *Pr = blk((uint32_t)t, has);
-    load_lrows<true>(Kr[t - 3], has, i, d, Pr);
+    write_slot_t(R0g, i, d, Lr[t - 1]);
+    wave_sync();
+    read_slot(Kr[t - 3], R0g, i);
+    wave_sync();
   }
-  const bool in_m = lg > 0, in_p = b0 + RK < N;
-  // zb: [group][first, last knot][lane]
+  {
+    float Ls[16];
+    load_lrows(Ls, ok(RK), i, d, Pw + S_STRIDE * RK, roff);
+    write_slot_t(K8g, i, d, Ls);
+    load_lrows(Ls, ok(0), i, d, Pw, roff);
+    write_slot(R0g, i, Ls);
+  }
+  // zb: [group][first, last knot][lane]; a group without a neighbour reads
+  // the zero entries behind the last group's
   float *zbg = sh.zb + g * 32 + i;
+  const float *zm_src = lg > 0 ? zbg - 16 : sh.zb + NGRP * 32 + i, *zp_src = b0 + RK < N ? zbg + 32 : sh.zb + NGRP * 32 + i;
   auto stage = [&](const float (&v)[RK]) {
     zbg[0] = v[0];
     zbg[16] = v[RK - 1];
@@ -370,10 +441,6 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   auto stage_neg = [&](const float (&v)[RK]) {
     zbg[0] = -v[0];
     zbg[16] = -v[RK - 1];
-  };
-  auto neighbours = [&](float &vm, float &vp) {
-    vm = in_m ? zbg[-16] : 0.f;
-    vp = in_p ? zbg[32] : 0.f;
   };
   // y = S^ x: y_t = -x_t + L^_t x_{t-1} + L^_{t+1}^T x_{t+1}; xm / xp: the
   // elements of knots 8lg - 1 and 8lg + 8.  Lanes 14, 15 of every block row
@@ -414,7 +481,7 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   float *redg = &sh.red[0][mine ? slot : 0][lg & (NGRP - 1)];
   auto post = [&](int k, float part) {
     const float v = row_total(part);
-    if (i == 0) redg[k * MAXI * NGRP] = v;
+    redg[k * MAXI * NGRP] = v;  // the row's lanes write the same value
   };
   const float2 *red2 = reinterpret_cast<const float2 *>(&sh.red[0][mine ? slot : 0][0]) + i;
   auto total = [&](int k) {
@@ -422,39 +489,29 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
     return row_total(v.x + v.y);
   };
   stage(lam);
+  // an instance's act word, set here and cleared when it stops (its lanes all
+  // write the same, between the second barrier of its last iteration and the
+  // first of the next).  `run` is the same in every wave of an instance; a
+  // wave that runs knows that some instance does, and the others read the
+  // words between the two barriers, where they do not change, so all waves
+  // leave the loop in the same iteration.  The loop has no branch on a value
+  // that differs between lanes: one would put every branch of it on EXEC
+  // masks (several hundred clocks of mask bookkeeping per iteration).
+  bool run = live;
+  if (run) sh.act[slot] = 1u;
   __syncthreads();
-  float pm, pp;
-  neighbours(pm, pp);
+  float pm = *zm_src, pp = *zp_src;
 
-  // ---- prologue: r = gamma^ - S^ lambda^, z = -r, p = z, eta = r.z
-  smv(lam, pm, pp);
-  float part = 0.f;
+  // The first pass is the prologue, through the same code (one copy of the
+  // products): p = lambda^, r = gamma^ - S^ lambda^ (alpha = 1, lambda^ kept),
+  // z = -r, then p = z (beta = 0) and eta = r.z; the others are the
+  // iterations.
 #pragma unroll
-  for (int t = 0; t < RK; ++t) {
-    r[t] = lane_ok ? gh[t] - y[t] : 0.f;
-    part -= r[t] * r[t];
-  }
-  __syncthreads();  // every neighbour lambda read before zb is reused
-  post(1, part);
-  stage_neg(r);
-  __syncthreads();
-  float eta = total(1);
-  neighbours(pm, pp);
-#pragma unroll
-  for (int t = 0; t < RK; ++t) p[t] = -r[t];
-  uint32_t it = 0;
-  // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
-  const float tol_i = tol < 0.f ? fmaxf(-tol * fabsf(eta), FLT_MIN) : tol;
-  bool conv = !live || fabsf(eta) < tol_i;
-  float eta_last = eta;
-  // the bin's count of iterating instances: each instance's first lane adds
-  // itself here and leaves when it stops (between the second barrier of its
-  // last iteration and the first of the next), so after the first barrier of
-  // an iteration every wave sees the same count
-  if (leader && !conv && cap > 0) atomicAdd(&sh.nlive, 1u);
-
+  for (int t = 0; t < RK; ++t) p[t] = lam[t];
+  uint32_t it = ~0u;  // the first pass is not counted
+  float eta = 0.f, tol_i = tol;
+  bool conv = !live, first = true;
   for (;;) {
-    const bool run = live && !conv && it < cap;  // uniform over the instance's waves
     if (run) {
       smv(p, pm, pp);
       float pyp = 0.f;
@@ -463,55 +520,59 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
       post(0, pyp);
     }
     __syncthreads();
-    if (sh.nlive == 0u) break;
+    float alpha = 0.f;
     if (run) {
-      const float alpha = eta / total(0);
+      const float quo = eta / total(0);
+      alpha = first ? 1.f : quo;
       float rz = 0.f;
 #pragma unroll
       for (int t = 0; t < RK; ++t) {
-        lam[t] += alpha * p[t];
         r[t] -= alpha * y[t];
         rz -= r[t] * r[t];
       }
       stage_neg(r);
       post(1, rz);
+    } else {
+      const uint4 a0 = reinterpret_cast<const uint4 *>(sh.act)[0], a1 = reinterpret_cast<const uint4 *>(sh.act)[1];
+      if (uniform((a0.x | a0.y | a0.z | a0.w | a1.x | a1.y | a1.z | a1.w) == 0u)) break;
     }
     __syncthreads();
     if (run) {
-      float zm, zp;
-      neighbours(zm, zp);
-      const float eta_new = total(1);
-      eta_last = eta_new;
-      ++it;
-      conv = fabsf(eta_new) < tol_i;
-      if (leader && (conv || it >= cap)) atomicSub(&sh.nlive, 1u);
-      if (!conv) {
-        const float beta = eta_new / eta;
-        eta = eta_new;
+      const float zm = *zm_src, zp = *zp_src, eta_new = total(1);
+      const float alpha_l = first ? 0.f : alpha;
 #pragma unroll
-        for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], -r[t]);
-        pm = fmaf(beta, pm, zm);
-        pp = fmaf(beta, pp, zp);
-      }
+      for (int t = 0; t < RK; ++t) lam[t] += alpha_l * p[t];
+      // taken in the last iteration too (p is not used after it): no branch
+      // around the next direction
+      const float quo = eta_new / eta, beta = first ? 0.f : quo;
+      eta = eta_new;
+#pragma unroll
+      for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], -r[t]);
+      pm = fmaf(beta, pm, zm);
+      pp = fmaf(beta, pp, zp);
+      // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
+      if (first && tol < 0.f) tol_i = fmaxf(-tol * fabsf(eta), FLT_MIN);
+      ++it;
+      first = false;
+      conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
+      run = !conv && it < cap;
+      if (!run) sh.act[slot] = 0u;
     }
   }
 
   if (!live) return;
-  // lambda = W lambda^, two knots at a time
+  // lambda = W lambda^, two knots at a time (the offsets formed again, not
+  // held through the iterations)
+  uint32_t ie = i;
+  asm volatile("" : "+v"(ie));
+  uint32_t woff[16];
+  block_offsets(woff, b0, ie, d);
 #pragma unroll
   for (int t = 0; t < RK; t += 2) {
     float Wr[2][16];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const uint32_t bk = b0 + (uint32_t)(t + u);
-      const bool has = bk < N && lane_ok;
-      const float *Wb = Ps + (size_t)S_STRIDE * (K0 + (bk < N ? bk : 0u)) + NXX;
-#pragma unroll
-      for (int n = 0; n < 16; ++n) {
-        const uint32_t j = (i + (uint32_t)n * d) & 15u;
-        Wr[u][n] = has && j < (uint32_t)NX ? Wb[i + NX * j] : 0.f;
-      }
-    }
+    for (int u = 0; u < 2; ++u)
+      load_lrows(Wr[u], lane_ok && b0 + (uint32_t)(t + u) < N, i, d, Pw + S_STRIDE * (t + u) + NXX, woff);
     float va, vb;
     rot_mv2(Wr[0], lam[t], va, Wr[1], lam[t + 1], vb);
     if (b0 + t < N && lane_ok) lambda[(size_t)NX * (K0 + b0 + t) + i] = va;
@@ -520,7 +581,7 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   if (lg == 0 && i == 0) {
     if (iters_out) iters_out[inst] = it;
     if (flag_out) flag_out[inst] = conv ? 0u : 1u;
-    if (eta_out) eta_out[inst] = fabsf(eta_last);
+    if (eta_out) eta_out[inst] = fabsf(eta);
   }
 }
 

@@ -489,41 +489,35 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
     return row_total(v.x + v.y);
   };
   stage(lam);
-  // an instance's act word, set here and cleared when it stops (its lanes all
+  // an instance's act word: set here, cleared when it stops (its lanes all
   // write the same, between the second barrier of its last iteration and the
-  // first of the next).  `run` is the same in every wave of an instance; a
-  // wave that runs knows that some instance does, and the others read the
-  // words between the two barriers, where they do not change, so all waves
-  // leave the loop in the same iteration.  The loop has no branch on a value
-  // that differs between lanes: one would put every branch of it on EXEC
-  // masks (several hundred clocks of mask bookkeeping per iteration).
-  bool run = live;
-  if (run) sh.act[slot] = 1u;
+  // first of the next)
+  if (live) sh.act[slot] = 1u;
   __syncthreads();
   float pm = *zm_src, pp = *zp_src;
 
   // The first pass is the prologue, through the same code (one copy of the
   // products): p = lambda^, r = gamma^ - S^ lambda^ (alpha = 1, lambda^ kept),
   // z = -r, then p = z (beta = 0) and eta = r.z; the others are the
-  // iterations.
+  // iterations.  The loop has no branch on a value that differs between
+  // lanes (one would put every branch of it on EXEC masks, several hundred
+  // clocks of mask bookkeeping per iteration) and none but its own for a wave
+  // that iterates.
 #pragma unroll
   for (int t = 0; t < RK; ++t) p[t] = lam[t];
   uint32_t it = ~0u;  // the first pass is not counted
   float eta = 0.f, tol_i = tol;
-  bool conv = !live, first = true;
-  for (;;) {
-    if (run) {
+  bool conv = !live;
+  if (live) {
+    bool first = true, run;
+    do {
       smv(p, pm, pp);
       float pyp = 0.f;
 #pragma unroll
       for (int t = 0; t < RK; ++t) pyp += p[t] * y[t];
       post(0, pyp);
-    }
-    __syncthreads();
-    float alpha = 0.f;
-    if (run) {
-      const float quo = eta / total(0);
-      alpha = first ? 1.f : quo;
+      __syncthreads();
+      const float quo = eta / total(0), alpha = first ? 1.f : quo;
       float rz = 0.f;
 #pragma unroll
       for (int t = 0; t < RK; ++t) {
@@ -532,19 +526,13 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
       }
       stage_neg(r);
       post(1, rz);
-    } else {
-      const uint4 a0 = reinterpret_cast<const uint4 *>(sh.act)[0], a1 = reinterpret_cast<const uint4 *>(sh.act)[1];
-      if (uniform((a0.x | a0.y | a0.z | a0.w | a1.x | a1.y | a1.z | a1.w) == 0u)) break;
-    }
-    __syncthreads();
-    if (run) {
+      __syncthreads();
       const float zm = *zm_src, zp = *zp_src, eta_new = total(1);
       const float alpha_l = first ? 0.f : alpha;
 #pragma unroll
       for (int t = 0; t < RK; ++t) lam[t] += alpha_l * p[t];
-      // taken in the last iteration too (p is not used after it): no branch
-      // around the next direction
-      const float quo = eta_new / eta, beta = first ? 0.f : quo;
+      // taken in the last iteration too (p is not used after it)
+      const float quo_b = eta_new / eta, beta = first ? 0.f : quo_b;
       eta = eta_new;
 #pragma unroll
       for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], -r[t]);
@@ -556,8 +544,18 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
       first = false;
       conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
       run = !conv && it < cap;
-      if (!run) sh.act[slot] = 0u;
-    }
+    } while (run);
+    sh.act[slot] = 0u;
+  }
+  // Waves that iterate no more (or have no instance) keep the others'
+  // barriers until no instance of the bin iterates.  They read the act words
+  // between the two barriers, where those do not change, so all leave in the
+  // same round.
+  for (;;) {
+    __syncthreads();
+    const uint4 a0 = reinterpret_cast<const uint4 *>(sh.act)[0], a1 = reinterpret_cast<const uint4 *>(sh.act)[1];
+    if (uniform((a0.x | a0.y | a0.z | a0.w | a1.x | a1.y | a1.z | a1.w) == 0u)) break;
+    __syncthreads();
   }
 
   if (!live) return;

@@ -49,6 +49,7 @@ struct mpc_handle {
   float *pcg_eta = nullptr;  // [B] |r^T Pinv r| at each instance's last PCG exit test
   unsigned long long *t0 = nullptr;  // [1] device clock at the start of a batched solve
   double clock_ticks_per_us = 0.0;   // device wall clock rate
+  uint32_t n_cu = 0;                 // compute units of the device
   uint32_t *knot_inst = nullptr, *inst_k0 = nullptr;
   // PCG dispatch of a batch: bins of small instances (resident kernel) and
   // the list of instances beyond the teams (streaming kernel)
@@ -310,14 +311,16 @@ int mpc_create(const mpc_config *cfg, mpc_handle **out) {
   if (!h) return MPC_ERR_ARG;
   h->cfg = *cfg;
   weights_from_config(h);
-  int clock_khz = 0;
+  int clock_khz = 0, n_cu = 0;
   if (hipGetDevice(&h->device) != hipSuccess ||
       hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, h->device) != hipSuccess ||
-      clock_khz <= 0) {
+      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess ||
+      clock_khz <= 0 || n_cu <= 0) {
     delete h;
     return MPC_ERR_HIP;
   }
   h->clock_ticks_per_us = clock_khz * 1e-3;
+  h->n_cu = (uint32_t)n_cu;
   const size_t T = cfg->max_total_knots, B = cfg->max_instances;
   auto alloc = [&](void **p, size_t bytes) { return hipMalloc(p, bytes) == hipSuccess; };
   bool ok = alloc((void **)&h->G, sizeof(float) * G_STRIDE * T) &&
@@ -727,7 +730,22 @@ static int build_pcg_plan(mpc_handle *h) {
   if (h->split_ok) {
     std::vector<uint32_t> all(n_inst);
     for (uint32_t i = 0; i < n_inst; ++i) all[i] = i;
-    const std::vector<BinB> sb = pack(all, pcg_split_bin_groups(), pcg_split_groups);
+    // A bin runs as long as its longest instance, and an iteration of a
+    // workgroup takes less the fewer of its waves work (173 iterations: 186 us
+    // with one, 215 with four, 327 with eight).  So while the bins fit the
+    // device at once they are kept as empty as that allows: 4, 8 or 16 groups
+    // instead of 32 per bin (instances of more groups have their own).
+    // Every packing is the same solve, bitwise.  256 instances of N = 64 (256
+    // bins instead of 64): layer and adjoint 5.9 -> 4.3 ms; 16 of N = 5..97:
+    // two SQP iterations 765 -> 533 us.
+    std::vector<BinB> sb;
+    for (uint32_t cap = 4; cap <= pcg_split_bin_groups(); cap *= 2) {
+      double fill = 0.0;  // a lower bound on the bins, before packing them
+      for (uint32_t i = 0; i < n_inst; ++i) fill += std::min(1.0, (double)pcg_split_groups(horizons[i]) / cap);
+      if (cap < pcg_split_bin_groups() && fill > (double)h->n_cu) continue;
+      sb = pack(all, cap, pcg_split_groups);
+      if (sb.size() <= h->n_cu) break;
+    }
     std::vector<uint4> sitems;
     std::vector<uint32_t> soff(1, 0);
     for (auto &bb : sb) {

@@ -16,13 +16,10 @@
 // (1e-4..1e-2 relative on these systems); each step multiplies the error by
 // about that factor, down to the fp32 storage of lambda.
 //
-// Mapping: one 16-lane group per instance, 4 groups per 64-lane workgroup
-// (one wave), instances longest first.  The factorisation stages B_b and E_b
-// in LDS (every group runs the wave's longest trip count; wave-level ordering
-// suffices); the solve sweeps keep one vector element per lane and broadcast the
-// vector inside the group by ds_swizzle, so they need no LDS and no barrier,
-// and each loads the next knot's factor rows ahead.  The residual is formed
-// for all knots of all instances at once, one group per knot.
+// Mapping: one wave per instance, instances longest first (few waves, one per
+// SIMD: the sweeps are bound by their dependent chains, so what counts is the
+// instructions and latencies of a step, below).  The residual is formed for
+// all knots of all instances at once, one group per knot.
 //
 // Reference: the QDLDL path of sqpSolve (PCG_SOLVE = 0, toplevel.cuh:160-215,
 // :314-335) solves the same system by a sparse LDL^T on the host.
@@ -38,397 +35,501 @@ namespace {
 constexpr int GROUP = 16;
 constexpr int GROUPS_PER_WG = 4;
 constexpr int WG = GROUP * GROUPS_PER_WG;
-constexpr int BPL = (NXX + GROUP - 1) / GROUP;  // B entries per lane (13)
-
-struct FacLds {
-  float B[NXX];  // B_b (column-major)
-  float E[NXX];  // E_b (column-major)
-};
 
 __device__ __forceinline__ float *slot_E(float *work, size_t row) { return work + (size_t)S_STRIDE * row; }
 __device__ __forceinline__ float *slot_Dinv(float *work, size_t row) { return work + (size_t)S_STRIDE * row + NXX; }
 __device__ __forceinline__ float *slot_z(float *work, size_t row) { return work + (size_t)S_STRIDE * row + 2 * NXX; }
 
-// LDS ordering among the lanes of the (single-wave) workgroup: wave_sync
-// (common.h), which does not wait for outstanding global loads (the next
-// knot's prefetch)
-
-// sum_m w[m] v_m, v_m the value v of lane m of the group (m < 14), in order
-template <int... M>
-__device__ __forceinline__ float bdot_seq(const float (&w)[NX], float v, std::integer_sequence<int, M...>) {
-  float s = 0.f;
-  ((s += w[M] * bcast16<M>(v)), ...);
-  return s;
-}
-__device__ __forceinline__ float bdot(const float (&w)[NX], float v) {
-  return bdot_seq(w, v, std::make_integer_sequence<int, NX>{});
-}
-
-// instance of list slot `slot` and the workgroup's longest horizon
+// the instance of a wave
 struct Pick {
-  uint32_t inst, K0, N, Nmax;
+  uint32_t inst, K0, N;
   bool live;
 };
 
-__device__ __forceinline__ Pick pick_instance(const Batch &b, const uint32_t *order, uint32_t n_list,
-                                              const uint32_t *status, uint32_t slot) {
+__device__ __forceinline__ Pick pick_instance(const Batch &b, const uint32_t *order, const uint32_t *status,
+                                              uint32_t slot) {
   Pick p;
-  const bool in_list = slot < n_list;
-  const uint32_t s = in_list ? slot : n_list - 1;
-  p.inst = order ? order[s] : s;
+  p.inst = order ? order[slot] : slot;
   p.K0 = inst_first(b, p.inst);
   p.N = inst_len(b, p.inst);
-  p.live = in_list && !(status && !(status[p.inst] & ST_ACTIVE));
-  const uint32_t first = (slot / GROUPS_PER_WG) * GROUPS_PER_WG;
-  p.Nmax = inst_len(b, order ? order[first] : first);
+  p.live = !(status && !(status[p.inst] & ST_ACTIVE));
   return p;
 }
 
-// factorisation sweep of one instance: E_b, D_b^-1 into the workspace
-__device__ __forceinline__ void factor(FacLds &L, const float *__restrict__ S, float *__restrict__ work, const Pick &p,
-                                      int lane) {
-  const int j = lane < NX ? lane : NX - 1;
-  float dinv[NX];  // column j of D_{b-1}^-1
-#pragma unroll
-  for (int r = 0; r < NX; ++r) dinv[r] = 0.f;
-  float a_cur[NX], b_cur[BPL], a_nxt[NX], b_nxt[BPL];
-  auto load = [&](float (&a)[NX], float (&bb)[BPL], uint32_t k) {
-    const float *Sr = S + (size_t)S_STRIDE * (p.K0 + k);
-#pragma unroll
-    for (int r = 0; r < NX; ++r) a[r] = -Sr[NXX + r + NX * j];
-#pragma unroll
-    for (int t = 0; t < BPL; ++t) {
-      const int i = lane + GROUP * t;
-      bb[t] = (k > 0 && i < NXX) ? -Sr[i] : 0.f;
-    }
-  };
-  load(a_cur, b_cur, 0);
-  for (uint32_t k = 0; k < p.Nmax; ++k) {
-    const bool on = p.live && k < p.N;
-    load(a_nxt, b_nxt, k + 1 < p.N ? k + 1 : p.N - 1);
-#pragma unroll
-    for (int t = 0; t < BPL; ++t) {
-      const int i = lane + GROUP * t;
-      if (i < NXX) L.B[i] = b_cur[t];
-    }
-    wave_sync();
-    // E_b (column j) = sum_m B(:, m) D_{b-1}^-1(m, j)
-    float e[NX];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) e[r] = 0.f;
-#pragma unroll
-    for (int m = 0; m < NX; ++m) {
-      const float d = dinv[m];
-#pragma unroll
-      for (int r = 0; r < NX; ++r) e[r] += L.B[r + NX * m] * d;
-    }
-    if (lane < NX) {
-#pragma unroll
-      for (int r = 0; r < NX; ++r) L.E[r + NX * lane] = e[r];
-      if (on) {
-        float *w = slot_E(work, p.K0 + k) + NX * lane;
-#pragma unroll
-        for (int r = 0; r < NX; ++r) w[r] = e[r];
-      }
-    }
-    wave_sync();
-    // D_b (column j) = A_b(:, j) - sum_m E(:, m) B(j, m)
-    float a[NX];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) a[r] = a_cur[r];
-#pragma unroll
-    for (int m = 0; m < NX; ++m) {
-      const float bjm = L.B[j + NX * m];
-#pragma unroll
-      for (int r = 0; r < NX; ++r) a[r] -= L.E[r + NX * m] * bjm;
-    }
-    pin(a);
-    gj_inverse<NX>(lane, a, dinv);
-    if (on && lane < NX) {
-      float *w = slot_Dinv(work, p.K0 + k) + NX * lane;
-#pragma unroll
-      for (int r = 0; r < NX; ++r) w[r] = dinv[r];
-    }
-    wave_sync();  // every read of B and E is done before the next knot overwrites them
-#pragma unroll
-    for (int r = 0; r < NX; ++r) a_cur[r] = a_nxt[r];
-#pragma unroll
-    for (int t = 0; t < BPL; ++t) b_cur[t] = b_nxt[t];
-  }
-}
-
-// ---- factorisation with one wave per instance --------------------------------
+// ---- factorisation -----------------------------------------------------------
 // Lane 16 q + j (q = 0..3) holds, for column j of a block, the rows
 // r = 4 t + q (t = 0..3, r < 14): the products and the Gauss-Jordan updates
-// of a column are split over four lanes, each element with the operation
-// sequence of factor() (so E_b and D_b^-1 are bitwise the same), and the
-// 1024-instance batch runs four waves per CU instead of one.  Blocks that
-// every lane reads in full (B_b, E_b, D_{b-1}^-1) go through LDS.
+// of a column are split over four lanes, one row of 16 lanes per quarter.
+// Per knot:
+//   E_b = B_b D_{b-1}^-1: the lane's rows of B_b and its column of D_{b-1}^-1
+//     from LDS (the latter written by the quarters after their inverse);
+//   D_b = A_b - E_b B_b^T: the element E(r, m) is in lane m of the lane's own
+//     row, so the 14 x 4 multiply-adds take it by DPP row_newbcast:m;
+//   D_b^-1 by Gauss-Jordan, 14 pivots.  In step P the updates of the lane's
+//     rows take column P by DPP (in the multiply-add itself), and row P comes
+//     from its quarter by ds_bpermute (about 64 clocks).  Row P + 1 is updated
+//     first and sent; its pivot is read by readlane and inverted between the
+//     updates of the other rows, which cover both latencies.
+// Every element sees the operations of a one-lane-per-column elimination in
+// their order (a product m by m from zero, a pivot after the other).
+// N = 512: 3.4 -> 1.27 us per knot (before: pivot columns by ds_swizzle, a
+// division on the chain, 528 clocks per pivot).
 constexpr int RS = 16;  // LDS row stride of a block (16-byte aligned rows)
-struct FacWaveLds {
-  float B[NX * RS];     // B_b by rows: B(r, c) at c + RS r
-  float E[NX * RS];     // E_b by rows
-  float Dinv[NX * RS];  // D_{b-1}^-1 by columns: (m, j) at m + RS j
+struct alignas(16) FacWaveLds {
+  float B[2][NX * RS + RS];  // B_b by rows: B(r, c) at c + RS r, knots alternating (the last RS: unused lanes' writes)
+  float Dinv[NX * RS];       // D_{b-1}^-1 by columns: (m, j) at m + RS j
 };
 
-__device__ __forceinline__ float lane_value(float v, uint32_t src) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((int)(src << 2), __builtin_bit_cast(int, v)));
+__device__ __forceinline__ float lane_value(float v, uint32_t byte_addr) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((int)byte_addr, __builtin_bit_cast(int, v)));
+}
+template <int l>
+__device__ __forceinline__ float read_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
-template <int P>
-__device__ __forceinline__ void gj_wave_step(uint32_t q, uint32_t j, float (&a)[4], float (&x)[4]) {
-  constexpr uint32_t QP = P & 3, TP = P >> 2;  // owner quarter and slot of row P
-  float pc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) pc[t] = bcast16<P>(a[t]);  // column P, the lane's rows
-  const float piv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a[TP]), 16 * QP + P));
-  const float inv = 1.f / piv;
-  const float ap = lane_value(a[TP], 16u * QP + j) * inv, xp = lane_value(x[TP], 16u * QP + j) * inv;
+// a pivot whose inverse pivot_rest gives as the division does (below)
+__device__ __forceinline__ bool mid_range(float v) {
+  return ((__builtin_bit_cast(uint32_t, v) >> 23) & 255u) - 80u < 95u;  // 2^-47 <= |v| < 2^48
+}
+
+#define MPC_NB " row_newbcast:%c[l] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+// One slot of a pivot step: x -= column * xp, a -= column * ap, the column's
+// element by DPP from lane l of the row; then the next pivot from lane pl of
+// a.  A DPP read needs two wait states after the write of what it reads: a was
+// written in the step before, at least the two products ap and xp ago.
+template <int l, int pl>
+__device__ __forceinline__ float pivot_first(float &x, float &a, float xp, float ap) {
+  float piv;
+  asm("v_fmac_f32_dpp %[x], %[a], -%[xp]" MPC_NB
+      "v_fmac_f32_dpp %[a], %[a], -%[ap]" MPC_NB
+      "s_nop 0\n"
+      "v_readlane_b32 %[p], %[a], %[pl]\n"
+      : [x] "+v"(x), [a] "+v"(a), [p] "=s"(piv)
+      : [xp] "v"(xp), [ap] "v"(ap), [l] "i"(l), [pl] "i"(pl));
+  return piv;
+}
+
+// The other three slots of the step, with the next pivot's inverse between
+// them: v_rcp_f32, one refinement and two residual steps, which is the
+// division's own sequence without its scaling and fix-up, so the correctly
+// rounded 1 / piv for a mid_range pivot.  Last, row P (quarter mask) becomes
+// [ap, xp] in its slot.  In a step that is not the last of its slot, that is
+// the slot of row P + 1 (pivot_first's), else one of the three.
+#define MPC_SLOT_X(k) "v_fmac_f32_dpp %[x" #k "], %[a" #k "], -%[xp]" MPC_NB
+#define MPC_SLOT_A(k) "v_fmac_f32_dpp %[a" #k "], %[a" #k "], -%[ap]" MPC_NB
+#define MPC_PIVOT_REST                          \
+  MPC_SLOT_X(0) MPC_SLOT_X(1) MPC_SLOT_X(2)     \
+  "v_rcp_f32 %[r], %[p]\n"                      \
+  MPC_SLOT_A(0)                                 \
+  "v_fma_f32 %[t], -%[p], %[r], 1.0\n"          \
+  MPC_SLOT_A(1)                                 \
+  "v_fma_f32 %[r], %[t], %[r], %[r]\n"          \
+  MPC_SLOT_A(2)                                 \
+  "v_fma_f32 %[t], -%[p], %[r], 1.0\n"          \
+  "v_fma_f32 %[i], %[t], %[r], %[r]\n"          \
+  "v_fma_f32 %[t], -%[p], %[i], 1.0\n"          \
+  "v_fma_f32 %[i], %[t], %[r], %[i]\n"
+template <int l>
+__device__ __forceinline__ float pivot_rest(float &x0, float &a0, float &x1, float &a1, float &x2, float &a2, float xp,
+                                            float ap, float piv, float &xc, float &ac, uint64_t mask) {
+  float inv, r, t;
+  asm(MPC_PIVOT_REST
+      "v_cndmask_b32_e64 %[ac], %[ac], %[ap], %[m]\n"
+      "v_cndmask_b32_e64 %[xc], %[xc], %[xp], %[m]\n"
+      : [x0] "+v"(x0), [a0] "+v"(a0), [x1] "+v"(x1), [a1] "+v"(a1), [x2] "+v"(x2), [a2] "+v"(a2), [xc] "+v"(xc),
+        [ac] "+v"(ac), [i] "=&v"(inv), [r] "=&v"(r), [t] "=&v"(t)
+      : [xp] "v"(xp), [ap] "v"(ap), [p] "s"(piv), [m] "s"(mask), [l] "i"(l));
+  return inv;
+}
+// row P in the first of the three slots
+template <int l>
+__device__ __forceinline__ float pivot_rest(float &x0, float &a0, float &x1, float &a1, float &x2, float &a2, float xp,
+                                            float ap, float piv, uint64_t mask) {
+  float inv, r, t;
+  asm(MPC_PIVOT_REST
+      "v_cndmask_b32_e64 %[a0], %[a0], %[ap], %[m]\n"
+      "v_cndmask_b32_e64 %[x0], %[x0], %[xp], %[m]\n"
+      : [x0] "+v"(x0), [a0] "+v"(a0), [x1] "+v"(x1), [a1] "+v"(a1), [x2] "+v"(x2), [a2] "+v"(a2), [i] "=&v"(inv),
+        [r] "=&v"(r), [t] "=&v"(t)
+      : [xp] "v"(xp), [ap] "v"(ap), [p] "s"(piv), [m] "s"(mask), [l] "i"(l));
+  return inv;
+}
+#undef MPC_PIVOT_REST
+#undef MPC_SLOT_A
+#undef MPC_SLOT_X
+// x -= column * xp (the last pivot: A is not used after it)
+template <int l>
+__device__ __forceinline__ void pivot_last(float (&x)[4], const float (&a)[4], float xp) {
+  asm("s_nop 1\n"
+      "v_fmac_f32_dpp %[x0], %[a0], -%[xp]" MPC_NB
+      "v_fmac_f32_dpp %[x1], %[a1], -%[xp]" MPC_NB
+      "v_fmac_f32_dpp %[x2], %[a2], -%[xp]" MPC_NB
+      "v_fmac_f32_dpp %[x3], %[a3], -%[xp]" MPC_NB
+      : [x0] "+v"(x[0]), [x1] "+v"(x[1]), [x2] "+v"(x[2]), [x3] "+v"(x[3])
+      : [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]), [xp] "v"(xp), [l] "i"(l));
+}
+
+// a[t] -= E(4 t + q, m) b for the lane's four rows, E(., m) by DPP from lane m
+#define MPC_BLOCK_UPDATE(nop)                                                                 \
+  asm(nop "v_fmac_f32_dpp %[a0], %[e0], -%[b]" MPC_NB                                         \
+          "v_fmac_f32_dpp %[a1], %[e1], -%[b]" MPC_NB                                         \
+          "v_fmac_f32_dpp %[a2], %[e2], -%[b]" MPC_NB                                         \
+          "v_fmac_f32_dpp %[a3], %[e3], -%[b]" MPC_NB                                         \
+      : [a0] "+v"(a[0]), [a1] "+v"(a[1]), [a2] "+v"(a[2]), [a3] "+v"(a[3])                    \
+      : [e0] "v"(e[0]), [e1] "v"(e[1]), [e2] "v"(e[2]), [e3] "v"(e[3]), [b] "v"(b), [l] "i"(l))
+template <int l>
+__device__ __forceinline__ void block_update(float (&a)[4], const float (&e)[4], float b) {
+  if constexpr (l == 0)
+    MPC_BLOCK_UPDATE("s_nop 1\n");  // the wait states between the writes of e and their first DPP read
+  else
+    MPC_BLOCK_UPDATE("");
+}
+#undef MPC_BLOCK_UPDATE
+template <int... M>
+__device__ __forceinline__ void block_updates(float (&a)[4], const float (&e)[4], const float (&b)[NX],
+                                              std::integer_sequence<int, M...>) {
+  (block_update<M>(a, e, b[M]), ...);
+}
+
+// the quarters' lanes in scalar registers, and the ds_bpermute address of the
+// lane's column in each quarter
+struct Quarters {
+  uint64_t mask[4];
+  uint32_t from[4];
+};
+
+// Gauss-Jordan inverse of the block in a into x: pivot steps P .. 13.  rowa,
+// rowx: row P of [A | X] in every quarter; piv, inv: its pivot and inverse;
+// pivots: lane P holds pivot P.  DIV: inverses by division.
+template <bool DIV, int P = 0>
+__device__ __forceinline__ void gj_wave_steps(const Quarters &qs, float (&a)[4], float (&x)[4], float rowa, float rowx,
+                                             float piv, float inv, float &pivots) {
+  constexpr int QP = P & 3, TP = P >> 2;              // owner quarter and slot of row P
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(pivots) : "s"(piv), "i"(P));
+  if constexpr (DIV) inv = 1.f / piv;
+  const float ap = rowa * inv, xp = rowx * inv;
+  if constexpr (P + 1 < NX) {
+    constexpr int Q1 = (P + 1) & 3, T1 = (P + 1) >> 2;  // and of row P + 1
+    const float next = pivot_first<P, 16 * Q1 + P + 1>(x[T1], a[T1], xp, ap);
+    const float ra = lane_value(a[T1], qs.from[Q1]), rx = lane_value(x[T1], qs.from[Q1]);
+    float ni;
+    if constexpr (T1 == TP) {
+      constexpr int o0 = T1 == 0 ? 1 : 0, o1 = T1 <= 1 ? 2 : 1, o2 = T1 <= 2 ? 3 : 2;
+      ni = pivot_rest<P>(x[o0], a[o0], x[o1], a[o1], x[o2], a[o2], xp, ap, next, x[T1], a[T1], qs.mask[QP]);
+    } else {
+      constexpr int o1 = TP == 0 ? 2 : 0, o2 = TP <= 1 ? 3 : 1;
+      static_assert(TP != T1 && o1 != TP && o2 != TP && o1 != T1 && o2 != T1 && o1 != o2, "the three other slots");
+      ni = pivot_rest<P>(x[TP], a[TP], x[o1], a[o1], x[o2], a[o2], xp, ap, next, qs.mask[QP]);
+    }
+    gj_wave_steps<DIV, P + 1>(qs, a, x, ra, rx, next, ni, pivots);
+  } else {
+    pivot_last<P>(x, a, xp);
+    const bool own = (qs.mask[QP] >> (threadIdx.x & 63u)) & 1u;
+    x[TP] = own ? xp : x[TP];
+  }
+}
+
+// base[off + c]: a lane's 32-bit element offset and a constant from a uniform base
+__device__ __forceinline__ const float *at(const float *base, uint32_t off) {
+  return reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + 4u * off);
+}
+__device__ __forceinline__ float *at(float *base, uint32_t off) {
+  return reinterpret_cast<float *>(reinterpret_cast<char *>(base) + 4u * off);
+}
+
+__device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restrict__ S, float *work, const Pick &p,
+                                           uint32_t lane) {
+  const uint32_t q = lane >> 4, jl = lane & 15u, j = jl < (uint32_t)NX ? jl : NX - 1;
+  const bool tail = q < 2u;  // slot 3 holds rows 12, 13 in quarters 0, 1
+  Quarters qs;
+  uint32_t rr[4], bl[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const uint32_t r = 4u * t + q;
-    if (r == (uint32_t)P) {
-      a[t] = ap;
-      x[t] = xp;
-    } else {
-      a[t] -= pc[t] * ap;
-      x[t] -= pc[t] * xp;
-    }
+    qs.mask[t] = 0xFFFFull << (16 * t);
+    qs.from[t] = 4u * (16u * t + jl);
+    const uint32_t r = 4u * t + q, i = lane + 64u * t;
+    rr[t] = r < (uint32_t)NX ? r : 0u;                                               // clamped row
+    bl[t] = i < (uint32_t)NXX ? i / NX + RS * (i % NX) : (uint32_t)(NX * RS) + jl;   // place of element i of B
   }
-  pin(a);
-  pin(x);
-}
-
-template <int P = 0>
-__device__ __forceinline__ void gj_wave_steps(uint32_t q, uint32_t j, float (&a)[4], float (&x)[4]) {
-  if constexpr (P < NX) {
-    gj_wave_step<P>(q, j, a, x);
-    gj_wave_steps<P + 1>(q, j, a, x);
-  }
-}
-
-__device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restrict__ S, float *__restrict__ work,
-                                           const Pick &p, uint32_t lane) {
-  const uint32_t q = lane >> 4, jl = lane & 15u, j = jl < (uint32_t)NX ? jl : NX - 1;
-  const bool col_ok = jl < (uint32_t)NX;
-  for (uint32_t i = lane; i < (uint32_t)(NX * RS); i += 64) L.Dinv[i] = 0.f;
-  float a_cur[4], b_cur[4], a_nxt[4], b_nxt[4];
+  const float *Sp = S + (size_t)S_STRIDE * p.K0;
+  float *W = work + (size_t)S_STRIDE * p.K0;
+  const uint32_t oa = NXX + q + NX * j, oe = q + NX * j;  // column j of a block from row q on, rows 4 apart
+  // the knot's column elements and its B, read two knots ahead (what lies
+  // past the block in its row is read with it and not used)
+  float a_nxt[2][4], b_nxt[2][4];
   auto load = [&](float (&a)[4], float (&bb)[4], uint32_t k) {
-    const float *Sr = S + (size_t)S_STRIDE * (p.K0 + k);
+    const float *Sr = Sp + (size_t)S_STRIDE * (k < p.N ? k : p.N - 1u);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const uint32_t r = 4u * t + q, i = lane + 64u * t;
-      a[t] = r < (uint32_t)NX ? -Sr[NXX + r + NX * j] : 0.f;
-      bb[t] = (k > 0 && i < (uint32_t)NXX) ? -Sr[i] : 0.f;
+      a[t] = at(Sr, oa)[4 * t];
+      bb[t] = at(Sr, lane)[64 * t];
     }
   };
-  load(a_cur, b_cur, 0);
-  for (uint32_t k = 0; k < p.N; ++k) {
-    load(a_nxt, b_nxt, k + 1 < p.N ? k + 1 : p.N - 1);
+  auto put_b = [&](const float (&bb)[4], uint32_t k) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const uint32_t i = lane + 64u * t;  // B(i % 14, i / 14)
-      if (i < (uint32_t)NXX) L.B[i / NX + RS * (i % NX)] = b_cur[t];
-    }
-    wave_sync();
-    // E_b(r, j) = sum_m B(r, m) D_{b-1}^-1(m, j), m in order
-    float dv[NX];
+    for (int t = 0; t < 4; ++t) L.B[k & 1u][bl[t]] = -bb[t];
+  };
+  float a[4], x[4], b0[4];
+  load(a, b0, 0);
+  load(a_nxt[1], b_nxt[1], 1);
+  load(a_nxt[0], b_nxt[0], 2);
+  auto step = [&](uint32_t k, float (&an)[4], float (&bn)[4]) {
+    float br[4][NX], bj[NX];
+    float e[4] = {0.f, 0.f, 0.f, 0.f};
+    if (k > 0) {
+      // D_{k-1}^-1 from the quarters to columns
 #pragma unroll
-    for (int m = 0; m < NX; ++m) dv[m] = L.Dinv[m + RS * j];
-    float e[4];
+      for (int t = 0; t < 3; ++t) L.Dinv[4u * t + q + RS * j] = x[t];
+      if (tail) L.Dinv[12u + q + RS * j] = x[3];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) e[t] = 0.f;
+      for (int m = 0; m < NX; ++m) {
+        bj[m] = L.B[k & 1u][m + RS * j];
 #pragma unroll
-    for (int m = 0; m < NX; ++m) {
-      const float d = dv[m];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint32_t r = 4u * t + q;
-        e[t] += L.B[m + RS * (r < (uint32_t)NX ? r : 0u)] * d;
+        for (int t = 0; t < 4; ++t) br[t][m] = L.B[k & 1u][m + RS * rr[t]];
       }
-    }
-    if (col_ok) {
-      float *w = slot_E(work, p.K0 + k) + NX * j;
+      wave_sync();
+      float dv[NX];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint32_t r = 4u * t + q;
-        if (r < (uint32_t)NX) {
-          L.E[j + RS * r] = e[t];
-          if (p.live) w[r] = e[t];
-        }
-      }
+      for (int m = 0; m < NX; ++m) dv[m] = L.Dinv[m + RS * j];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[t] = an[t];
+      load(an, bn, k + 2);
+      // E_b(r, j) = sum_m B(r, m) D_{b-1}^-1(m, j), m in order
+#pragma unroll
+      for (int m = 0; m < NX; ++m)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) e[t] += br[t][m] * dv[m];
     }
-    wave_sync();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) a[t] = t < 3 || tail ? -a[t] : 0.f;
     // D_b(r, j) = A_b(r, j) - sum_m E(r, m) B(j, m), m in order
-    float a[4];
+    if (k > 0) block_updates(a, e, bj, std::make_integer_sequence<int, NX>{});
+    float *Wk = W + (size_t)S_STRIDE * k;
+    // lanes 14 and 15 store what lane 13 does
 #pragma unroll
-    for (int t = 0; t < 4; ++t) a[t] = a_cur[t];
-#pragma unroll
-    for (int m = 0; m < NX; ++m) {
-      const float bjm = L.B[m + RS * j];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint32_t r = 4u * t + q;
-        a[t] -= L.E[m + RS * (r < (uint32_t)NX ? r : 0u)] * bjm;
-      }
-    }
-    pin(a);
-    float x[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x[t] = 4u * t + q == j ? 1.f : 0.f;
-    gj_wave_steps(q, jl, a, x);
-    wave_sync();  // every read of D_{b-1}^-1, B and E is done
-    if (col_ok) {
-      float *w = slot_Dinv(work, p.K0 + k) + NX * j;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint32_t r = 4u * t + q;
-        if (r < (uint32_t)NX) {
-          L.Dinv[r + RS * j] = x[t];
-          if (p.live) w[r] = x[t];
-        }
-      }
-    }
+    for (int t = 0; t < 3; ++t) at(Wk, oe)[4 * t] = e[t];
+    if (tail) at(Wk, oe)[12] = e[3];
+    float keep[4], pivots = 1.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      a_cur[t] = a_nxt[t];
-      b_cur[t] = b_nxt[t];
+      keep[t] = a[t];
+      x[t] = 4u * t + q == j ? 1.f : 0.f;
     }
+    const float rowa = lane_value(a[0], qs.from[0]), rowx = j == 0 ? 1.f : 0.f, piv = read_lane<0>(a[0]);
+    gj_wave_steps<false>(qs, a, x, rowa, rowx, piv, 1.f / piv, pivots);
+    if (__builtin_amdgcn_ballot_w64(!mid_range(pivots)) != 0) {  // again, with divisions
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        a[t] = keep[t];
+        x[t] = 4u * t + q == j ? 1.f : 0.f;
+      }
+      gj_wave_steps<true>(qs, a, x, rowa, rowx, piv, 1.f, pivots);
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) at(Wk, oe)[NXX + 4 * t] = x[t];
+    if (tail) at(Wk, oe)[NXX + 12] = x[3];
+  };
+  // B of the next knot goes to LDS ahead of the step that reads it
+  put_b(b_nxt[1], 1);
+  step(0, a_nxt[0], b_nxt[0]);
+  for (uint32_t k = 1; k < p.N; k += 2) {
+    put_b(b_nxt[0], k + 1);
+    wave_sync();
+    step(k, a_nxt[1], b_nxt[1]);
+    if (k + 1 >= p.N) break;
+    put_b(b_nxt[1], k + 2);
+    wave_sync();
+    step(k + 1, a_nxt[0], b_nxt[0]);
   }
-  wave_sync();
+}
+#undef MPC_NB
+
+// ---- substitution ------------------------------------------------------------
+// The sweeps' chain is one 14-term dot product per knot (the terms by DPP
+// row_newbcast in the multiply-adds, one after the other: about 70 clocks).
+// The four rows of the wave hold the factor rows of four consecutive knots
+// (so one set of reads serves four), and take their turns in the order 0, 1,
+// 3, 2: from each to the next, and from the last to the first of the next
+// four, the result moves by one lane swap.  What is off the chain (z_k =
+// D_k^-1 y_k) runs once for the four knots.
+// N = 256, both sweeps: 186 -> 49 us (before: one row, the vector by ds_swizzle).
+
+// sum_m w[m] v_m, v_m the value v of lane m of the row (m < 14), in order
+__device__ __forceinline__ float bdot(const float (&w)[NX], float v) {
+  float s = 0.f;
+#define MPC_BD(m, k) "v_fmac_f32_dpp %0, %1, %" #k " row_newbcast:" #m " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+  asm("s_nop 1\n" MPC_BD(0, 2) MPC_BD(1, 3) MPC_BD(2, 4) MPC_BD(3, 5) MPC_BD(4, 6) MPC_BD(5, 7) MPC_BD(6, 8)
+          MPC_BD(7, 9) MPC_BD(8, 10) MPC_BD(9, 11) MPC_BD(10, 12) MPC_BD(11, 13) MPC_BD(12, 14) MPC_BD(13, 15)
+      : "+v"(s)
+      : "v"(v), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]),
+        "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]));
+#undef MPC_BD
+  return s;
+}
+
+// v of the row of turn s (rows 0, 1, 3, 2) in the row of the next turn:
+// 0 -> 1 and 3 -> 2 by swapping neighbouring rows, 1 -> 3 and 2 -> 0 by
+// swapping halves
+template <int s>
+__device__ __forceinline__ float pass_on(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  uint32_t o;
+  if constexpr (s & 1)
+    o = __builtin_amdgcn_permlane32_swap(u, u, false, false)[s >> 1];
+  else
+    o = __builtin_amdgcn_permlane16_swap(u, u, false, false)[s >> 1];
+  return __builtin_bit_cast(float, o);
+}
+
+// 14 consecutive floats at p, in pairs (a caller's workspace may lie at any
+// multiple of four bytes, which 64-bit global reads take)
+typedef float pair_u __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ void load14(float (&v)[NX], const float *p) {
+  const pair_u *p2 = reinterpret_cast<const pair_u *>(p);
+#pragma unroll
+  for (int c = 0; c < NX / 2; ++c) {
+    const pair_u t = p2[c];
+    v[2 * c] = t.x;
+    v[2 * c + 1] = t.y;
+  }
 }
 
 // forward and backward sweeps of one instance on the right-hand side
-// r = -gamma (gamma != nullptr) or the workspace's z slot; lambda = x, or
-// lambda += x with accumulate.  No barriers: the group's lanes share its
-// trip count.
-__device__ __forceinline__ void substitute(const float *__restrict__ gamma, float *__restrict__ work,
-                                          float *__restrict__ lambda, const Pick &p, bool accumulate, int lane) {
-  const int j = lane < NX ? lane : NX - 1;
-  const bool wr = p.live && lane < NX;
-  auto rhs = [&](uint32_t k) {
-    return gamma ? -gamma[(size_t)NX * (p.K0 + k) + j] : slot_z(work, p.K0 + k)[j];
+// r = -gamma, or with ACCUMULATE the workspace's z slots; lambda = x, or
+// lambda += x with ACCUMULATE
+template <bool ACCUMULATE>
+__device__ __forceinline__ void substitute(const float *__restrict__ gamma, float *work,
+                                          float *__restrict__ lambda, const Pick &p, uint32_t lane) {
+  const uint32_t q = lane >> 4, i = lane & 15u, j = i < (uint32_t)NX ? i : NX - 1;
+  const uint32_t turn = q ^ (q >> 1);  // rows 0, 1, 3, 2 in order
+  const bool el = i < (uint32_t)NX;
+  const uint32_t last = p.N - 1u;
+  float *W = work + (size_t)S_STRIDE * p.K0, *lp = lambda + (size_t)NX * p.K0;
+  const float *gp = ACCUMULATE ? nullptr : gamma + (size_t)NX * p.K0;
+  // knots k0 .. k0 + 3 of the forward sweep, knot k0 + turn in the row (the
+  // last knot's data again past the end): row j of E_k (strided; E_0 = 0),
+  // row j of D_k^-1 (= column j, D^-1 symmetric) and the right-hand side
+  struct Fwd {
+    float er[NX], dr[NX], r;
   };
-  // row j of E_k (strided) and of D_k^-1 (= column j, D^-1 symmetric)
-  auto load_rows = [&](float (&er)[NX], float (&dr)[NX], uint32_t k) {
-    const float *E = slot_E(work, p.K0 + k), *D = slot_Dinv(work, p.K0 + k) + NX * j;
+  auto load_f = [&](Fwd &f, uint32_t k0) {
+    const uint32_t k = k0 + turn < last ? k0 + turn : last;
+    const float *E = at(W, S_STRIDE * k + j);
 #pragma unroll
-    for (int m = 0; m < NX; ++m) {
-      er[m] = k > 0 ? E[j + NX * m] : 0.f;
-      dr[m] = D[m];
-    }
+    for (int m = 0; m < NX; ++m) f.er[m] = E[NX * m];
+    load14(f.dr, at(W, S_STRIDE * k + NX * j) + NXX);
+    f.r = ACCUMULATE ? E[2 * NXX] : -*at(gp, NX * k + j);
   };
-  // a ring of PF buffers, knot k in buffer k % PF: each knot's rows are
-  // loaded PF knots ahead and only waited for where they are used
-  constexpr int PF = 4;
-  float er[PF][NX], dr[PF][NX], rv[PF];
   float y = 0.f;
-#pragma unroll
-  for (int d = 0; d < PF; ++d)
-    if ((uint32_t)d < p.N) {
-      load_rows(er[d], dr[d], (uint32_t)d);
-      rv[d] = rhs((uint32_t)d);
+  auto run_f = [&](const Fwd &f, uint32_t k0) {
+    float yo, t;  // the row's own y
+    t = f.r - bdot(f.er, y);
+    yo = t;
+    y = pass_on<0>(t);
+    if (k0 + 1 < p.N) {
+      t = f.r - bdot(f.er, y);
+      yo = turn == 1u ? t : yo;
+      y = pass_on<1>(t);
     }
-  auto step = [&](const float (&e_)[NX], const float (&d_)[NX], float r, uint32_t k) {
-    const float yk = r - bdot(e_, y);
-    const float zk = bdot(d_, yk);
-    if (wr) slot_z(work, p.K0 + k)[lane] = zk;
-    y = yk;
+    if (k0 + 2 < p.N) {
+      t = f.r - bdot(f.er, y);
+      yo = turn == 2u ? t : yo;
+      y = pass_on<2>(t);
+    }
+    if (k0 + 3 < p.N) {
+      t = f.r - bdot(f.er, y);
+      yo = turn == 3u ? t : yo;
+      y = pass_on<3>(t);
+    }
+    const float z = bdot(f.dr, yo);
+    if (el && k0 + turn < p.N) *at(W, S_STRIDE * (k0 + turn) + 2 * NXX + i) = z;
   };
-  for (uint32_t k = 0; k < p.N; k += PF) {
+  Fwd f[3];
 #pragma unroll
-    for (int d = 0; d < PF; ++d) {
-      if (k + d >= p.N) break;
-      step(er[d], dr[d], rv[d], k + d);
-      if (k + d + PF < p.N) {
-        load_rows(er[d], dr[d], k + d + PF);
-        rv[d] = rhs(k + d + PF);
-      }
+  for (int u = 0; u < 3; ++u) load_f(f[u], 4u * u);
+  for (uint32_t k0 = 0; k0 < p.N; k0 += 12) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const uint32_t k = k0 + 4u * u;
+      if (k >= p.N) break;
+      run_f(f[u], k);
+      load_f(f[u], k + 12u);
     }
   }
-  // backward: column j of E_{k+1} (contiguous), through a ring the same way
-  const float *zs = slot_z(work, p.K0);
-  float ec[PF][NX], zv[PF];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // z is read by other lanes below
+  // backward: knot top - turn in the row (knot 0 again past the start):
+  // column j of E_{k+1} (x = 0 past the last knot, whatever is read there),
+  // z_k and the value that x_k is added to
+  struct Bwd {
+    float ec[NX], z, l;
+  };
+  auto load_b = [&](Bwd &f, int top) {
+    const uint32_t k = top - (int)turn > 0 ? (uint32_t)(top - (int)turn) : 0u;
+    load14(f.ec, at(W, S_STRIDE * (k < last ? k + 1u : last) + NX * j));
+    f.z = *at(W, S_STRIDE * k + 2 * NXX + j);
+    f.l = ACCUMULATE ? *at(lp, NX * k + j) : 0.f;
+  };
   float x = 0.f;
-  auto load_col = [&](float (&c_)[NX], float &z, int k) {  // E_{k+1} column, z_k
-    const float *E = slot_E(work, p.K0 + (uint32_t)k + 1) + NX * j;
-#pragma unroll
-    for (int m = 0; m < NX; ++m) c_[m] = (uint32_t)k + 1 < p.N ? E[m] : 0.f;
-    z = zs[(size_t)S_STRIDE * (uint32_t)k + j];
-  };
-#pragma unroll
-  for (int d = 0; d < PF; ++d)
-    if ((int)p.N - 1 - d >= 0) load_col(ec[d], zv[d], (int)p.N - 1 - d);
-  auto bstep = [&](const float (&c_)[NX], float z, int k) {
-    const float xk = z - bdot(c_, x);
-    if (wr) {
-      float *l = lambda + (size_t)NX * (p.K0 + (uint32_t)k) + lane;
-      *l = accumulate ? *l + xk : xk;
+  auto run_b = [&](const Bwd &f, int top) {
+    float xo, t;
+    t = f.z - bdot(f.ec, x);
+    xo = t;
+    x = pass_on<0>(t);
+    if (top >= 1) {
+      t = f.z - bdot(f.ec, x);
+      xo = turn == 1u ? t : xo;
+      x = pass_on<1>(t);
     }
-    x = xk;
+    if (top >= 2) {
+      t = f.z - bdot(f.ec, x);
+      xo = turn == 2u ? t : xo;
+      x = pass_on<2>(t);
+    }
+    if (top >= 3) {
+      t = f.z - bdot(f.ec, x);
+      xo = turn == 3u ? t : xo;
+      x = pass_on<3>(t);
+    }
+    if (el && top >= (int)turn) *at(lp, NX * (uint32_t)(top - (int)turn) + i) = ACCUMULATE ? f.l + xo : xo;
   };
-  for (int k = (int)p.N - 1; k >= 0; k -= PF) {
+  Bwd g[3];
+  const int n = (int)p.N;
 #pragma unroll
-    for (int d = 0; d < PF; ++d) {
-      if (k - d < 0) break;
-      bstep(ec[d], zv[d], k - d);
-      if (k - d - PF >= 0) load_col(ec[d], zv[d], k - d - PF);
+  for (int u = 0; u < 3; ++u) load_b(g[u], n - 1 - 4 * u);
+  for (int top0 = n - 1; top0 >= 0; top0 -= 12) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int top = top0 - 4 * u;
+      if (top < 0) break;
+      run_b(g[u], top);
+      load_b(g[u], top - 12);
     }
   }
 }
 
-__global__ void __launch_bounds__(WG) k_direct_factor_solve(Batch b, const uint32_t *__restrict__ order,
-                                                            uint32_t n_list, const float *__restrict__ S,
-                                                            const float *__restrict__ gamma,
-                                                            const uint32_t *__restrict__ status,
-                                                            float *__restrict__ work, float *__restrict__ lambda,
-                                                            int do_factor, uint32_t *__restrict__ iters,
-                                                            uint32_t *__restrict__ flag) {
-  __shared__ FacLds lds[GROUPS_PER_WG];
-  const int grp = threadIdx.x / GROUP, lane = threadIdx.x % GROUP;
-  const Pick p = pick_instance(b, order, n_list, status, blockIdx.x * GROUPS_PER_WG + grp);
-  if (do_factor) factor(lds[grp], S, work, p, lane);
-  substitute(gamma, work, lambda, p, false, lane);
-  if (p.live && lane == 0) {
-    if (iters) iters[p.inst] = 0;
-    if (flag) flag[p.inst] = 0;
-  }
-}
-
-// one wave per instance: the factorisation on all 64 lanes, then the
-// substitution sweeps on the first 16-lane group (the others follow them
-// without writing)
-__global__ void __launch_bounds__(64) k_direct_factor_wave(Batch b, const uint32_t *__restrict__ order,
-                                                          uint32_t n_list, const float *__restrict__ S,
-                                                          const float *__restrict__ gamma,
-                                                          const uint32_t *__restrict__ status,
-                                                          float *__restrict__ work, float *__restrict__ lambda,
-                                                          uint32_t *__restrict__ iters, uint32_t *__restrict__ flag) {
+// one wave per instance: the factorisation (FACTOR; else the factors a
+// previous launch left in work), then the substitution sweeps on
+// r = -gamma, or with ACCUMULATE on the z slots, added to lambda
+template <bool FACTOR, bool ACCUMULATE>
+__global__ void __launch_bounds__(64) k_direct_wave(Batch b, const uint32_t *__restrict__ order,
+                                                   const float *__restrict__ S, const float *__restrict__ gamma,
+                                                   const uint32_t *__restrict__ status, float *work,
+                                                   float *__restrict__ lambda, uint32_t *__restrict__ iters,
+                                                   uint32_t *__restrict__ flag) {
   __shared__ FacWaveLds lds;
   const uint32_t lane = threadIdx.x;
-  Pick p;
-  p.inst = order ? order[blockIdx.x] : blockIdx.x;
-  p.K0 = inst_first(b, p.inst);
-  p.N = inst_len(b, p.inst);
-  p.Nmax = p.N;
-  p.live = !(status && !(status[p.inst] & ST_ACTIVE));
-  factor_wave(lds, S, work, p, lane);
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the factor rows written above are read below
-  Pick ps = p;
-  ps.live = p.live && lane < 16u;
-  substitute(gamma, work, lambda, ps, false, (int)(lane & 15u));
-  if (p.live && lane == 0) {
+  const Pick p = pick_instance(b, order, status, blockIdx.x);
+  if (!p.live) return;
+  if constexpr (FACTOR) {
+    factor_wave(lds, S, work, p, lane);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the factor rows written above are read below
+  }
+  substitute<ACCUMULATE>(gamma, work, lambda, p, lane);
+  if (!ACCUMULATE && lane == 0) {
     if (iters) iters[p.inst] = 0;
     if (flag) flag[p.inst] = 0;
   }
-}
-
-__global__ void __launch_bounds__(WG) k_direct_refine(Batch b, const uint32_t *__restrict__ order, uint32_t n_list,
-                                                      const uint32_t *__restrict__ status, float *__restrict__ work,
-                                                      float *__restrict__ lambda) {
-  const int grp = threadIdx.x / GROUP, lane = threadIdx.x % GROUP;
-  const Pick p = pick_instance(b, order, n_list, status, blockIdx.x * GROUPS_PER_WG + grp);
-  substitute(nullptr, work, lambda, p, true, lane);
 }
 
 // z slot of every knot <- -gamma + S lambda (fp64 accumulation), one group per knot
@@ -461,20 +562,20 @@ hipError_t launch_direct_solve(const Batch &b, const uint32_t *order, uint32_t n
                                const float *gamma, const uint32_t *status, float *work, float *lambda,
                                uint32_t refine, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
   if (n_list == 0) return hipSuccess;
-  const dim3 grid((n_list + GROUPS_PER_WG - 1) / GROUPS_PER_WG);
   if (do_factor)
-    hipLaunchKernelGGL(k_direct_factor_wave, dim3(n_list), dim3(64), 0, st, b, order, n_list, S, gamma, status, work,
+    hipLaunchKernelGGL((k_direct_wave<true, false>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
                        lambda, iters, flag);
   else
-    hipLaunchKernelGGL(k_direct_factor_solve, grid, dim3(WG), 0, st, b, order, n_list, S, gamma, status, work, lambda,
-                       0, iters, flag);
+    hipLaunchKernelGGL((k_direct_wave<false, false>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
+                       lambda, iters, flag);
   hipError_t e = hipGetLastError();
   for (uint32_t s = 0; s < refine && e == hipSuccess; ++s) {
     hipLaunchKernelGGL(k_schur_residual, dim3((b.total_knots + GROUPS_PER_WG - 1) / GROUPS_PER_WG), dim3(WG), 0, st,
                        b, S, gamma, (const float *)lambda, work);
     e = hipGetLastError();
     if (e != hipSuccess) break;
-    hipLaunchKernelGGL(k_direct_refine, grid, dim3(WG), 0, st, b, order, n_list, status, work, lambda);
+    hipLaunchKernelGGL((k_direct_wave<false, true>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
+                       lambda, (uint32_t *)nullptr, (uint32_t *)nullptr);
     e = hipGetLastError();
   }
   return e;

@@ -171,10 +171,6 @@ __device__ __forceinline__ void read_slot(float (&M)[16], const float *Sl, uint3
   }
 }
 
-// a condition that has the same value in every lane of the wave, in a scalar
-// register (a branch on it leaves EXEC alone)
-__device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
-
 // total of the 16 lanes of each row, in every lane of the row (fixed order;
 // each step adds two values in either order, so the lanes agree bitwise)
 __device__ __forceinline__ float row_total(float v) {

@@ -25,6 +25,12 @@
 // algorithm and exit rule as k_pcg.hip (GPU-PCG pcg<T,14,N>,
 // toplevel.cuh:143-157).
 //
+// Of the 8500 clocks of an iteration at 128 knots a part, products and
+// preconditioner take some 3700 (issue of two waves per SIMD), the two
+// exchanges 1100 - 1400 each.  173 iterations, with divergent loop conditions
+// and a readlane ahead of every addition of a total / now: N = 256 642 / 618
+// us, N = 512 758 / 649 us; stair 1182 / 888 us, 1437 / 941 us.
+//
 // Two launch forms, both cooperative (all workgroups co-resident):
 // - k_pcg_team: one team per Q workgroups; more teams than fit at once are
 //   solved by consecutive launches (four-workgroup teams, single instances);
@@ -74,36 +80,53 @@ constexpr int RK = 4;
 constexpr int KNOTS = NGRP * RK;  // knots per part
 constexpr uint32_t SPIN_LIMIT = 1u << 16;
 // mailbox words of a part: 0..7 wave partials, MB_FIRST.. its first row,
-// MB_LAST.. its last row; lanes of a polling wave: 0 .. 8(Q-1)-1 the other
-// parts' partials, LANE_M.. the row before the part, LANE_P.. the row after
+// MB_LAST.. its last row; lanes of a polling wave: 0..7, 16..23 and 8..15 the
+// partials of the first, second and third other part, LANE_M.. the row before
+// the part, LANE_P.. the row after
 constexpr uint32_t MB_FIRST = 8, MB_LAST = 24, LANE_M = 32, LANE_P = 48;
 static_assert(MB_FIRST == NWAV && MB_LAST >= MB_FIRST + NX && MB_LAST + NX <= 40, "mailbox layout");
-static_assert(8 * 3 <= LANE_M && LANE_M + NX <= LANE_P && LANE_P + NX <= 64, "polling lanes");
+static_assert(24 <= LANE_M && LANE_M + NX <= LANE_P && LANE_P + NX <= 64, "polling lanes");
 
 struct TeamShared {
   float L[(KNOTS + 1) * L_SLOT + L_GUARD];
   float zb[(KNOTS + 1) * 16];
   float wb[(KNOTS + 1) * 16];  // stair preconditioner: staged D^-1 r
-  float red[2][NWAV];
+  alignas(16) float red[2][NWAV];
   float recv[2][16];  // rows from the part before / after
   uint32_t fail;
 };
 static_assert(((KNOTS + 1) * L_SLOT + L_GUARD) % 4 == 0, "L and zb are cleared as one float4 range");
 
 __device__ __forceinline__ float sum8(const float *red) {
-  float s = 0.f;
-#pragma unroll
-  for (int v = 0; v < NWAV; ++v) s += red[v];
+  const float4 x = *reinterpret_cast<const float4 *>(red), y = *reinterpret_cast<const float4 *>(red + 4);
+  return ((((((x.x + x.y) + x.z) + x.w) + y.x) + y.y) + y.z) + y.w;
+}
+
+// per row of the wave, x of its lanes 0..7 (HIGH: 8..15) summed in lane order
+// (the order of sum8), in every lane of the row: eight DPP additions, the
+// broadcast in each (a readlane ahead of every addition took 115 clocks a term)
+template <bool HIGH>
+__device__ __forceinline__ float row_sum8(float x) {
+  float s;
+#define MPC_RS(op, l) op "_dpp %0, %1, %0 row_newbcast:" #l " row_mask:0xf bank_mask:0xf\n"
+  if constexpr (!HIGH)
+    asm("s_nop 1\nv_mov_b32_dpp %0, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n" MPC_RS("v_add_f32", 1)
+            MPC_RS("v_add_f32", 2) MPC_RS("v_add_f32", 3) MPC_RS("v_add_f32", 4) MPC_RS("v_add_f32", 5)
+                MPC_RS("v_add_f32", 6) MPC_RS("v_add_f32", 7) "s_nop 1"
+        : "=&v"(s)
+        : "v"(x));
+  else
+    asm("s_nop 1\nv_mov_b32_dpp %0, %1 row_newbcast:8 row_mask:0xf bank_mask:0xf\n" MPC_RS("v_add_f32", 9)
+            MPC_RS("v_add_f32", 10) MPC_RS("v_add_f32", 11) MPC_RS("v_add_f32", 12) MPC_RS("v_add_f32", 13)
+                MPC_RS("v_add_f32", 14) MPC_RS("v_add_f32", 15) "s_nop 1"
+        : "=&v"(s)
+        : "v"(x));
+#undef MPC_RS
   return s;
 }
 
-// x of lanes l0 .. l0+7 (l0 uniform), summed in lane order (the order of sum8)
-__device__ __forceinline__ float sum_lanes8(float x, uint32_t l0) {
-  float s = 0.f;
-#pragma unroll
-  for (uint32_t v = 0; v < (uint32_t)NWAV; ++v)
-    s += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), (int)(l0 + v)));
-  return s;
+__device__ __forceinline__ float lane_of(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
 // tag_xor: 0, or a bit pattern that makes the tag wrong (the poison hook)
@@ -171,6 +194,7 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     constexpr uint32_t n4 = ((KNOTS + 1) * L_SLOT + L_GUARD + (KNOTS + 1) * 16) / 4;
     for (uint32_t idx = tid; idx < n4; idx += NT) z4[idx] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (tid == 0) sh.fail = 0u;
+    if (tid < 32u) (&sh.recv[0][0])[tid] = 0.f;  // lanes 14, 15 stay zero
   }
   __syncthreads();
   // every part but the last: L_ke into the slot after its own knots
@@ -193,6 +217,7 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     const bool has = lk < n_own;
     load_row(R[t], sh.L + lk * L_SLOT, has, i, d, S, Pinv, K0, kb + lk);
     lam[t] = has && lane_ok ? lambda[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
+    r[t] = has && lane_ok ? gamma[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
   }
   // the group's outer neighbours: in the own zb, from the next / previous
   // part, or none
@@ -224,8 +249,8 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   // 3 = the row after it (wave wl)
   constexpr uint32_t PART_WORDS = sizeof(TeamMailbox{}.w[0][0]) / sizeof(unsigned long long);  // 40
   uint32_t role = 0, word = 0;
-  if (lane64 < 8u * (Q - 1)) {
-    const uint32_t q = lane64 >> 3;
+  if (lane64 < 8u || (Q == 4 && lane64 < 24u)) {
+    const uint32_t q = lane64 < 8u ? 0u : lane64 < 16u ? 2u : 1u;
     role = 1u;
     word = (q < part ? q : q + 1u) * PART_WORDS + (lane64 & 7u);
   } else if (has_prev && w == 0 && lane64 >= LANE_M && lane64 < LANE_M + NX) {
@@ -237,7 +262,8 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   }
   auto collect = [&](bool partials, bool rows) {
     const bool rm = rows && has_prev && w == 0, rp = rows && has_next && w == wl;
-    const bool want = (role == 1u && partials) || (role == 2u && rows) || (role == 3u && rows);
+    // after a wait that ran out nothing more is waited for
+    const bool want = ok && ((role == 1u && partials) || (role == 2u && rows) || (role == 3u && rows));
     float x = 0.f;
     if (partials || rm || rp) {
       x = mb_wait(&mb->w[mb_buf(set, e)][0][0] + word, want, e, ok);
@@ -251,9 +277,14 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     }
     return x;
   };
+  // the outer neighbours' elements: own slots, received rows, or the zero
+  // slot behind the own ones
+  const float *zero = sh.zb + KNOTS * 16 + i;
+  const float *far_m_src = far_m ? sh.recv[0] + i : zero, *far_p_src = far_p ? sh.recv[1] + i : zero;
+  const float *zm_src = own_m ? zb0 - 16 : far_m_src, *zp_src = own_p ? zb0 + RK * 16 : far_p_src;
   auto neighbours = [&](float &vm, float &vp) {
-    vm = own_m ? zb0[-16] : (far_m && lane_ok ? sh.recv[0][i] : 0.f);
-    vp = own_p ? zb0[RK * 16] : (far_p && lane_ok ? sh.recv[1][i] : 0.f);
+    vm = *zm_src;
+    vp = *zp_src;
   };
   // stair preconditioner: w = D^-1 r staged like z, in its own buffer, and
   // its row at the split exchanged on an epoch of its own (row only)
@@ -263,18 +294,23 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     wb0[(RK - 1) * 16] = v[RK - 1];
     post_rows(v);
   };
+  const float *wm_src = own_m ? wb0 - 16 : far_m_src, *wp_src = own_p ? wb0 + RK * 16 : far_p_src;
   auto neighbours_w = [&](float &vm, float &vp) {
-    vm = own_m ? wb0[-16] : (far_m && lane_ok ? sh.recv[0][i] : 0.f);
-    vp = own_p ? wb0[RK * 16] : (far_p && lane_ok ? sh.recv[1][i] : 0.f);
+    vm = *wm_src;
+    vp = *wp_src;
   };
   auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, sh.L + b0 * L_SLOT, i, x, xm, xp, y); };
   // ((part 0 + part 1) + part 2) + part 3: the own part from LDS, the others
   // from the partial lanes x of collect
   auto total = [&](float mine, float x) {
-    float t = 0.f;
-#pragma unroll
-    for (uint32_t q = 0; q < (uint32_t)Q; ++q) t += q == part ? mine : sum_lanes8(x, 8u * (q < part ? q : q - 1u));
-    return t;
+    const float a = row_sum8<false>(x);
+    const float o0 = lane_of(a, 0);  // the first other part
+    if constexpr (Q == 2) return part == 0 ? mine + o0 : o0 + mine;
+    const float c = row_sum8<true>(x);
+    const float o1 = lane_of(a, 16), o2 = lane_of(c, 0);
+    const float v0 = part == 0 ? mine : o0, v1 = part == 1 ? mine : part < 1 ? o0 : o1,
+                v2 = part == 2 ? mine : part < 2 ? o1 : o2, v3 = part == 3 ? mine : o2;
+    return ((v0 + v1) + v2) + v3;
   };
 
   // boundary lambda to the partner
@@ -285,72 +321,43 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   float pm, pp;
   neighbours(pm, pp);
 
-  // prologue: r = gamma - S lambda, z = Pinv r, p = z, eta = r.z
-  smv(lam, pm, pp);
-  float part_sum = 0.f;
-#pragma unroll
-  for (int t = 0; t < RK; ++t) {
-    const uint32_t lk = b0 + (uint32_t)t;
-    r[t] = lk < n_own && lane_ok ? gamma[(size_t)NX * (K0 + kb + lk) + i] - y[t] : 0.f;
-  }
-  if constexpr (STAIR) {
-    float wv[RK], v[RK], wm, wp;
-    group_precond<RK>(R, r, wv);
-    __syncthreads();  // every read of the lambda row in recv is done
-    ++e;
-    stage_w(wv);
-    __syncthreads();
-    if (sh.fail) return fault();
-    collect(false, true);
-    neighbours_w(wm, wp);
-    smv(wv, wm, wp);
-#pragma unroll
-    for (int t = 0; t < RK; ++t) v[t] = lane_ok ? 2.f * r[t] - y[t] : 0.f;
-    group_precond<RK>(R, v, z);
-  } else {
-    group_precond<RK>(R, r, z);
-  }
-#pragma unroll
-  for (int t = 0; t < RK; ++t) part_sum += r[t] * z[t];
-  part_sum = wave_sum(part_sum);
-  __syncthreads();  // neighbour and row reads done before zb / recv are reused
-  ++e;
-  if (lane64 == 0) {
-    sh.red[1][w] = part_sum;
-    mb_post(mb, set, part, e, w, part_sum, tag_xor);
-  }
-  stage(z);
-  __syncthreads();
-  if (sh.fail) return fault();
-  float eta = total(sum8(sh.red[1]), collect(true, true));
-  neighbours(pm, pp);
-#pragma unroll
-  for (int t = 0; t < RK; ++t) p[t] = z[t];
-  uint32_t it = 0;
-  // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
-  const float tol_i = tol < 0.f ? fmaxf(-tol * fabsf(eta), FLT_MIN) : tol;
-  bool conv = fabsf(eta) < tol_i;
-  float eta_last = eta;  // of the last exit test
-
-  while (!conv && it < cap) {
+  // y = S p, its share of p.y posted; the next epoch begins here
+  auto product = [&](bool post) {
     smv(p, pm, pp);
     float pyp = 0.f;
 #pragma unroll
     for (int t = 0; t < RK; ++t) pyp += p[t] * y[t];
     pyp = wave_sum(pyp);
     ++e;
-    if (lane64 == 0) {
-      sh.red[0][w] = pyp;
-      mb_post(mb, set, part, e, w, pyp, tag_xor);
-    }
+    sh.red[0][w] = pyp;  // the wave's lanes write the same value
+    if (post && lane64 == 0) mb_post(mb, set, part, e, w, pyp, tag_xor);
     __syncthreads();
-    if (sh.fail) return fault();
-    const float alpha = eta / total(sum8(sh.red[0]), collect(true, false));
+  };
+
+  // The first pass is the prologue, through the same code: p = lambda,
+  // r = gamma - S lambda (alpha = 1, lambda kept), z = M r, then p = z
+  // (beta = 0) and eta = r.z; the others are the iterations.  The loop has
+  // one branch, back, on a scalar condition (with more the compiler puts all
+  // of them on EXEC masks), and it stands behind the barrier of the next
+  // product: the waves of a workgroup may see different sums once a wait has
+  // run out, but sh.fail is the same for all of them there, so that all leave
+  // together.  The product that the last pass takes ahead is not used (one
+  // more in the number of iterations).
+#pragma unroll
+  for (int t = 0; t < RK; ++t) p[t] = lam[t];
+  product(true);
+  uint32_t it = ~0u;  // the first pass is not counted
+  float eta = 0.f, tol_i = tol;
+  bool first = true, conv, failed, run;
+  do {
+    const float own0 = sum8(sh.red[0]);
+    const float quo = eta / total(own0, collect(true, false)), alpha = first ? 1.f : quo;
+    const float alpha_l = first ? 0.f : alpha;
     float rz = 0.f;
 #pragma unroll
     for (int t = 0; t < RK; ++t) {
-      lam[t] += alpha * p[t];
-      r[t] = lane_ok ? r[t] - alpha * y[t] : 0.f;
+      lam[t] += alpha_l * p[t];
+      r[t] -= alpha * y[t];
     }
     if constexpr (STAIR) {
       // z = D^-1 (2 r - S w), w = D^-1 r; the previous z row in recv was
@@ -360,12 +367,11 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
       ++e;
       stage_w(wv);
       __syncthreads();
-      if (sh.fail) return fault();
       collect(false, true);
       neighbours_w(wm, wp);
       smv(wv, wm, wp);
 #pragma unroll
-      for (int t = 0; t < RK; ++t) wv[t] = lane_ok ? 2.f * r[t] - y[t] : 0.f;  // w is no longer needed
+      for (int t = 0; t < RK; ++t) wv[t] = 2.f * r[t] - y[t];  // w is no longer needed
       group_precond<RK>(R, wv, z);
     } else {
       group_precond<RK>(R, r, z);
@@ -374,32 +380,33 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     for (int t = 0; t < RK; ++t) rz += r[t] * z[t];
     rz = wave_sum(rz);
     ++e;
-    if (lane64 == 0) {
-      sh.red[1][w] = rz;
-      mb_post(mb, set, part, e, w, rz, tag_xor);
-    }
+    sh.red[1][w] = rz;
+    if (lane64 == 0) mb_post(mb, set, part, e, w, rz, tag_xor);
     stage(z);
     __syncthreads();
-    if (sh.fail) return fault();
-    float zm = own_m ? zb0[-16] : 0.f, zp = own_p ? zb0[RK * 16] : 0.f;  // issued before the wait
-    const float eta_new = total(sum8(sh.red[1]), collect(true, true));
-    eta_last = eta_new;
-    if (far_m && lane_ok) zm = sh.recv[0][i];
-    if (far_p && lane_ok) zp = sh.recv[1][i];
-    ++it;
-    if (fabsf(eta_new) < tol_i) {
-      conv = true;
-      break;
-    }
-    const float beta = eta_new / eta;
+    const float own1 = sum8(sh.red[1]);
+    const float x = collect(true, true);
+    float zm, zp;
+    neighbours(zm, zp);
+    const float eta_new = total(own1, x);
+    // taken in the last iteration too (p is not used after it)
+    const float quo_b = eta_new / eta, beta = first ? 0.f : quo_b;
     eta = eta_new;
 #pragma unroll
     for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], z[t]);
     pm = fmaf(beta, pm, zm);
     pp = fmaf(beta, pp, zp);
-  }
-  __syncthreads();
-  if (sh.fail) return fault();
+    // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
+    tol_i = first && tol < 0.f ? fmaxf(-tol * fabsf(eta), FLT_MIN) : tol_i;
+    ++it;
+    first = false;
+    conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
+    run = !conv && it < cap;
+    product(run);
+    failed = uniform(sh.fail != 0u);
+    run = run && !failed;
+  } while (run);
+  if (failed) return fault();
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
     const uint32_t lk = b0 + (uint32_t)t;
@@ -408,7 +415,7 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   if (tid == 0) {
     if (part == 0) {
       if (iters_out) iters_out[inst] = it;
-      if (eta_out) eta_out[inst] = fabsf(eta_last);
+      if (eta_out) eta_out[inst] = fabsf(eta);
       if (flag_out) flag_out[inst] = conv ? 0u : 1u;
     }
     if (done) atomicAdd(done + inst, 1u);

@@ -160,8 +160,9 @@ static uint32_t sqp_pcg_cap(const mpc_config &c) {
 
 
 
-// PCG of one instance: resident kernel when its Schur system fits one
-// workgroup, a two-workgroup team up to twice that, streaming otherwise.
+// PCG of one instance: the one-workgroup kernel for a lone instance (stair:
+// the resident kernel) when its Schur system fits one workgroup, a team of
+// two or four up to four times that, streaming otherwise.
 static hipError_t pcg_single(mpc_handle *h, uint32_t N, const float *S, const float *P, const float *gamma,
                              float *lambda, uint32_t max_iter, float tol, uint32_t *iters, uint32_t *flag,
                              hipStream_t st) {
@@ -171,6 +172,8 @@ static hipError_t pcg_single(mpc_handle *h, uint32_t N, const float *S, const fl
                                h->cfg.direct_refine, true, iters, flag, st);
   const bool stair = flags & FLAG_PCG_STAIR;
   if (!(flags & FLAG_PCG_STREAM)) {
+    if (N <= pcg_lone_max_knots() && !stair)
+      return launch_pcg_lone(N, S, P, gamma, lambda, max_iter, tol, iters, flag, h->pcg_eta, st);
     if (N <= pcg_res_max_knots(512))
       return launch_pcg_res(single(N), nullptr, nullptr, 0, 1, 512, S, P, gamma, lambda, max_iter, tol, nullptr,
                             iters, flag, h->pcg_eta, stair, st);

@@ -91,10 +91,14 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
+// a condition that has the same value in every lane of the wave, in a scalar
+// register (a branch on it leaves EXEC alone)
+__device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
+
 // Registers of one block row (knot k of the instance starting at global
 // knot K0) for lane i; zeros for absent rows and lanes >= 14.  Also writes
 // L_k = S(k,k-1) pre-rotated into the LDS slot Ls (lanes i < 14; zeros for
-// k = 0).
+// k = 0).  One branch for the row's 48 reads, none between them.
 struct RowRegs {
   float D[16], P[16];
 };
@@ -102,17 +106,26 @@ struct RowRegs {
 __device__ __forceinline__ void load_row(RowRegs &R, float *Ls, bool has, uint32_t i, uint32_t d,
                                          const float *__restrict__ S, const float *__restrict__ Pinv,
                                          uint32_t K0, uint32_t k) {
-  const bool row = has && i < (uint32_t)NX;
   const float *Sb = S + (size_t)S_STRIDE * (K0 + k);
   const float *Pb = Pinv + (size_t)S_STRIDE * (K0 + k);
-  const bool left = row && k > 0;
 #pragma unroll
-  for (int n = 0; n < 16; ++n) {
-    const uint32_t j = (i + (uint32_t)n * d) & 15u;
-    const bool col = j < (uint32_t)NX;
-    R.D[n] = row && col ? Sb[NXX + i + NX * j] : 0.f;
-    R.P[n] = row && col ? Pb[NXX + i + NX * j] : 0.f;
-    if (row) Ls[i * L_LANE + n] = left && col ? Sb[i + NX * j] : 0.f;
+  for (int n = 0; n < 16; ++n) R.D[n] = R.P[n] = 0.f;
+  if (has && i < (uint32_t)NX) {
+    float l[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      const uint32_t j = (i + (uint32_t)n * d) & 15u, at = i + (j < (uint32_t)NX ? NX * j : 0u);
+      R.D[n] = Sb[NXX + at];
+      R.P[n] = Pb[NXX + at];
+      l[n] = Sb[at];
+    }
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      const bool col = ((i + (uint32_t)n * d) & 15u) < (uint32_t)NX;
+      R.D[n] = col ? R.D[n] : 0.f;
+      R.P[n] = col ? R.P[n] : 0.f;
+      Ls[i * L_LANE + n] = col && k > 0 ? l[n] : 0.f;
+    }
   }
 }
 
@@ -126,30 +139,66 @@ __device__ __forceinline__ void read_lrow(float (&Lr)[16], const float *Ls, uint
   }
 }
 
-// (L^T x)_i from the rotated rows Lr of L held by the lanes of the row.
-// The products are formed first so that no DPP read directly follows the
-// VALU write of its source; two partial sums (odd / even n) shorten the
-// dependency chain.
-__device__ __forceinline__ float rot_mtv(const float (&Lr)[16], float x) {
-  float m[16];
-#pragma unroll
-  for (int n = 0; n < 16; ++n) m[n] = Lr[(16 - n) & 15] * x;
-  float a = m[0], b = dpp_f<0x121>(m[1]);
-  a += dpp_f<0x122>(m[2]);
-  b += dpp_f<0x123>(m[3]);
-  a += dpp_f<0x124>(m[4]);
-  b += dpp_f<0x125>(m[5]);
-  a += dpp_f<0x126>(m[6]);
-  b += dpp_f<0x127>(m[7]);
-  a += dpp_f<0x128>(m[8]);
-  b += dpp_f<0x129>(m[9]);
-  a += dpp_f<0x12A>(m[10]);
-  b += dpp_f<0x12B>(m[11]);
-  a += dpp_f<0x12C>(m[12]);
-  b += dpp_f<0x12D>(m[13]);
-  a += dpp_f<0x12E>(m[14]);
-  b += dpp_f<0x12F>(m[15]);
-  return a + b;
+// (D x + L xl) + M^T xr of one knot, M the rows of the next knot's left
+// block: two direct chains, and the contributions of M's rows (header) in an
+// even and an odd sum, m_0 + ror_2(m_2) of the even one a multiply-add; all
+// four taken together step by step.  A pair of steps n, n + 1 (n odd): the products
+// of the contributions come first, so that each DPP read is at least two
+// instructions behind the write of what it reads.
+#define MPC_DPPM " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define MPC_PAIR(n, n1)                                                                                       \
+  asm("v_mul_f32 %4, %13, %8\n"                                                                               \
+      "v_mul_f32 %5, %14, %8\n"                                                                               \
+      "v_fmac_f32_dpp %0, %6, %9 row_ror:" #n MPC_DPPM                                                        \
+      "v_fmac_f32_dpp %1, %7, %11 row_ror:" #n MPC_DPPM                                                       \
+      "v_add_f32_dpp %3, %4, %3 row_ror:" #n MPC_DPPM                                                         \
+      "v_fmac_f32_dpp %0, %6, %10 row_ror:" #n1 MPC_DPPM                                                      \
+      "v_fmac_f32_dpp %1, %7, %12 row_ror:" #n1 MPC_DPPM                                                      \
+      "v_add_f32_dpp %2, %5, %2 row_ror:" #n1 MPC_DPPM                                                        \
+      : "+v"(yd), "+v"(yl), "+v"(a), "+v"(b), "=&v"(t0), "=&v"(t1)                                            \
+      : "v"(x), "v"(xl), "v"(xr), "v"(D[n]), "v"(D[n1]), "v"(L[n]), "v"(L[n1]), "v"(M[16 - n]), "v"(M[16 - n1]))
+__device__ __forceinline__ float row_product(const float (&D)[16], float x, const float (&L)[16], float xl,
+                                             const float (&M)[16], float xr) {
+  float yd = D[0] * x, yl = L[0] * xl, a, b, t0 = M[15] * xr, t1 = M[14] * xr;
+  asm("s_nop 1\n"
+      "v_fmac_f32_dpp %0, %4, %8 row_ror:1" MPC_DPPM
+      "v_fmac_f32_dpp %1, %5, %10 row_ror:1" MPC_DPPM
+      "v_mov_b32_dpp %3, %6 row_ror:1" MPC_DPPM
+      "v_mov_b32_dpp %2, %7 row_ror:2" MPC_DPPM
+      "v_fmac_f32_dpp %0, %4, %9 row_ror:2" MPC_DPPM
+      "v_fmac_f32_dpp %1, %5, %11 row_ror:2" MPC_DPPM
+      "v_fmac_f32 %2, %12, %13\n"
+      : "+v"(yd), "+v"(yl), "=&v"(a), "=&v"(b)
+      : "v"(x), "v"(xl), "v"(t0), "v"(t1), "v"(D[1]), "v"(D[2]), "v"(L[1]), "v"(L[2]), "v"(M[0]), "v"(xr));
+  MPC_PAIR(3, 4);
+  MPC_PAIR(5, 6);
+  MPC_PAIR(7, 8);
+  MPC_PAIR(9, 10);
+  MPC_PAIR(11, 12);
+  MPC_PAIR(13, 14);
+  asm("v_mul_f32 %3, %8, %9\n"
+      "v_fmac_f32_dpp %0, %4, %6 row_ror:15" MPC_DPPM
+      "v_fmac_f32_dpp %1, %5, %7 row_ror:15" MPC_DPPM
+      "v_add_f32_dpp %2, %3, %2 row_ror:15" MPC_DPPM
+      : "+v"(yd), "+v"(yl), "+v"(b), "=&v"(t0)
+      : "v"(x), "v"(xl), "v"(D[15]), "v"(L[15]), "v"(M[1]), "v"(xr));
+  return (yd + yl) + (a + b);
+}
+#undef MPC_PAIR
+#undef MPC_DPPM
+
+// z = P r
+__device__ __forceinline__ float row_precond(const float (&P)[16], float r) {
+  float z = P[0] * r;
+#define MPC_RP(n, k) "v_fmac_f32_dpp %0, %1, %" #k " row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+  asm("s_nop 1\n" MPC_RP(1, 2) MPC_RP(2, 3) MPC_RP(3, 4) MPC_RP(4, 5) MPC_RP(5, 6) MPC_RP(6, 7) MPC_RP(7, 8)
+          MPC_RP(8, 9) MPC_RP(9, 10) MPC_RP(10, 11) MPC_RP(11, 12) MPC_RP(12, 13) MPC_RP(13, 14) MPC_RP(14, 15)
+              MPC_RP(15, 16)
+      : "+v"(z)
+      : "v"(r), "v"(P[1]), "v"(P[2]), "v"(P[3]), "v"(P[4]), "v"(P[5]), "v"(P[6]), "v"(P[7]), "v"(P[8]), "v"(P[9]),
+        "v"(P[10]), "v"(P[11]), "v"(P[12]), "v"(P[13]), "v"(P[14]), "v"(P[15]));
+#undef MPC_RP
+  return z;
 }
 
 // y = S x for the RK consecutive knots of a group: Ls0 is the LDS slot of
@@ -159,27 +208,23 @@ __device__ __forceinline__ float rot_mtv(const float (&Lr)[16], float x) {
 template <int RK>
 __device__ __forceinline__ void group_smv(const RowRegs (&R)[RK], const float *Ls0, uint32_t i, const float (&x)[RK],
                                           float xm, float xp, float (&y)[RK]) {
-  float La[16], Lb[16];
-  read_lrow(La, Ls0, i);
+  // three buffers: the rows of slot t + 2 are read while knot t's products,
+  // which take those of slots t and t + 1, run
+  float L[3][16];
+  read_lrow(L[0], Ls0, i);
+  read_lrow(L[1], Ls0 + L_SLOT, i);
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
-    float(&Lc)[16] = (t & 1) ? Lb : La;  // L_b rows of knot t
-    float(&Ln)[16] = (t & 1) ? La : Lb;  // rows of knot t + 1
-    read_lrow(Ln, Ls0 + (t + 1) * L_SLOT, i);
-    const float xl = t > 0 ? x[t - 1] : xm, xr = t < RK - 1 ? x[t + 1] : xp;
-    float a, bm;
-    rot_mv2(R[t].D, x[t], a, Lc, xl, bm);
-    const float bp = rot_mtv(Ln, xr);
-    y[t] = (a + bm) + bp;
+    if (t + 2 <= RK) read_lrow(L[(t + 2) % 3], Ls0 + (t + 2) * L_SLOT, i);
+    y[t] = row_product(R[t].D, x[t], L[t % 3], t > 0 ? x[t - 1] : xm, L[(t + 1) % 3], t < RK - 1 ? x[t + 1] : xp);
   }
 }
 
-// z = Pinv r for the RK knots of a group, two interleaved chains at a time
+// z = Pinv r for the RK knots of a group
 template <int RK>
 __device__ __forceinline__ void group_precond(const RowRegs (&R)[RK], const float (&r)[RK], float (&z)[RK]) {
-  static_assert(RK % 2 == 0, "knots are taken in pairs");
 #pragma unroll
-  for (int t = 0; t < RK; t += 2) rot_mv2(R[t].P, r[t], z[t], R[t + 1].P, r[t + 1], z[t + 1]);
+  for (int t = 0; t < RK; ++t) z[t] = row_precond(R[t].P, r[t]);
 }
 
 }  // namespace onchip

@@ -26,6 +26,12 @@
 //   copies of the neighbouring groups' elements p_{4lg-1}[i], p_{4lg+4}[i]
 //   (the same fused multiply-add as their owners, so every copy stays
 //   bitwise equal to its owner).
+// The two waves of a SIMD issue their products one after the other (a DPP
+// multiply-add takes 4.5 clocks, a plain one 2.25), so the iteration is bound
+// by issue; branches on values that differ between lanes cost it several
+// hundred clocks in EXEC bookkeeping, so conditions are ballots and the loop
+// has one back branch.  Batch of 300 in stair mode 5.33 -> 3.98 ms, one stair
+// solve of N = 100 1.37 -> 1.24 ms.
 #pragma once
 #include "pcg_onchip.h"
 
@@ -51,14 +57,23 @@ struct ResShared {
   float L[(KNOTS + 1) * L_SLOT + L_GUARD];  // S(b,b-1) per knot slot (+ one zero slot), pre-rotated rows
   float zb[(KNOTS + 1) * 16];         // staged vector element per knot slot and lane
   float wb[(KNOTS + 1) * 16];         // stair preconditioner: staged D^-1 r
-  float red[2][NWAV];
-  uint32_t act[NWAV];
+  // dot-product partials of the waves, by instance of the bin and wave of the
+  // instance (zero past its waves)
+  alignas(16) float red[2][MAXI][NWAV];
+  uint32_t act[MAXI];  // by instance of the bin: 1 while it iterates
+  static_assert(NWAV % 4 == 0, "partials are read as 16-byte words");
   static_assert(((KNOTS + 1) * L_SLOT + L_GUARD) % 4 == 0, "L and zb are cleared as one float4 range");
 };
 
-__device__ __forceinline__ float seg_sum(const float *red, uint32_t w0, uint32_t nw) {
+// the partials in wave order
+template <int NWAV>
+__device__ __forceinline__ float seg_sum(const float (&red)[NWAV]) {
   float s = 0.f;
-  for (uint32_t v = 0; v < nw; ++v) s += red[w0 + v];
+#pragma unroll
+  for (int v = 0; v < NWAV; v += 4) {
+    const float4 x = *reinterpret_cast<const float4 *>(red + v);
+    s = (((s + x.x) + x.y) + x.z) + x.w;
+  }
   return s;
 }
 
@@ -74,7 +89,7 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
                                      float *__restrict__ lambda, uint32_t max_iter, float tol,
                                      const uint32_t *__restrict__ status, uint32_t *__restrict__ iters_out,
                                      uint32_t *__restrict__ flag_out, float *__restrict__ eta_out) {
-  constexpr int NGRP = ResShape<NT>::NGRP, NWAV = ResShape<NT>::NWAV, KNOTS = ResShape<NT>::KNOTS;
+  constexpr int NWAV = ResShape<NT>::NWAV, KNOTS = ResShape<NT>::KNOTS;
   ResShared<NT> &sh = *reinterpret_cast<ResShared<NT> *>(smem);
   const uint32_t g = tid >> 4, i = tid & 15u, w = tid >> 6;
   const uint32_t d = ror_step(tid);
@@ -91,25 +106,28 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
     i0 = bin_off[bin];
     ni = bin_off[bin + 1] - i0;
   }
+  // (whole waves per instance: everything about it is uniform over the wave)
+  const uint32_t ws = (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
   int slot = -1;
-  uint32_t inst = 0, g0 = 0, ng = NGRP;
+  uint32_t inst = 0, g0 = 0;
   const uint32_t ng1 = ((inst_len(b, 0) + RK - 1) / RK + 3u) & ~3u;  // lone instance: as in a bin
   for (uint32_t j = 0; j < ni; ++j) {
     const uint4 it = items ? items[i0 + j] : make_uint4(0u, 0u, ng1, 0u);
-    if (g >= it.y && g < it.y + it.z) {
+    if (4u * ws >= it.y && 4u * ws < it.y + it.z) {
       slot = (int)j;
       inst = it.x;
       g0 = it.y;
-      ng = it.z;
     }
   }
   const bool mine = slot >= 0;
   const uint32_t N = mine ? inst_len(b, inst) : 0u;
   const uint32_t K0 = mine ? inst_first(b, inst) : 0u;
-  const bool live = mine && !(status && !(status[inst] & ST_ACTIVE));
+  const bool live = uniform(mine && !(status && !(status[inst] & ST_ACTIVE)));
   const uint32_t cap = pcg_cap(max_iter, N);
-  const uint32_t lg = g - g0, w0 = g0 >> 2, nw = ng >> 2, lbase = g0 * RK;
+  const uint32_t lg = g - g0, lbase = g0 * RK;
   const bool lane_ok = i < (uint32_t)NX;
+  if (tid < (uint32_t)MAXI) sh.act[tid] = 0u;
+  if (tid < 2u * MAXI * NWAV) (&sh.red[0][0][0])[tid] = 0.f;
   __syncthreads();  // LDS cleared
 
   // ---- load: D, Pinv rows into registers, S(b,b-1) into LDS
@@ -122,6 +140,7 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
     const bool has = live && bk < N;
     load_row(R[t], sh.L + (s0 + t) * L_SLOT, has, i, d, S, Pinv, K0, bk);
     lam[t] = has && lane_ok ? lambda[(size_t)NX * (K0 + bk) + i] : 0.f;
+    r[t] = has && lane_ok ? gamma[(size_t)NX * (K0 + bk) + i] : 0.f;
   }
   // first / last element of the group to LDS; neighbouring groups' copies back
   const bool in_m = lg > 0, in_p = b0 + RK < N;
@@ -130,9 +149,11 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
     zb0[0] = v[0];
     zb0[(RK - 1) * 16] = v[RK - 1];
   };
+  // (the last knot's slot is followed by a zero one, and the first reads it)
+  const float *zm_src = in_m ? zb0 - 16 : sh.zb + KNOTS * 16 + i, *zp_src = in_p ? zb0 + RK * 16 : sh.zb + KNOTS * 16 + i;
   auto neighbours = [&](float &vm, float &vp) {
-    vm = in_m ? zb0[-16] : 0.f;
-    vp = in_p ? zb0[RK * 16] : 0.f;
+    vm = *zm_src;
+    vp = *zp_src;
   };
   // stair preconditioner: the first / last element of w = D^-1 r, the same way
   float *wb0 = sh.wb + s0 * 16 + i;
@@ -140,128 +161,101 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
     wb0[0] = v[0];
     wb0[(RK - 1) * 16] = v[RK - 1];
   };
+  const float *wm_src = in_m ? wb0 - 16 : sh.zb + KNOTS * 16 + i, *wp_src = in_p ? wb0 + RK * 16 : sh.zb + KNOTS * 16 + i;
   auto neighbours_w = [&](float &vm, float &vp) {
-    vm = in_m ? wb0[-16] : 0.f;
-    vp = in_p ? wb0[RK * 16] : 0.f;
+    vm = *wm_src;
+    vp = *wp_src;
   };
   // y = S x for the group's knots; xm / xp: elements of knots 4lg-1, 4lg+4
   auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, sh.L + s0 * L_SLOT, i, x, xm, xp, y); };
+  // an instance's act word: set here, cleared when it stops (its lanes all
+  // write the same, between the second barrier of its last iteration and the
+  // first of the next)
+  if (live) sh.act[slot] = 1u;
   stage(lam);
   __syncthreads();
   float pm, pp;
   neighbours(pm, pp);
 
-  // ---- prologue: r = gamma - S lambda, z = Pinv r, p = z, eta = r.z
-  smv(lam, pm, pp);
-  float part = 0.f;
+  // The first pass is the prologue, through the same code: p = lambda,
+  // r = gamma - S lambda (alpha = 1, lambda kept), z = M r, then p = z
+  // (beta = 0) and eta = r.z; the others are the iterations.  The loop's
+  // only branch is its own, on a scalar condition: with more the compiler
+  // puts all of them on EXEC masks (its divergent stores are none of them).
 #pragma unroll
-  for (int t = 0; t < RK; ++t) {
-    const uint32_t bk = b0 + (uint32_t)t;
-    r[t] = live && bk < N && lane_ok ? gamma[(size_t)NX * (K0 + bk) + i] - y[t] : 0.f;
-  }
-  if constexpr (STAIR) {
-    // z = D^-1 (2 r - S w), w = D^-1 r
-    float wv[RK], v[RK], wm, wp;
-    group_precond<RK>(R, r, wv);
-    stage_w(wv);
-    __syncthreads();
-    neighbours_w(wm, wp);
-    smv(wv, wm, wp);
-#pragma unroll
-    for (int t = 0; t < RK; ++t) v[t] = lane_ok ? 2.f * r[t] - y[t] : 0.f;
-    group_precond<RK>(R, v, z);
-  } else {
-    group_precond<RK>(R, r, z);
-  }
-#pragma unroll
-  for (int t = 0; t < RK; ++t) part += r[t] * z[t];
-  part = wave_sum(part);
-  __syncthreads();  // every neighbour lambda read before zb is reused
-  if ((tid & 63u) == 0) sh.red[1][w] = part;
-  stage(z);
-  __syncthreads();
-  float eta = seg_sum(sh.red[1], w0, nw);
-  neighbours(pm, pp);
-#pragma unroll
-  for (int t = 0; t < RK; ++t) p[t] = z[t];
-  uint32_t it = 0;
-  // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
-  const float tol_i = tol < 0.f ? fmaxf(-tol * fabsf(eta), FLT_MIN) : tol;
-  bool conv = !live || fabsf(eta) < tol_i;
-  float eta_last = eta;  // of the last exit test
-
-  for (;;) {
-    const bool run = live && !conv && it < cap;  // uniform over the instance's waves
-    float pyp = 0.f;
-    if (run) {
+  for (int t = 0; t < RK; ++t) p[t] = lam[t];
+  uint32_t it = ~0u;  // the first pass is not counted
+  float eta = 0.f, tol_i = tol;
+  bool conv = !live;
+  if (live) {
+    float(&red0)[NWAV] = sh.red[0][slot], (&red1)[NWAV] = sh.red[1][slot];
+    const uint32_t wi = ws - (g0 >> 2);  // wave of the instance
+    bool first = true, run;
+    do {
       smv(p, pm, pp);
+      float pyp = 0.f;
 #pragma unroll
       for (int t = 0; t < RK; ++t) pyp += p[t] * y[t];
-      pyp = wave_sum(pyp);
-    }
-    if ((tid & 63u) == 0) {
-      sh.red[0][w] = pyp;
-      sh.act[w] = run ? 1u : 0u;
-    }
-    __syncthreads();
-    uint32_t any = 0;
+      red0[wi] = wave_sum(pyp);  // the wave's lanes write the same value
+      __syncthreads();
+      const float quo = eta / seg_sum(red0), alpha = first ? 1.f : quo;
+      float rz = 0.f;
 #pragma unroll
-    for (int v = 0; v < NWAV; ++v) any |= sh.act[v];
-    if (!any) break;
-    float rz = 0.f;
-    float wv[RK];
-    if (run) {
-      const float alpha = eta / seg_sum(sh.red[0], w0, nw);
-#pragma unroll
-      for (int t = 0; t < RK; ++t) {
-        lam[t] += alpha * p[t];
-        r[t] = lane_ok ? r[t] - alpha * y[t] : 0.f;
-      }
+      for (int t = 0; t < RK; ++t) r[t] -= alpha * y[t];
       if constexpr (STAIR) {
+        // z = D^-1 (2 r - S w), w = D^-1 r
+        float wv[RK], wm, wp;
         group_precond<RK>(R, r, wv);
         stage_w(wv);
-      } else {
-        group_precond<RK>(R, r, z);
-#pragma unroll
-        for (int t = 0; t < RK; ++t) rz += r[t] * z[t];
-        stage(z);
-        rz = wave_sum(rz);
-      }
-    }
-    if constexpr (STAIR) {
-      __syncthreads();  // staged w visible
-      if (run) {
-        float v[RK], wm, wp;
+        __syncthreads();  // staged w visible
         neighbours_w(wm, wp);
         smv(wv, wm, wp);
 #pragma unroll
-        for (int t = 0; t < RK; ++t) v[t] = lane_ok ? 2.f * r[t] - y[t] : 0.f;
-        group_precond<RK>(R, v, z);
-#pragma unroll
-        for (int t = 0; t < RK; ++t) rz += r[t] * z[t];
-        stage(z);
-        rz = wave_sum(rz);
+        for (int t = 0; t < RK; ++t) wv[t] = 2.f * r[t] - y[t];
+        group_precond<RK>(R, wv, z);
+      } else {
+        group_precond<RK>(R, r, z);
       }
-    }
-    if ((tid & 63u) == 0) sh.red[1][w] = rz;
-    __syncthreads();
-    if (run) {
+#pragma unroll
+      for (int t = 0; t < RK; ++t) rz += r[t] * z[t];
+      stage(z);
+      red1[wi] = wave_sum(rz);
+      // lambda += alpha p on the way to the barrier
+      const float alpha_l = first ? 0.f : alpha;
+#pragma unroll
+      for (int t = 0; t < RK; ++t) lam[t] += alpha_l * p[t];
+      __syncthreads();
       float zm, zp;
       neighbours(zm, zp);
-      const float eta_new = seg_sum(sh.red[1], w0, nw);
-      eta_last = eta_new;
-      ++it;
-      if (fabsf(eta_new) < tol_i) {
-        conv = true;
-      } else {
-        const float beta = eta_new / eta;
-        eta = eta_new;
+      const float eta_new = seg_sum(red1);
+      // taken in the last iteration too (p is not used after it)
+      const float quo_b = eta_new / eta, beta = first ? 0.f : quo_b;
+      eta = eta_new;
 #pragma unroll
-        for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], z[t]);
-        pm = fmaf(beta, pm, zm);
-        pp = fmaf(beta, pp, zp);
-      }
-    }
+      for (int t = 0; t < RK; ++t) p[t] = fmaf(beta, p[t], z[t]);
+      pm = fmaf(beta, pm, zm);
+      pp = fmaf(beta, pp, zp);
+      // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
+      tol_i = first && tol < 0.f ? fmaxf(-tol * fabsf(eta), FLT_MIN) : tol_i;
+      ++it;
+      first = false;
+      conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
+      run = !conv && it < cap;
+    } while (run);
+    sh.act[slot] = 0u;
+  }
+  // Waves that iterate no more (or have no instance) keep the others'
+  // barriers until no instance of the bin iterates.  They read the act words
+  // between the first two barriers, where those do not change, so all leave
+  // in the same round.
+  for (;;) {
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int v = 0; v < MAXI; ++v) any |= sh.act[v];
+    if (uniform(any == 0u)) break;
+    if constexpr (STAIR) __syncthreads();
+    __syncthreads();
   }
 
   if (!live) return;
@@ -271,7 +265,7 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
   if (lg == 0 && i == 0) {
     if (iters_out) iters_out[inst] = it;
     if (flag_out) flag_out[inst] = conv ? 0u : 1u;
-    if (eta_out) eta_out[inst] = fabsf(eta_last);
+    if (eta_out) eta_out[inst] = fabsf(eta);
   }
 }
 

@@ -107,22 +107,25 @@ struct Params {
   unsigned long long budget_ticks;
 };
 
-// mailbox of a PCG team of up to 4 workgroups: per buffer and part, 40
-// self-validating words {epoch (high 32 bits), float bits (low 32 bits)}:
-// words 0..7 the partial sums of the part's 8 waves, 8..21 the vector
-// elements of its first row (for the part before it), 24..37 of its last
-// row (for the part after it).  Epoch e of a solve uses buffer
-// 4 set + (e mod 4).  Four buffers per set: a part overwrites the words of
-// epoch e only when it posts epoch e + 4, and between the two it has
-// waited for the partials of every wave of every other part at an
-// all-to-all epoch, which each wave posts only after its reads of epoch e
-// (no two consecutive epochs are rows-only exchanges).  Two sets: the
-// persistent pool alternates them between the consecutive teams of a slot.
-// `next` carries the pool's team index from part 0 to part 1 {round, index}.
-struct TeamMailbox {
-  unsigned long long w[8][4][40];
+// mailbox of a PCG team of up to 4 workgroups: per buffer, self-validating
+// words {epoch (high 32 bits), float bits (low 32 bits)}: words 0..3 the dot
+// product sums of the parts (one 128-byte line, all that most waves read),
+// then per part two lines with the vector elements of its first row (for the
+// part before it) and of its last row (for the part after it).  Epoch e of a
+// solve uses buffer 4 set + (e mod 4).  Four buffers per set: a part
+// overwrites the words of epoch e only when it posts epoch e + 4, and between
+// the two it has waited for the sum of every other part at an all-to-all
+// epoch, which that part posts behind a workgroup barrier that all its reads
+// of epoch e precede (no two consecutive epochs are rows-only exchanges).
+// Two sets: the persistent pool alternates them between the consecutive teams
+// of a slot.  `next` carries the pool's team index from part 0 to part 1
+// {round, index}.
+struct alignas(128) TeamMailbox {
+  static constexpr uint32_t ROWS = 16, PART = 32, LAST = 16;  // first row word, words per part, offset of the last row
+  unsigned long long w[8][160];
   unsigned long long next;
 };
+static_assert(TeamMailbox::ROWS + 4 * TeamMailbox::PART <= 160, "mailbox layout");
 
 // work queues of the persistent PCG pool (k_pcg_pool), one cache line each
 struct PoolCounters {

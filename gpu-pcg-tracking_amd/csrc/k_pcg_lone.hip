@@ -71,23 +71,6 @@ __device__ __forceinline__ float low_to_high(float v) {
   return __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_permlane32_swap(u, u, false, false)[0]);
 }
 
-// rotated rows of the column-major 14 x 14 block at base + off (floats);
-// zeros where ok is false and for columns and lanes past 13
-__device__ __forceinline__ void load_block(float (&R)[16], bool ok, uint32_t i, uint32_t d, const float *__restrict__ base,
-                                           uint32_t off) {
-#pragma unroll
-  for (int n = 0; n < 16; ++n) R[n] = 0.f;
-  if (ok) {
-#pragma unroll
-    for (int n = 0; n < 16; ++n) {
-      const uint32_t j = (i + (uint32_t)n * d) & 15u;
-      R[n] = base[off + i + (j < (uint32_t)NX ? NX * j : 0u)];
-    }
-#pragma unroll
-    for (int n = 0; n < 16; ++n) R[n] = ((i + (uint32_t)n * d) & 15u) < (uint32_t)NX ? R[n] : 0.f;
-  }
-}
-
 template <int KR>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pinv, const float *__restrict__ gamma,
@@ -106,19 +89,16 @@ k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pi
   const bool lane_ok = i < (uint32_t)NX;
   const uint32_t cap = pcg_cap(max_iter, N);
 
-  float D[KR][16], P[KR][16], L[KR + 1][16];
+  Rows<KR> R;
+  R.load(S, Pinv, b0, N, N, i, d);
   float lam[KR], r[KR], p[KR], y[KR], z[KR];
 #pragma unroll
   for (int t = 0; t < KR; ++t) {
     const uint32_t k = b0 + (uint32_t)t;
     const bool has = lane_ok && k < N;
-    load_block(D[t], has, i, d, S, S_STRIDE * k + NXX);
-    load_block(P[t], has, i, d, Pinv, S_STRIDE * k + NXX);
-    load_block(L[t], has && k > 0, i, d, S, S_STRIDE * k);
     lam[t] = has ? lambda[NX * k + i] : 0.f;
     r[t] = has ? gamma[NX * k + i] : 0.f;
   }
-  load_block(L[KR], lane_ok && b0 + KR < N, i, d, S, S_STRIDE * (b0 + KR));
   __syncthreads();  // LDS cleared
   // the row's first and last knot staged, its neighbours' read
   float *zb0 = sh.zb + (b0 + 1u) * 16u + i;
@@ -200,16 +180,15 @@ k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pi
   float eta = 0.f, tol_i = tol;
   bool first = true, conv, run;
   do {
-#pragma unroll
-    for (int t = 0; t < KR; ++t)
-      y[t] = row_product(D[t], p[t], L[t], t > 0 ? p[t - 1] : pm, L[t + 1], t < KR - 1 ? p[t + 1] : pp);
+    group_smv<KR>(R, p, pm, pp, y);
     post(0, group_dot(p, y));
     __syncthreads();
     const float quo = eta / total(0), alpha = first ? 1.f : quo;
+    // (knot by knot: all updates first cost 1 % of a solve)
 #pragma unroll
     for (int t = 0; t < KR; ++t) {
       r[t] -= alpha * y[t];
-      z[t] = row_precond(P[t], r[t]);
+      z[t] = row_precond(R.P[t], r[t]);
     }
     stage(z);
     post(1, group_dot(r, z));

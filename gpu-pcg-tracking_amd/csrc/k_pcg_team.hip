@@ -5,9 +5,9 @@
 //
 // Part p owns knots [p C, min(N, (p+1) C)), C = ceil(N/Q) rounded up to a
 // multiple of 4 (at most 128); each workgroup's 32 groups of 16 lanes serve 4
-// consecutive knots each (local knot 4 g + t).  Every part but the last also
-// keeps L_ke = S(ke, ke-1) of the next part's first knot in the LDS slot
-// after its own, for its last row's S(ke-1, ke) p_ke term.  The knots next
+// consecutive knots each (local knot 4 g + t) and hold L of the knot after
+// them, which may be the next part's first.  lambda alone lives in LDS, for
+// want of registers.  The knots next
 // to a split (the last of a part's last group, the first of the next part's
 // group 0) take their outer neighbour's vector element from that part.
 //
@@ -15,21 +15,26 @@
 // carries the rows of w = D^-1 r at the splits for the extra block product.
 //
 // Exchange through an L2 mailbox, twice per iteration (p.Sp, then r.z with
-// z of the rows next to the splits): before the workgroup barrier that
-// publishes the wave partials in LDS, every wave also posts its partial to
-// the mailbox, and the boundary groups post their rows; after the barrier
-// every wave polls the other parts' partials itself (the boundary waves also
-// the rows they need), so no second barrier is needed.  Totals are
+// z of the rows next to the splits): the boundary groups post their rows
+// before the workgroup barrier that publishes the wave partials in LDS;
+// after it every wave sums them, one wave posts the part's sum, and every
+// wave polls the other parts' sums itself (the boundary waves also the rows
+// they need), so no second barrier is needed.  The sums of all parts are one
+// 128-byte line: with 256 workgroups polling, the reads of a wave's line
+// count (a line per part with the partials of its waves, posted before the
+// barrier, was no slower for one team and 11 % slower for 64 at once).  Totals are
 // ((part 0 + part 1) + part 2) + part 3, each part's the sum of its waves in
 // wave order, on every part, so all parts take identical decisions.  Same
 // algorithm and exit rule as k_pcg.hip (GPU-PCG pcg<T,14,N>,
 // toplevel.cuh:143-157).
 //
-// Of the 8500 clocks of an iteration at 128 knots a part, products and
-// preconditioner take some 3700 (issue of two waves per SIMD), the two
-// exchanges 1100 - 1400 each.  173 iterations, with divergent loop conditions
-// and a readlane ahead of every addition of a total / now: N = 256 642 / 618
-// us, N = 512 758 / 649 us; stair 1182 / 888 us, 1437 / 941 us.
+// Of the 7000 clocks of an iteration at 128 knots a part, products and
+// preconditioner take some 2600 (issue of two waves per SIMD), the two
+// exchanges 1100 - 1400 each.  173 iterations of one team: N = 256 642 us with
+// divergent loop conditions and totals by readlanes in a chain, 618 without,
+// 515 with S(b,b-1) in registers instead of LDS; N = 512 758, 649, 528; stair
+// 1182, 888, 782 and 1437, 941, 791.  Batch of 4096 with horizons to 512: 107,
+// 95, 80 ms.
 //
 // Two launch forms, both cooperative (all workgroups co-resident):
 // - k_pcg_team: one team per Q workgroups; more teams than fit at once are
@@ -78,86 +83,57 @@ constexpr int NGRP = NT / 16;  // 32 groups
 constexpr int NWAV = NT / 64;  // 8 waves
 constexpr int RK = 4;
 constexpr int KNOTS = NGRP * RK;  // knots per part
-constexpr uint32_t SPIN_LIMIT = 1u << 16;
-// mailbox words of a part: 0..7 wave partials, MB_FIRST.. its first row,
-// MB_LAST.. its last row; lanes of a polling wave: 0..7, 16..23 and 8..15 the
-// partials of the first, second and third other part, LANE_M.. the row before
-// the part, LANE_P.. the row after
-constexpr uint32_t MB_FIRST = 8, MB_LAST = 24, LANE_M = 32, LANE_P = 48;
-static_assert(MB_FIRST == NWAV && MB_LAST >= MB_FIRST + NX && MB_LAST + NX <= 40, "mailbox layout");
-static_assert(24 <= LANE_M && LANE_M + NX <= LANE_P && LANE_P + NX <= 64, "polling lanes");
+constexpr uint32_t SPIN_LIMIT = 3u << 15;  // some 25 ms of reads
+// lanes of a polling wave: 0..3 the sums of the parts, 32.. the row before
+// the part, 48.. the row after; lane 15 posts the sum
+constexpr uint32_t LANE_M = 32, LANE_P = 48, LANE_SUM = 15;
 
 struct TeamShared {
-  float L[(KNOTS + 1) * L_SLOT + L_GUARD];
-  float zb[(KNOTS + 1) * 16];
+  float zb[(KNOTS + 1) * 16];  // staged vector element per knot slot and lane, and a zero slot
   float wb[(KNOTS + 1) * 16];  // stair preconditioner: staged D^-1 r
+  float lam[KNOTS * 16];       // lambda by local knot and lane (registers are short)
   alignas(16) float red[2][NWAV];
-  float recv[2][16];  // rows from the part before / after
   uint32_t fail;
 };
-static_assert(((KNOTS + 1) * L_SLOT + L_GUARD) % 4 == 0, "L and zb are cleared as one float4 range");
 
 __device__ __forceinline__ float sum8(const float *red) {
   const float4 x = *reinterpret_cast<const float4 *>(red), y = *reinterpret_cast<const float4 *>(red + 4);
   return ((((((x.x + x.y) + x.z) + x.w) + y.x) + y.y) + y.z) + y.w;
 }
 
-// per row of the wave, x of its lanes 0..7 (HIGH: 8..15) summed in lane order
-// (the order of sum8), in every lane of the row: eight DPP additions, the
-// broadcast in each (a readlane ahead of every addition took 115 clocks a term)
-template <bool HIGH>
-__device__ __forceinline__ float row_sum8(float x) {
-  float s;
-#define MPC_RS(op, l) op "_dpp %0, %1, %0 row_newbcast:" #l " row_mask:0xf bank_mask:0xf\n"
-  if constexpr (!HIGH)
-    asm("s_nop 1\nv_mov_b32_dpp %0, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n" MPC_RS("v_add_f32", 1)
-            MPC_RS("v_add_f32", 2) MPC_RS("v_add_f32", 3) MPC_RS("v_add_f32", 4) MPC_RS("v_add_f32", 5)
-                MPC_RS("v_add_f32", 6) MPC_RS("v_add_f32", 7) "s_nop 1"
-        : "=&v"(s)
-        : "v"(x));
-  else
-    asm("s_nop 1\nv_mov_b32_dpp %0, %1 row_newbcast:8 row_mask:0xf bank_mask:0xf\n" MPC_RS("v_add_f32", 9)
-            MPC_RS("v_add_f32", 10) MPC_RS("v_add_f32", 11) MPC_RS("v_add_f32", 12) MPC_RS("v_add_f32", 13)
-                MPC_RS("v_add_f32", 14) MPC_RS("v_add_f32", 15) "s_nop 1"
-        : "=&v"(s)
-        : "v"(x));
-#undef MPC_RS
-  return s;
-}
-
 __device__ __forceinline__ float lane_of(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
+
+typedef __attribute__((address_space(1))) unsigned long long MailWord;  // in global memory
 
 // tag_xor: 0, or a bit pattern that makes the tag wrong (the poison hook)
 // buffer of epoch e in the set `set` (0 or 1) of the mailbox
 __device__ __forceinline__ uint32_t mb_buf(uint32_t set, uint32_t e) { return (set << 2) | (e & 3u); }
 
-__device__ __forceinline__ void mb_post(TeamMailbox *mb, uint32_t set, uint32_t part, uint32_t e, uint32_t word,
-                                        float v, uint32_t tag_xor) {
-  __hip_atomic_store(&mb->w[mb_buf(set, e)][part][word],
-                     ((unsigned long long)(e ^ tag_xor) << 32) | __float_as_uint(v), __ATOMIC_RELAXED,
+__device__ __forceinline__ void mb_post(MailWord *dst, uint32_t tag, float v) {
+  __hip_atomic_store(dst, ((unsigned long long)tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Lanes with `want` wait for the mailbox word at src to carry epoch e and
-// return its value (0 in other lanes, whose src is not read); ok is cleared
-// when a word did not arrive in time.  Every mailbox word carries its epoch,
-// so a word is taken only once its tag shows the current epoch.
-__device__ __forceinline__ float mb_wait(const unsigned long long *src, bool want, uint32_t e, bool &ok) {
-  bool got = !want;
-  unsigned long long v = 0;
-  uint32_t spins = 0;
-  while (!__all(got)) {
-    if (!got) {
-      v = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      got = (uint32_t)(v >> 32) == e;
-    }
-    if (++spins > SPIN_LIMIT) break;
-    if (!__all(got)) __builtin_amdgcn_s_sleep(1);
-  }
-  if (!__all(got)) ok = false;
-  return want ? __uint_as_float((uint32_t)v) : 0.f;
+// Lanes with `want` wait for the mailbox word src[word] to carry epoch e and
+// return its value (0 in other lanes, whose word is read but not looked at);
+// late is set when a word did not arrive in time.  Every mailbox word carries
+// its epoch, so a word is taken only once its tag shows the current epoch.
+__device__ __forceinline__ float mb_wait(const MailWord *src, uint32_t word, bool want, uint32_t e,
+                                         bool &late) {
+  auto read = [&]() { return __hip_atomic_load(src + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  bool wait = true;
+  float v = 0.f;
+  unsigned long long got = __builtin_amdgcn_ballot_w64(!want);
+  auto take = [&](unsigned long long x) {
+    v = want && (uint32_t)(x >> 32) == e ? __uint_as_float((uint32_t)x) : v;
+    got |= __builtin_amdgcn_ballot_w64((uint32_t)(x >> 32) == e);
+    wait = ~got != 0;  // some lane still waits
+  };
+  for (uint32_t spins = 0; wait && spins <= SPIN_LIMIT; ++spins) take(read());
+  late = late || wait;
+  return v;
 }
 
 // Part `part` of the PCG of team `team` (instance team_inst[team]) on a
@@ -175,7 +151,8 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
                                            float *__restrict__ eta_out, uint32_t *__restrict__ done,
                                            uint32_t *__restrict__ err, uint32_t poison) {
   TeamShared &sh = *reinterpret_cast<TeamShared *>(smem);
-  const uint32_t g = tid >> 4, i = tid & 15u, w = tid >> 6, lane64 = tid & 63u;
+  const uint32_t g = tid >> 4, i = tid & 15u, lane64 = tid & 63u;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t d = ror_step(tid);
   static_assert(Q == 2 || Q == 4, "teams of 2 or 4 workgroups");
   const uint32_t inst = team_inst[team];
@@ -189,140 +166,121 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   const uint32_t cap = pcg_cap(max_iter, N);
   const bool has_prev = part > 0, has_next = ke < N;
 
-  {
-    float4 *z4 = reinterpret_cast<float4 *>(sh.L);
-    constexpr uint32_t n4 = ((KNOTS + 1) * L_SLOT + L_GUARD + (KNOTS + 1) * 16) / 4;
-    for (uint32_t idx = tid; idx < n4; idx += NT) z4[idx] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tid == 0) sh.fail = 0u;
-    if (tid < 32u) (&sh.recv[0][0])[tid] = 0.f;  // lanes 14, 15 stay zero
-  }
-  __syncthreads();
-  // every part but the last: L_ke into the slot after its own knots
-  if (has_next && g == 0 && lane_ok) {
-    const float *Sn = S + (size_t)S_STRIDE * (K0 + ke);
-    float *Ls = sh.L + n_own * L_SLOT;
-#pragma unroll
-    for (int n = 0; n < 16; ++n) {
-      const uint32_t j = (i + (uint32_t)n * d) & 15u;
-      Ls[i * L_LANE + n] = j < (uint32_t)NX ? Sn[i + NX * j] : 0.f;
-    }
-  }
+  if (tid < 16u) sh.zb[KNOTS * 16 + tid] = 0.f;  // the zero slot
+  if (tid == 0) sh.fail = 0u;
 
   const uint32_t b0 = g * RK;  // first local knot of the group (and its slot)
-  RowRegs R[RK];
-  float lam[RK], r[RK], p[RK], y[RK], z[RK];
+  Rows<RK> R;
+  R.load(S + (size_t)S_STRIDE * K0, Pinv + (size_t)S_STRIDE * K0, kb + b0, ke, N, i, d);
+  float *lam = sh.lam + b0 * 16 + i;
+  float r[RK], p[RK], y[RK], z[RK];
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
     const uint32_t lk = b0 + (uint32_t)t;
-    const bool has = lk < n_own;
-    load_row(R[t], sh.L + lk * L_SLOT, has, i, d, S, Pinv, K0, kb + lk);
-    lam[t] = has && lane_ok ? lambda[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
-    r[t] = has && lane_ok ? gamma[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
+    const bool has = lk < n_own && lane_ok;
+    p[t] = has ? lambda[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
+    lam[t * 16] = p[t];
+    r[t] = has ? gamma[(size_t)NX * (K0 + kb + lk) + i] : 0.f;
   }
+  __syncthreads();  // LDS cleared
   // the group's outer neighbours: in the own zb, from the next / previous
   // part, or none
   const bool own_m = g > 0 && b0 < n_own, own_p = b0 + RK < n_own;
   const bool far_m = has_prev && g == 0, far_p = has_next && b0 + RK == n_own;
   const uint32_t gl = n_own / RK - 1u, wl = gl >> 2;  // last group / its wave (n_own % RK == 0 with has_next)
-  const bool first_lane = has_prev && g == 0 && lane_ok, last_lane = has_next && g == gl && lane_ok;
   float *zb0 = sh.zb + b0 * 16 + i;
   uint32_t e = e0;  // mailbox epoch
-  bool ok = true;
-  // a wait timed out somewhere in the workgroup: the solve is abandoned
-  // (this part is not counted in `done`, so the instance gets PCG_FLAG_FAULT)
-  auto fault = [&]() { return false; };
-  // own first / last element to LDS, the rows at the splits to the mailbox
-  auto post_rows = [&](const float (&v)[RK]) {
-    if (first_lane) mb_post(mb, set, part, e, MB_FIRST + i, v[0], tag_xor);
-    if (last_lane) mb_post(mb, set, part, e, MB_LAST + i, v[RK - 1], tag_xor);
+  bool late = false;  // a wait of this wave ran out
+  // the epoch's buffer, as a scalar the compiler does not take apart (lanes
+  // then address it by one 32-bit offset each)
+  auto buffer = [&]() {
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)mb_buf(set, e));
+    MailWord *p = (MailWord *)&mb->w[k][0];
+    asm("" : "+s"(p));
+    return p;
   };
+  // own words to the mailbox: the part's sum, and the rows next to the splits
+  // (never under a valid tag what a wave computed after a wait ran out: the
+  // other parts then run out of time too, and leave)
+  auto post_sum = [&](float sum) {
+    if (w == 0 && lane64 == LANE_SUM) mb_post(buffer() + part, e ^ tag_xor, sum);
+  };
+  const bool first_lane = far_m && lane_ok, last_lane = far_p && lane_ok;
+  const uint32_t own_word = TeamMailbox::ROWS + part * TeamMailbox::PART + (last_lane ? TeamMailbox::LAST : 0u) + i;
+  auto post_rows = [&](const float (&v)[RK]) {
+    if (first_lane || last_lane) mb_post(buffer() + own_word, e ^ (late ? 0x80000000u : tag_xor), last_lane ? v[RK - 1] : v[0]);
+  };
+  // own first / last element to LDS
   auto stage = [&](const float (&v)[RK]) {
     zb0[0] = v[0];
     zb0[(RK - 1) * 16] = v[RK - 1];
-    post_rows(v);
   };
-  // after the barrier: the other parts' partials (every wave) and, when the
+  // after the barrier: the other parts' sums (every wave) and, when the
   // exchange carries them, the rows next to the part (the waves of group 0
-  // and of the last group, into sh.recv); returns the partial lanes
-  // each polling lane's role and mailbox word (within one epoch's parity):
-  // 1 = a partial of another part, 2 = the row before the part (wave 0),
-  // 3 = the row after it (wave wl)
-  constexpr uint32_t PART_WORDS = sizeof(TeamMailbox{}.w[0][0]) / sizeof(unsigned long long);  // 40
-  uint32_t role = 0, word = 0;
-  if (lane64 < 8u || (Q == 4 && lane64 < 24u)) {
-    const uint32_t q = lane64 < 8u ? 0u : lane64 < 16u ? 2u : 1u;
-    role = 1u;
-    word = (q < part ? q : q + 1u) * PART_WORDS + (lane64 & 7u);
-  } else if (has_prev && w == 0 && lane64 >= LANE_M && lane64 < LANE_M + NX) {
-    role = 2u;
-    word = (part - 1u) * PART_WORDS + MB_LAST + lane64 - LANE_M;
-  } else if (has_next && w == wl && lane64 >= LANE_P && lane64 < LANE_P + NX) {
-    role = 3u;
-    word = (part + 1u) * PART_WORDS + MB_FIRST + lane64 - LANE_P;
-  }
-  auto collect = [&](bool partials, bool rows) {
-    const bool rm = rows && has_prev && w == 0, rp = rows && has_next && w == wl;
+  // and of the last group); returns what each lane read
+  const bool gets_sum = lane64 < (uint32_t)Q && lane64 != part;
+  const bool gets_m = has_prev && w == 0 && lane64 >= LANE_M && lane64 < LANE_M + NX;
+  const bool gets_p = has_next && w == wl && lane64 >= LANE_P && lane64 < LANE_P + NX;
+  const uint32_t word = gets_m   ? TeamMailbox::ROWS + (part - 1u) * TeamMailbox::PART + TeamMailbox::LAST + lane64 - LANE_M
+                        : gets_p ? TeamMailbox::ROWS + (part + 1u) * TeamMailbox::PART + lane64 - LANE_P
+                                 : lane64 & 3u;
+  auto collect = [&](bool sums, bool rows) {
     // after a wait that ran out nothing more is waited for
-    const bool want = ok && ((role == 1u && partials) || (role == 2u && rows) || (role == 3u && rows));
-    float x = 0.f;
-    if (partials || rm || rp) {
-      x = mb_wait(&mb->w[mb_buf(set, e)][0][0] + word, want, e, ok);
-      if (want && role == 2u) sh.recv[0][lane64 - LANE_M] = x;
-      if (want && role == 3u) sh.recv[1][lane64 - LANE_P] = x;
-      if (rm || rp) wave_sync();
-    }
-    if (!ok) {
-      sh.fail = 1u;
-      if (lane64 == 0) atomicOr(err, 1u);
-    }
+    const bool want = !late && ((gets_sum && sums) || ((gets_m || gets_p) && rows));
+    const float x = mb_wait(buffer(), word, want, e, late);
+    if (late) sh.fail = 1u;
     return x;
   };
-  // the outer neighbours' elements: own slots, received rows, or the zero
-  // slot behind the own ones
+  // the outer neighbours' elements: own slots, the received rows (x of
+  // collect: row 2 of wave 0, row 3 of wave wl), or the zero slot behind the
+  // own ones
   const float *zero = sh.zb + KNOTS * 16 + i;
-  const float *far_m_src = far_m ? sh.recv[0] + i : zero, *far_p_src = far_p ? sh.recv[1] + i : zero;
-  const float *zm_src = own_m ? zb0 - 16 : far_m_src, *zp_src = own_p ? zb0 + RK * 16 : far_p_src;
-  auto neighbours = [&](float &vm, float &vp) {
-    vm = *zm_src;
-    vp = *zp_src;
+  const float *zm_src = own_m ? zb0 - 16 : zero, *zp_src = own_p ? zb0 + RK * 16 : zero;
+  const int far_lane = (int)((far_p ? LANE_P : LANE_M) + i) * 4;
+  auto neighbours = [&](const float *m_src, const float *p_src, float x, float &vm, float &vp) {
+    const float far = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(far_lane, __builtin_bit_cast(int, x)));
+    const float m = *m_src, q = *p_src;
+    vm = far_m ? far : m;
+    vp = far_p ? far : q;
   };
   // stair preconditioner: w = D^-1 r staged like z, in its own buffer, and
   // its row at the split exchanged on an epoch of its own (row only)
-  float *wb0 = sh.wb + b0 * 16 + i;
-  auto stage_w = [&](const float (&v)[RK]) {
-    wb0[0] = v[0];
-    wb0[(RK - 1) * 16] = v[RK - 1];
-    post_rows(v);
-  };
-  const float *wm_src = own_m ? wb0 - 16 : far_m_src, *wp_src = own_p ? wb0 + RK * 16 : far_p_src;
-  auto neighbours_w = [&](float &vm, float &vp) {
-    vm = *wm_src;
-    vp = *wp_src;
-  };
-  auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, sh.L + b0 * L_SLOT, i, x, xm, xp, y); };
-  // ((part 0 + part 1) + part 2) + part 3: the own part from LDS, the others
-  // from the partial lanes x of collect
+  constexpr int WB = (KNOTS + 1) * 16;
+  static_assert(offsetof(TeamShared, wb) == WB * sizeof(float), "wb is behind zb");
+  const float *wm_src = own_m ? zm_src + WB : zero, *wp_src = own_p ? zp_src + WB : zero;
+  auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, x, xm, xp, y); };
+  // ((part 0 + part 1) + part 2) + part 3: the own sum, the others from the
+  // sum lanes x of collect
   auto total = [&](float mine, float x) {
-    const float a = row_sum8<false>(x);
-    const float o0 = lane_of(a, 0);  // the first other part
-    if constexpr (Q == 2) return part == 0 ? mine + o0 : o0 + mine;
-    const float c = row_sum8<true>(x);
-    const float o1 = lane_of(a, 16), o2 = lane_of(c, 0);
-    const float v0 = part == 0 ? mine : o0, v1 = part == 1 ? mine : part < 1 ? o0 : o1,
-                v2 = part == 2 ? mine : part < 2 ? o1 : o2, v3 = part == 3 ? mine : o2;
-    return ((v0 + v1) + v2) + v3;
+    if constexpr (Q == 2) {
+      const float other = part == 0 ? lane_of(x, 1) : lane_of(x, 0);
+      return part == 0 ? mine + other : other + mine;
+    }
+    const float v = lane64 == part ? mine : x;
+    float s;
+    asm("s_nop 1\n"
+        "v_mov_b32_dpp %0, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_add_f32_dpp %0, %1, %0 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_add_f32_dpp %0, %1, %0 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_add_f32_dpp %0, %1, %0 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        : "=&v"(s)
+        : "v"(v));
+    return lane_of(s, 0);
   };
 
   // boundary lambda to the partner
   ++e;
-  stage(lam);
+  stage(p);
+  post_rows(p);
   __syncthreads();
-  collect(false, true);
   float pm, pp;
-  neighbours(pm, pp);
+  neighbours(zm_src, zp_src, collect(false, true), pm, pp);
 
-  // y = S p, its share of p.y posted; the next epoch begins here
-  auto product = [&](bool post) {
+  // y = S p, its share of p.y summed and posted; the next epoch begins here
+  float own;
+  bool failed;
+  auto product = [&](bool wanted) {
     smv(p, pm, pp);
     float pyp = 0.f;
 #pragma unroll
@@ -330,8 +288,10 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     pyp = wave_sum(pyp);
     ++e;
     sh.red[0][w] = pyp;  // the wave's lanes write the same value
-    if (post && lane64 == 0) mb_post(mb, set, part, e, w, pyp, tag_xor);
     __syncthreads();
+    own = sum8(sh.red[0]);
+    failed = uniform(sh.fail != 0u);
+    if (wanted && !failed) post_sum(own);
   };
 
   // The first pass is the prologue, through the same code: p = lambda,
@@ -343,32 +303,28 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   // run out, but sh.fail is the same for all of them there, so that all leave
   // together.  The product that the last pass takes ahead is not used (one
   // more in the number of iterations).
-#pragma unroll
-  for (int t = 0; t < RK; ++t) p[t] = lam[t];
   product(true);
   uint32_t it = ~0u;  // the first pass is not counted
   float eta = 0.f, tol_i = tol;
-  bool first = true, conv, failed, run;
+  bool first = true, conv, run;
   do {
-    const float own0 = sum8(sh.red[0]);
-    const float quo = eta / total(own0, collect(true, false)), alpha = first ? 1.f : quo;
+    const float quo = eta / total(own, collect(true, false)), alpha = first ? 1.f : quo;
     const float alpha_l = first ? 0.f : alpha;
     float rz = 0.f;
 #pragma unroll
-    for (int t = 0; t < RK; ++t) {
-      lam[t] += alpha_l * p[t];
-      r[t] -= alpha * y[t];
-    }
+    for (int t = 0; t < RK; ++t) lam[t * 16] += alpha_l * p[t];
+#pragma unroll
+    for (int t = 0; t < RK; ++t) r[t] -= alpha * y[t];
     if constexpr (STAIR) {
-      // z = D^-1 (2 r - S w), w = D^-1 r; the previous z row in recv was
-      // consumed before this iteration's first barrier
+      // z = D^-1 (2 r - S w), w = D^-1 r
       float wv[RK], wm, wp;
       group_precond<RK>(R, r, wv);
       ++e;
-      stage_w(wv);
+      zb0[WB] = wv[0];
+      zb0[WB + (RK - 1) * 16] = wv[RK - 1];
+      post_rows(wv);
       __syncthreads();
-      collect(false, true);
-      neighbours_w(wm, wp);
+      neighbours(wm_src, wp_src, collect(false, true), wm, wp);
       smv(wv, wm, wp);
 #pragma unroll
       for (int t = 0; t < RK; ++t) wv[t] = 2.f * r[t] - y[t];  // w is no longer needed
@@ -381,13 +337,14 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     rz = wave_sum(rz);
     ++e;
     sh.red[1][w] = rz;
-    if (lane64 == 0) mb_post(mb, set, part, e, w, rz, tag_xor);
+    post_rows(z);
     stage(z);
     __syncthreads();
     const float own1 = sum8(sh.red[1]);
+    if (uniform(sh.fail == 0u)) post_sum(own1);
     const float x = collect(true, true);
     float zm, zp;
-    neighbours(zm, zp);
+    neighbours(zm_src, zp_src, x, zm, zp);
     const float eta_new = total(own1, x);
     // taken in the last iteration too (p is not used after it)
     const float quo_b = eta_new / eta, beta = first ? 0.f : quo_b;
@@ -403,14 +360,16 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
     run = !conv && it < cap;
     product(run);
-    failed = uniform(sh.fail != 0u);
     run = run && !failed;
   } while (run);
-  if (failed) return fault();
+  if (failed) {
+    if (lane64 == 0) atomicOr(err, 1u);
+    return false;  // this part is not counted in `done`: the instance gets PCG_FLAG_FAULT
+  }
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
     const uint32_t lk = b0 + (uint32_t)t;
-    if (lk < n_own && lane_ok) lambda[(size_t)NX * (K0 + kb + lk) + i] = lam[t];
+    if (lk < n_own && lane_ok) lambda[(size_t)NX * (K0 + kb + lk) + i] = lam[t * 16];
   }
   if (tid == 0) {
     if (part == 0) {
@@ -537,7 +496,7 @@ __global__ void k_team_reset(TeamMailbox *mb, uint32_t n_mb, const uint32_t *__r
                              PoolCounters *ctr) {
   constexpr uint32_t W = sizeof(TeamMailbox) / sizeof(unsigned long long);
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_mb * W) (&mb[0].w[0][0][0])[i] = 0ull;
+  if (i < n_mb * W) (&mb[0].w[0][0])[i] = 0ull;
   if (i < n) {
     const uint32_t inst = team_inst[team0 + i];
     if (!status || (status[inst] & ST_ACTIVE)) done[inst] = 0u;

@@ -15,23 +15,19 @@
 // with each lane holding its row of M "rotated": Mr[n] = M(i, src(i, n)),
 // zero where src >= 14 or i >= 14.  One v_fmac_f32_dpp per term.
 //
-// Blocks of block row b: D = S(b,b) and P = Pinv(b,b) in registers;
-// L_b = S(b,b-1) in LDS, pre-rotated per lane (Lr[n] at lane offset
-// i * L_LANE + n, read as 8 x 64-bit words; L_LANE = 18 spreads the 14 lanes
-// over all 32 banks).  S(b,b+1) = L_{b+1}^T is applied from the rows of
-// L_{b+1} in "contribution" form: lane j forms L_{b+1}(j, i) x_j for the lane
-// i that reads it under row_ror:n, i.e.
+// Blocks of block row b, all in registers: D = S(b,b), P = Pinv(b,b) and
+// L_b = S(b,b-1), rotated; the group also holds the L of the knot after its
+// last.  S(b,b+1) = L_{b+1}^T is applied from the rows of L_{b+1} in
+// "contribution" form: lane j forms L_{b+1}(j, i) x_j for the lane i that
+// reads it under row_ror:n, i.e.
 //     (L^T x)_i = sum_n ror_n(Lr[(16 - n) mod 16] * x)_i,
-// so no transposed copy is stored.
+// so no transposed copy is held.  With four knots per group that is 208 of
+// the 256 registers that two waves per SIMD have.
 #pragma once
 #include "common.h"
 
 namespace mpc {
 namespace onchip {
-
-constexpr int L_LANE = 18;              // floats per lane row of a stored L block
-constexpr int L_SLOT = NX * L_LANE;     // 252 floats per knot slot (lanes 14, 15 read into the next slot)
-constexpr int L_GUARD = 2 * L_LANE;     // finite tail read by lanes 14, 15 past the last slot
 
 // direction of row_ror on this device: src(i, 1) - i (mod 16), 1 or 15.
 // Must run with every lane of the row active; tid = the lane's thread index.
@@ -95,49 +91,46 @@ __device__ __forceinline__ float wave_sum(float v) {
 // register (a branch on it leaves EXEC alone)
 __device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
 
-// Registers of one block row (knot k of the instance starting at global
-// knot K0) for lane i; zeros for absent rows and lanes >= 14.  Also writes
-// L_k = S(k,k-1) pre-rotated into the LDS slot Ls (lanes i < 14; zeros for
-// k = 0).  One branch for the row's 48 reads, none between them.
-struct RowRegs {
-  float D[16], P[16];
+// rotated rows of the column-major 14 x 14 block at base + off (floats);
+// zeros where ok is false and for columns and lanes past 13
+__device__ __forceinline__ void load_block(float (&R)[16], bool ok, uint32_t i, uint32_t d, const float *__restrict__ base,
+                                           uint32_t off) {
+#pragma unroll
+  for (int n = 0; n < 16; ++n) R[n] = 0.f;
+  if (ok) {
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      const uint32_t j = (i + (uint32_t)n * d) & 15u;
+      R[n] = base[off + i + (j < (uint32_t)NX ? NX * j : 0u)];
+    }
+#pragma unroll
+    for (int n = 0; n < 16; ++n) R[n] = ((i + (uint32_t)n * d) & 15u) < (uint32_t)NX ? R[n] : 0.f;
+  }
+}
+
+// Block rows of RK consecutive knots for lane i, and the L of the knot after
+// them; zeros for absent ones and lanes >= 14.
+template <int RK>
+struct Rows {
+  float D[RK][16], P[RK][16], L[RK + 1][16];
+
+  // S, Pinv: of the instance; k0 the first knot, n its knots in all, own the
+  // first knot past this workgroup's part
+  __device__ __forceinline__ void load(const float *__restrict__ S, const float *__restrict__ Pinv, uint32_t k0,
+                                       uint32_t own, uint32_t n, uint32_t i, uint32_t d) {
+    const bool lane_ok = i < (uint32_t)NX;
+#pragma unroll
+    for (int t = 0; t < RK; ++t) {
+      const uint32_t k = k0 + (uint32_t)t;
+      const bool has = lane_ok && k < own;
+      load_block(D[t], has, i, d, S, S_STRIDE * k + NXX);
+      load_block(P[t], has, i, d, Pinv, S_STRIDE * k + NXX);
+      load_block(L[t], has && k > 0, i, d, S, S_STRIDE * k);
+    }
+    const uint32_t k = k0 + RK;
+    load_block(L[RK], lane_ok && k0 < own && k < n, i, d, S, S_STRIDE * k);
+  }
 };
-
-__device__ __forceinline__ void load_row(RowRegs &R, float *Ls, bool has, uint32_t i, uint32_t d,
-                                         const float *__restrict__ S, const float *__restrict__ Pinv,
-                                         uint32_t K0, uint32_t k) {
-  const float *Sb = S + (size_t)S_STRIDE * (K0 + k);
-  const float *Pb = Pinv + (size_t)S_STRIDE * (K0 + k);
-#pragma unroll
-  for (int n = 0; n < 16; ++n) R.D[n] = R.P[n] = 0.f;
-  if (has && i < (uint32_t)NX) {
-    float l[16];
-#pragma unroll
-    for (int n = 0; n < 16; ++n) {
-      const uint32_t j = (i + (uint32_t)n * d) & 15u, at = i + (j < (uint32_t)NX ? NX * j : 0u);
-      R.D[n] = Sb[NXX + at];
-      R.P[n] = Pb[NXX + at];
-      l[n] = Sb[at];
-    }
-#pragma unroll
-    for (int n = 0; n < 16; ++n) {
-      const bool col = ((i + (uint32_t)n * d) & 15u) < (uint32_t)NX;
-      R.D[n] = col ? R.D[n] : 0.f;
-      R.P[n] = col ? R.P[n] : 0.f;
-      Ls[i * L_LANE + n] = col && k > 0 ? l[n] : 0.f;
-    }
-  }
-}
-
-__device__ __forceinline__ void read_lrow(float (&Lr)[16], const float *Ls, uint32_t i) {
-  const float2 *l2 = reinterpret_cast<const float2 *>(Ls + i * L_LANE);
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const float2 v = l2[c];
-    Lr[2 * c] = v.x;
-    Lr[2 * c + 1] = v.y;
-  }
-}
 
 // (D x + L xl) + M^T xr of one knot, M the rows of the next knot's left
 // block: two direct chains, and the contributions of M's rows (header) in an
@@ -201,30 +194,21 @@ __device__ __forceinline__ float row_precond(const float (&P)[16], float r) {
   return z;
 }
 
-// y = S x for the RK consecutive knots of a group: Ls0 is the LDS slot of
-// its first knot (slot t + 1 holds L of the next knot, finite and multiplied
-// by xp = 0 after the last knot); xm / xp are the elements of the knots just
-// before / after the group.  Each slot's rows are read once.
+// y = S x for the RK knots of a group; xm / xp the elements of the knots
+// before and after them
 template <int RK>
-__device__ __forceinline__ void group_smv(const RowRegs (&R)[RK], const float *Ls0, uint32_t i, const float (&x)[RK],
-                                          float xm, float xp, float (&y)[RK]) {
-  // three buffers: the rows of slot t + 2 are read while knot t's products,
-  // which take those of slots t and t + 1, run
-  float L[3][16];
-  read_lrow(L[0], Ls0, i);
-  read_lrow(L[1], Ls0 + L_SLOT, i);
+__device__ __forceinline__ void group_smv(const Rows<RK> &R, const float (&x)[RK], float xm, float xp,
+                                          float (&y)[RK]) {
 #pragma unroll
-  for (int t = 0; t < RK; ++t) {
-    if (t + 2 <= RK) read_lrow(L[(t + 2) % 3], Ls0 + (t + 2) * L_SLOT, i);
-    y[t] = row_product(R[t].D, x[t], L[t % 3], t > 0 ? x[t - 1] : xm, L[(t + 1) % 3], t < RK - 1 ? x[t + 1] : xp);
-  }
+  for (int t = 0; t < RK; ++t)
+    y[t] = row_product(R.D[t], x[t], R.L[t], t > 0 ? x[t - 1] : xm, R.L[t + 1], t < RK - 1 ? x[t + 1] : xp);
 }
 
 // z = Pinv r for the RK knots of a group
 template <int RK>
-__device__ __forceinline__ void group_precond(const RowRegs (&R)[RK], const float (&r)[RK], float (&z)[RK]) {
+__device__ __forceinline__ void group_precond(const Rows<RK> &R, const float (&r)[RK], float (&z)[RK]) {
 #pragma unroll
-  for (int t = 0; t < RK; ++t) z[t] = row_precond(R[t].P, r[t]);
+  for (int t = 0; t < RK; ++t) z[t] = row_precond(R.P[t], r[t]);
 }
 
 }  // namespace onchip

@@ -20,7 +20,7 @@
 // block product, one more staged vector and one more barrier per iteration.
 //
 // Per iteration, two workgroup barriers (block Jacobi):
-//   y = S p (registers + L from LDS); p.y -> B1 -> alpha; lambda, r;
+//   y = S p; p.y -> B1 -> alpha; lambda, r;
 //   z = Pinv r; stage z of the group's first and last knot; r.z -> B2 ->
 //   beta; p = z + beta p for the own knots and, from the staged z, for the
 //   copies of the neighbouring groups' elements p_{4lg-1}[i], p_{4lg+4}[i]
@@ -30,8 +30,9 @@
 // multiply-add takes 4.5 clocks, a plain one 2.25), so the iteration is bound
 // by issue; branches on values that differ between lanes cost it several
 // hundred clocks in EXEC bookkeeping, so conditions are ballots and the loop
-// has one back branch.  Batch of 300 in stair mode 5.33 -> 3.98 ms, one stair
-// solve of N = 100 1.37 -> 1.24 ms.
+// has one back branch.  Batch of 300 in stair mode 5.34 -> 3.98 ms, 3.73 with
+// S(b,b-1) in registers too (it was read from LDS twice per product); one
+// stair solve of N = 100 1.46 -> 1.15 ms.
 #pragma once
 #include "pcg_onchip.h"
 
@@ -44,7 +45,7 @@ constexpr int RK = 4;    // knots per group
 constexpr int MAXI = 8;  // instances per bin
 
 // Workgroup shapes: NT = 512 lanes (32 groups, 8 waves, 128 knots; one per
-// CU) or 256 (16 groups, 4 waves, 64 knots; two per CU share its LDS).
+// CU) or 256 (16 groups, 4 waves, 64 knots; two per CU).
 template <int NT>
 struct ResShape {
   static_assert(NT == 256 || NT == 512, "workgroup of 4 or 8 waves");
@@ -54,15 +55,13 @@ struct ResShape {
 template <int NT>
 struct ResShared {
   static constexpr int KNOTS = ResShape<NT>::KNOTS, NWAV = ResShape<NT>::NWAV;
-  float L[(KNOTS + 1) * L_SLOT + L_GUARD];  // S(b,b-1) per knot slot (+ one zero slot), pre-rotated rows
-  float zb[(KNOTS + 1) * 16];         // staged vector element per knot slot and lane
-  float wb[(KNOTS + 1) * 16];         // stair preconditioner: staged D^-1 r
+  float zb[(KNOTS + 1) * 16];  // staged vector element per knot slot and lane (+ one zero slot)
+  float wb[(KNOTS + 1) * 16];  // stair preconditioner: staged D^-1 r
   // dot-product partials of the waves, by instance of the bin and wave of the
   // instance (zero past its waves)
   alignas(16) float red[2][MAXI][NWAV];
   uint32_t act[MAXI];  // by instance of the bin: 1 while it iterates
   static_assert(NWAV % 4 == 0, "partials are read as 16-byte words");
-  static_assert(((KNOTS + 1) * L_SLOT + L_GUARD) % 4 == 0, "L and zb are cleared as one float4 range");
 };
 
 // the partials in wave order
@@ -93,11 +92,7 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
   ResShared<NT> &sh = *reinterpret_cast<ResShared<NT> *>(smem);
   const uint32_t g = tid >> 4, i = tid & 15u, w = tid >> 6;
   const uint32_t d = ror_step(tid);
-  {
-    float4 *z4 = reinterpret_cast<float4 *>(sh.L);
-    constexpr uint32_t n4 = ((KNOTS + 1) * L_SLOT + L_GUARD + (KNOTS + 1) * 16) / 4;
-    for (uint32_t idx = tid; idx < n4; idx += NT) z4[idx] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+  for (uint32_t idx = tid; idx < (KNOTS + 1) * 16; idx += NT) sh.zb[idx] = 0.f;
 
   // my instance in this bin (items: {inst, first group, groups, -}); a null
   // item table means one instance (0) starting at group 0
@@ -130,17 +125,17 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
   if (tid < 2u * MAXI * NWAV) (&sh.red[0][0][0])[tid] = 0.f;
   __syncthreads();  // LDS cleared
 
-  // ---- load: D, Pinv rows into registers, S(b,b-1) into LDS
+  // ---- load: the block rows
   const uint32_t b0 = lg * RK, s0 = lbase + b0;  // first knot of the group and its slot
-  RowRegs R[RK];
+  Rows<RK> R;
+  R.load(S + (size_t)S_STRIDE * K0, Pinv + (size_t)S_STRIDE * K0, b0, live ? N : 0u, N, i, d);
   float lam[RK], r[RK], p[RK], y[RK], z[RK];
 #pragma unroll
   for (int t = 0; t < RK; ++t) {
     const uint32_t bk = b0 + (uint32_t)t;
-    const bool has = live && bk < N;
-    load_row(R[t], sh.L + (s0 + t) * L_SLOT, has, i, d, S, Pinv, K0, bk);
-    lam[t] = has && lane_ok ? lambda[(size_t)NX * (K0 + bk) + i] : 0.f;
-    r[t] = has && lane_ok ? gamma[(size_t)NX * (K0 + bk) + i] : 0.f;
+    const bool has = live && bk < N && lane_ok;
+    lam[t] = has ? lambda[(size_t)NX * (K0 + bk) + i] : 0.f;
+    r[t] = has ? gamma[(size_t)NX * (K0 + bk) + i] : 0.f;
   }
   // first / last element of the group to LDS; neighbouring groups' copies back
   const bool in_m = lg > 0, in_p = b0 + RK < N;
@@ -167,7 +162,7 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
     vp = *wp_src;
   };
   // y = S x for the group's knots; xm / xp: elements of knots 4lg-1, 4lg+4
-  auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, sh.L + s0 * L_SLOT, i, x, xm, xp, y); };
+  auto smv = [&](const float (&x)[RK], float xm, float xp) { group_smv<RK>(R, x, xm, xp, y); };
   // an instance's act word: set here, cleared when it stops (its lanes all
   // write the same, between the second barrier of its last iteration and the
   // first of the next)

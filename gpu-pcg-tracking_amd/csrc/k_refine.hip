@@ -100,6 +100,28 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// f(v, i) over v[i], i = threadIdx.x, threadIdx.x + NT_NORM, ... < n, eight
+// elements at a time with their reads in flight together (past the end the
+// last element again, f not called); one at a time they were a trip to memory
+// each (k_rhs_normalise at N = 512 27 -> 10 us)
+template <typename F>
+__device__ __forceinline__ void for_each8(const float *v, uint32_t n, F f) {
+  constexpr int U = 8;
+  for (uint32_t i0 = threadIdx.x; i0 < n; i0 += NT_NORM * U) {
+    float x[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const uint32_t i = i0 + (uint32_t)(k * NT_NORM);
+      x[k] = v[i < n ? i : n - 1u];
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const uint32_t i = i0 + (uint32_t)(k * NT_NORM);
+      if (i < n) f(x[k], i);
+    }
+  }
+}
+
 // per instance: s = max |[rz; rc]| (1 if zero), then rz /= s, rc /= s
 __global__ void __launch_bounds__(NT_NORM) k_rhs_normalise(Batch b, float *__restrict__ rz, float *__restrict__ rc,
                                                            float *__restrict__ scale) {
@@ -109,8 +131,9 @@ __global__ void __launch_bounds__(NT_NORM) k_rhs_normalise(Batch b, float *__res
   float *z = rz + (size_t)NXU * K0, *c = rc + (size_t)NX * K0;
   const uint32_t nz = NXU * N, nc = NX * N;
   float m = 0.f;
-  for (uint32_t i = threadIdx.x; i < nz; i += NT_NORM) m = fmaxf(m, fabsf(z[i]));
-  for (uint32_t i = threadIdx.x; i < nc; i += NT_NORM) m = fmaxf(m, fabsf(c[i]));
+  auto largest = [&](float v, uint32_t) { m = fmaxf(m, fabsf(v)); };
+  for_each8(z, nz, largest);
+  for_each8(c, nc, largest);
   m = wave_max(m);
   if ((threadIdx.x & 63u) == 0) part[threadIdx.x / 64] = m;
   __syncthreads();
@@ -119,8 +142,8 @@ __global__ void __launch_bounds__(NT_NORM) k_rhs_normalise(Batch b, float *__res
   for (int w = 1; w < NT_NORM / 64; ++w) s = fmaxf(s, part[w]);
   if (!(s > 0.f)) s = 1.f;
   const float inv = 1.f / s;
-  for (uint32_t i = threadIdx.x; i < nz; i += NT_NORM) z[i] *= inv;
-  for (uint32_t i = threadIdx.x; i < nc; i += NT_NORM) c[i] *= inv;
+  for_each8(z, nz, [&](float v, uint32_t i) { z[i] = v * inv; });
+  for_each8(c, nc, [&](float v, uint32_t i) { c[i] = v * inv; });
   if (threadIdx.x == 0) scale[inst] = s;
 }
 

@@ -1,7 +1,7 @@
 // gj16.h -- 14x14 block algebra inside a 16-lane group (gfx950): lane j
 // holds column j of a block in registers; a pivot column is broadcast to
-// the group by ds_swizzle (Gauss-Jordan) or a DPP row broadcast (the
-// whitening factor), so neither needs an LDS buffer or a barrier.  Used by
+// the group by DPP, in the multiply-adds themselves (Gauss-Jordan) or ahead of
+// them (the whitening factor), so neither needs an LDS buffer or a barrier.  Used by
 // the Schur formation (k_schur.hip), the split PCG (k_pcg_split.hip) and
 // the direct block-tridiagonal solve (k_direct.hip).
 #pragma once
@@ -9,34 +9,25 @@
 
 namespace mpc {
 
-// value of lane P of the calling lane's 16-lane group (ds_swizzle bitmask
-// mode: lane' = (lane & 0x10) | P within each 32-lane half)
-template <int P>
-__device__ __forceinline__ float bcast16(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x10 | (P << 5)));
-}
-
-// The same broadcast by DPP row_newbcast:P (dpp_ctrl 0x150 + P, gfx90a and
-// later): lane P of each 16-lane row to the whole row, one VALU instruction
-// with no trip through the LDS pipeline.  Lane P must be active.  Used on
-// the dependent pivot chain of chol_inv_rows, where the swizzle's LDS
-// latency sits on the critical path of every step.
+// Value of lane P of the calling lane's 16-lane group by DPP row_newbcast:P
+// (dpp_ctrl 0x150 + P, gfx90a and later): lane P of each 16-lane row to the
+// whole row, one VALU instruction with no trip through the LDS pipeline.
+// Lane P must be active.
 template <int P>
 __device__ __forceinline__ float bcast16_dpp(float v) {
   static_assert(P >= 0 && P < 16, "row lane");
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + P, 0xf, 0xf, true));
 }
 
-// bcast16 (Dpp: bcast16_dpp) with the lane p given as a value that is a
-// constant after loop unrolling (both take the lane as an immediate)
-template <bool Dpp = false>
+// bcast16_dpp with the lane p given as a value that is a constant after loop
+// unrolling (the instruction takes the lane as an immediate)
 __device__ __forceinline__ float bcast_dyn16(float v, int p) {
 #define MPC_BCASE(P) \
-  case P: return Dpp ? bcast16_dpp<P>(v) : bcast16<P>(v);
+  case P: return bcast16_dpp<P>(v);
   switch (p) {
     MPC_BCASE(0) MPC_BCASE(1) MPC_BCASE(2) MPC_BCASE(3) MPC_BCASE(4) MPC_BCASE(5) MPC_BCASE(6) MPC_BCASE(7)
     MPC_BCASE(8) MPC_BCASE(9) MPC_BCASE(10) MPC_BCASE(11) MPC_BCASE(12) MPC_BCASE(13) MPC_BCASE(14)
-    default: return Dpp ? bcast16_dpp<15>(v) : bcast16<15>(v);
+    default: return bcast16_dpp<15>(v);
   }
 #undef MPC_BCASE
 }
@@ -50,25 +41,39 @@ __device__ __forceinline__ void pin(float (&v)[n]) {
   for (int r = 0; r < n; ++r) asm volatile("" : "+v"(v[r]));
 }
 
+// x -= c xp and a -= c ap for six rows (or one) of a pivot step, c the row's
+// element of the pivot column: lane p's a, by DPP.  (The s_nop: a DPP read
+// needs two wait states after the write of what it reads.)
+#define MPC_GJ_ROW(k)                                                                                        \
+  "v_fmac_f32_dpp %[x" #k "], %[a" #k "], -%[xp] row_newbcast:%c[p] row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+  "v_fmac_f32_dpp %[a" #k "], %[a" #k "], -%[ap] row_newbcast:%c[p] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define MPC_GJ_OPS(k) [x##k] "+v"(x[(r0 + k) % n]), [a##k] "+v"(a[(r0 + k) % n])
+template <int n, int p, int r0>
+__device__ __forceinline__ void gj_rows6(float (&x)[NX], float (&a)[NX], float xp, float ap) {
+  asm("s_nop 1\n" MPC_GJ_ROW(0) MPC_GJ_ROW(1) MPC_GJ_ROW(2) MPC_GJ_ROW(3) MPC_GJ_ROW(4) MPC_GJ_ROW(5)
+      : MPC_GJ_OPS(0), MPC_GJ_OPS(1), MPC_GJ_OPS(2), MPC_GJ_OPS(3), MPC_GJ_OPS(4), MPC_GJ_OPS(5)
+      : [xp] "v"(xp), [ap] "v"(ap), [p] "i"(p));
+}
+template <int n, int p, int r0>
+__device__ __forceinline__ void gj_rows1(float (&x)[NX], float (&a)[NX], float xp, float ap) {
+  asm("s_nop 1\n" MPC_GJ_ROW(0) : MPC_GJ_OPS(0) : [xp] "v"(xp), [ap] "v"(ap), [p] "i"(p));
+}
+#undef MPC_GJ_OPS
+#undef MPC_GJ_ROW
+
 template <int n, int p>
 __device__ __forceinline__ void gj_step(float (&a)[NX], float (&x)[NX]) {
-  float pc[n];
-#pragma unroll
-  for (int r = 0; r < n; ++r) pc[r] = bcast16<p>(a[r]);
-  const float inv = 1.f / pc[p];
+  static_assert(n == NX || n == NU, "6 + 6 + 1 or 6 rows beside the pivot's");
+  const float inv = 1.f / bcast_dyn16(a[p], p);
   const float ap = a[p] * inv, xp = x[p] * inv;
-#pragma unroll
-  for (int r = 0; r < n; ++r) {
-    if (r == p) continue;
-    a[r] -= pc[r] * ap;
-    x[r] -= pc[r] * xp;
+  // from the next pivot's row on, so that its division can start
+  gj_rows6<n, p, p + 1>(x, a, xp, ap);
+  if constexpr (n == NX) {
+    gj_rows6<n, p, p + 7>(x, a, xp, ap);
+    gj_rows1<n, p, p + 13>(x, a, xp, ap);
   }
   a[p] = ap;
   x[p] = xp;
-  // the x updates would otherwise sink to their use after the last step and
-  // keep every step's pivot column alive
-  pin(a);
-  pin(x);
 }
 
 template <int n, int p = 0>
@@ -111,7 +116,7 @@ __device__ __forceinline__ void chol_inv_rows(int lane, float (&a)[NX], float (&
   for (int p = 0; p < n; ++p) {
     float pc[NX];
 #pragma unroll
-    for (int r = p; r < n; ++r) pc[r] = bcast_dyn16<true>(a[r], p);
+    for (int r = p; r < n; ++r) pc[r] = bcast_dyn16(a[r], p);
     const float inv = __builtin_amdgcn_rcpf(pc[p]);
     const float s = __builtin_amdgcn_rsqf(pc[p]);
     const float ap = a[p], xp = x[p];

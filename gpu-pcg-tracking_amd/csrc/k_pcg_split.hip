@@ -381,13 +381,13 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
       float num = 0.f;
 #pragma unroll
       for (int t = 0; t < RK; ++t) {
-        const float v = bcast_dyn16<true>(lam[t], k);
+        const float v = bcast_dyn16(lam[t], k);
         num = td == (uint32_t)t ? v : num;
       }
       const float quo = num / den[k];
 #pragma unroll
       for (int t = 0; t < RK; ++t) {
-        const float xk = bcast_dyn16<true>(quo, t);
+        const float xk = bcast_dyn16(quo, t);
         lh[t] = (int)i == k ? xk : lh[t];
         lam[t] -= wr[t][k] * xk;
       }

@@ -7,9 +7,13 @@
 //   k_form_schur: per block row, the products, theta, its inverse and the
 //                 outputs, reading Q~^-1 / R~^-1 from G^-1.
 // Block inverses are Gauss-Jordan eliminations on [M | I]; the pivot column
-// is broadcast within the group by ds_swizzle (no LDS round trip, no
-// barrier).  The regularised blocks are symmetric positive definite, so no
-// pivoting is needed.
+// is broadcast within the group by DPP, and so are the left factors of the
+// block products, inside the multiply-adds.  The regularised blocks are
+// symmetric positive definite, so no pivoting is needed.
+// k_form_schur moves 5.3 KB a knot, 1.22 M knots in 1.58 ms (4.1 TB/s; a copy
+// reaches 5.1): bound by memory.  With the factors read from LDS by every
+// lane, swizzled pivot columns and the reads of a row behind its instance
+// lookup it took 2.77 ms; 128 knots 14.6 us, 8.2 now.
 //
 // Math (reference: oldschur.cuh:518-963, signs as there; C stores -A, -B):
 //   Q~_k = Q_k + rho I, R~_k = R_k + rho I
@@ -74,15 +78,61 @@ __global__ void __launch_bounds__(WG) k_invert_g(Batch b, const float *__restric
   }
 }
 
+// d[r] += s_l[r] * w (r < 14), s_l the s of lane l of the 16-lane group:
+// v_fmac_f32_dpp with DPP row_newbcast:l, so a block product whose left
+// factor is held by columns (lane l: column l) needs no LDS and no
+// separate broadcast instruction.  The s_nop ahead of each seven covers the
+// wait states between a VALU write of an operand (or of EXEC, Nop4) and its
+// DPP read.  The group's lanes must all be active.
+#define MPC_NBF(k) "v_fmac_f32_dpp %" #k ", %" MPC_NBS##k ", %14 row_newbcast:%15 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define MPC_NBS0 "7"
+#define MPC_NBS1 "8"
+#define MPC_NBS2 "9"
+#define MPC_NBS3 "10"
+#define MPC_NBS4 "11"
+#define MPC_NBS5 "12"
+#define MPC_NBS6 "13"
+#define MPC_NB7(nop)                                                                                          \
+  asm(nop MPC_NBF(0) MPC_NBF(1) MPC_NBF(2) MPC_NBF(3) MPC_NBF(4) MPC_NBF(5) MPC_NBF(6)                          \
+      : "+v"(d[o]), "+v"(d[o + 1]), "+v"(d[o + 2]), "+v"(d[o + 3]), "+v"(d[o + 4]), "+v"(d[o + 5]), "+v"(d[o + 6]) \
+      : "v"(s[o]), "v"(s[o + 1]), "v"(s[o + 2]), "v"(s[o + 3]), "v"(s[o + 4]), "v"(s[o + 5]), "v"(s[o + 6]),       \
+        "v"(w), "i"(l))
+template <int l, bool Nop4, int o>
+__device__ __forceinline__ void nb_fma7(float (&d)[NX], const float (&s)[NX], float w) {
+  static_assert(l >= 0 && l < 16 && o + 7 <= NX, "row lane, accumulator range");
+  if constexpr (Nop4)
+    MPC_NB7("s_nop 4\n");
+  else
+    MPC_NB7("s_nop 1\n");
+}
+#undef MPC_NB7
+#undef MPC_NBF
+#undef MPC_NBS0
+#undef MPC_NBS1
+#undef MPC_NBS2
+#undef MPC_NBS3
+#undef MPC_NBS4
+#undef MPC_NBS5
+#undef MPC_NBS6
+
+// d[r] += sum_{l in Ls, in order} s_l[r] * w[l]: a block product from the
+// left factor's columns (one per lane) and the calling lane's row of the
+// right factor's transpose
+template <bool Nop4, int... Ls>
+__device__ __forceinline__ void nb_product(float (&d)[NX], const float (&s)[NX], const float *w,
+                                           std::integer_sequence<int, Ls...>) {
+  ((nb_fma7<Ls, Nop4 && Ls == 0, 0>(d, s, w[Ls]), nb_fma7<Ls, false, 7>(d, s, w[Ls])), ...);
+}
+
 // 16-byte aligned blocks: AQ and A (reused for the S(b,b) and Pinv(b,b)
 // blocks on their way out) are read as float4 rows for coalesced stores
 struct alignas(16) SchurLds {
-  float AQ[NXX];  // A Q~_k^-1
+  float AQ[NXX];  // Q~_k^-1, then Q~_b^-1, then (not for a first knot) A Q~_k^-1
   float A[NXX];   // A_k (column-major)
-  float B[98];    // B_k
-  float BR[98];   // B R~_k^-1
+  float B[98];    // B_k, then B R~_k^-1
+  float R[49];    // R~_k^-1
   float qk[16], q1[16], rk[8], cb[16];
-};
+};  // 2384 B: sixteen workgroups' fit one CU's LDS
 static_assert(NXX % 4 == 0 && sizeof(float) * NXX % 16 == 0, "float4 rows of a 14 x 14 block");
 
 // a 14 x 14 block (element i at src[f(i)]) from the group's LDS to global
@@ -98,7 +148,7 @@ __device__ __forceinline__ void store_block(int lane, float *dst, F &&f) {
   }
 }
 
-__global__ void __launch_bounds__(WG) k_form_schur(Batch b, const float *__restrict__ G,
+__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) k_form_schur(Batch b, const float *__restrict__ G,
                                                    const float *__restrict__ C,
                                                    const float *__restrict__ g,
                                                    const float *__restrict__ cvec,
@@ -113,107 +163,107 @@ __global__ void __launch_bounds__(WG) k_form_schur(Batch b, const float *__restr
   const uint32_t gk_raw = blockIdx.x * GROUPS_PER_WG + grp;
   bool valid = gk_raw < b.total_knots;
   const uint32_t gk = valid ? gk_raw : b.total_knots - 1;
+  SchurLds &L = lds[grp];
+  // The block row's reads are issued before the instance lookup, all of them
+  // together: the previous knot's (for an instance's first knot another's
+  // last; what is formed from them is not stored there) and this knot's.
+  const size_t row = gk, kprev = gk > 0 ? gk - 1 : 0;  // block row b >= 1: k = b - 1
+  const float *Ck = C + (size_t)C_STRIDE * kprev;
+  const float *Qi = Ginv + (size_t)G_STRIDE * kprev;  // Q~_k^-1, then R~_k^-1
+  const float *Q1i = Ginv + (size_t)G_STRIDE * row;   // Q~_b^-1
+  const int j = lane < NX ? lane : NX - 1, ju = lane < NU ? lane : NU - 1;
+  float acol[NX], arow[NX], bcol[NX], brow[NU], qi[NX], ri[NU], th[NX];
+  float a1 = 0.f;  // (Q~_b^-1 q_b)_j
+  {
+    constexpr int NA = (NXX + GROUP - 1) / GROUP, NB = (98 + GROUP - 1) / GROUP, NR = (49 + GROUP - 1) / GROUP;
+    float va[NA], vb[NB], vq[NA], vr[NR], v1[NA];
+    // element lane + 16 k of a block of n, past its end the last one
+    auto at = [&](int k, int n) { return lane + GROUP * k < n ? lane + GROUP * k : n - 1; };
+#pragma unroll
+    for (int k = 0; k < NA; ++k) va[k] = Ck[at(k, NXX)];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) vb[k] = Ck[NXX + at(k, 98)];
+#pragma unroll
+    for (int k = 0; k < NA; ++k) vq[k] = Qi[at(k, NXX)];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) vr[k] = Qi[NXX + at(k, 49)];
+#pragma unroll
+    for (int k = 0; k < NA; ++k) v1[k] = Q1i[at(k, NXX)];
+    const float vk = g[(size_t)NXU * kprev + j], vu = g[(size_t)NXU * kprev + NX + ju],
+                vg = g[(size_t)NXU * row + j], vc = cvec ? cvec[(size_t)NX * row + j] : 0.f;  // no c: c = 0
+    // (past the end the last element again, to its place)
+#pragma unroll
+    for (int k = 0; k < NA; ++k) L.A[at(k, NXX)] = -va[k];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) L.B[at(k, 98)] = -vb[k];
+#pragma unroll
+    for (int k = 0; k < NA; ++k) L.AQ[at(k, NXX)] = vq[k];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) L.R[at(k, 49)] = vr[k];
+    L.qk[j] = vk;
+    L.rk[ju] = vu;
+    L.q1[j] = vg;
+    L.cb[j] = vc;
+    wave_sync();  // (a workgroup is one wave)
+    // columns j of A, Q~_k^-1, Q~_b^-1 and (j < 7) of B, R~_k^-1; rows j of A, B
+#pragma unroll
+    for (int l = 0; l < NX; ++l) {
+      acol[l] = L.A[l + NX * j];
+      arow[l] = L.A[j + NX * l];
+      bcol[l] = L.B[l + NX * ju];
+      qi[l] = L.AQ[l + NX * j];
+    }
+#pragma unroll
+    for (int l = 0; l < NU; ++l) {
+      brow[l] = L.B[j + NX * l];
+      ri[l] = L.R[l + NU * ju];
+    }
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < NA; ++k) L.AQ[at(k, NXX)] = v1[k];
+    wave_sync();
+#pragma unroll
+    for (int l = 0; l < NX; ++l) {
+      th[l] = L.AQ[l + NX * j];
+      a1 += L.AQ[j + NX * l] * L.q1[l];
+    }
+    wave_sync();
+  }
   const KnotRef kr = locate(b, gk);
   if (status && !(status[kr.inst] & ST_ACTIVE)) valid = false;
   const float rho = rho_dev ? rho_dev[kr.inst] : rho_s;
-  SchurLds &L = lds[grp];
   const uint32_t bk = kr.k;
-  const size_t row = (size_t)kr.K0 + bk;  // global block row
   float *Srow = S + (size_t)S_STRIDE * row;
   float *Prow = Pinv + (size_t)S_STRIDE * row;
-  // Every group runs the same sequence; block row 0 stages its own knot in
-  // the 'previous knot' slots and only keeps Q~_0^-1.
   const bool row0 = bk == 0;
-  const size_t kprev = row0 ? row : row - 1;  // block row b >= 1: k = b - 1
-  const float *Ck = C + (size_t)C_STRIDE * kprev;
-  const float *Qi = Ginv + (size_t)G_STRIDE * kprev;  // Q~_k^-1
-  const float *Ri = Qi + NXX;                         // R~_k^-1
-  const float *Q1i = Ginv + (size_t)G_STRIDE * row;   // Q~_b^-1
-  for (int i = lane; i < NXX; i += GROUP) L.A[i] = -Ck[i];
-  for (int i = lane; i < 98; i += GROUP) L.B[i] = -Ck[NXX + i];
-  if (lane < NX) {
-    L.qk[lane] = g[(size_t)NXU * kprev + lane];
-    L.q1[lane] = g[(size_t)NXU * row + lane];
-    L.cb[lane] = (row0 || !cvec) ? 0.f : cvec[(size_t)NX * row + lane];  // no c: c = 0
+  // AQ = A Q~_k^-1 (column j), BR = B R~_k^-1 (column j < 7): the left
+  // factor's columns from their lanes by DPP
+  float acc[NX], bacc[NX];
+#pragma unroll
+  for (int r = 0; r < NX; ++r) acc[r] = bacc[r] = 0.f;
+  nb_product<true>(acc, acol, qi, std::make_integer_sequence<int, NX>{});
+  nb_product<true>(bacc, bcol, ri, std::make_integer_sequence<int, NU>{});
+  if (!row0) {  // the same for the whole group
+#pragma unroll
+    for (int r = 0; r < NX; ++r) L.AQ[r + NX * j] = acc[r];
   }
-  if (lane < NU) L.rk[lane] = g[(size_t)NXU * kprev + NX + lane];
-  __syncthreads();
-
-  // AQ = A Q~_k^-1 (column j), BR = B R~_k^-1 (column j < 7)
-  const int j = lane < NX ? lane : NX - 1;
-  {
-    float qi[NX];
 #pragma unroll
-    for (int l = 0; l < NX; ++l) qi[l] = Qi[l + NX * j];
-    float acc[NX];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) acc[r] = 0.f;
-#pragma unroll
-    for (int l = 0; l < NX; ++l)
-#pragma unroll
-      for (int r = 0; r < NX; ++r) acc[r] += L.A[r + NX * l] * qi[l];
-    pin(acc);
-    if (lane < NX) {
-#pragma unroll
-      for (int r = 0; r < NX; ++r) L.AQ[r + NX * lane] = acc[r];
-    }
-  }
-  {
-    const int ju = lane < NU ? lane : NU - 1;
-    float ri[NU];
-#pragma unroll
-    for (int l = 0; l < NU; ++l) ri[l] = row0 ? 0.f : Ri[l + NU * ju];
-    float bacc[NX];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) bacc[r] = 0.f;
-#pragma unroll
-    for (int l = 0; l < NU; ++l)
-#pragma unroll
-      for (int r = 0; r < NX; ++r) bacc[r] += L.B[r + NX * l] * ri[l];
-    pin(bacc);
-    if (lane < NU) {
-#pragma unroll
-      for (int r = 0; r < NX; ++r) L.BR[r + NX * lane] = bacc[r];
-    }
-  }
-  __syncthreads();
+  for (int r = 0; r < NX; ++r) L.B[r + NX * ju] = bacc[r];
   // theta(:, j) = sum_l AQ(:, l) A(j, l) + sum_l BR(:, l) B(j, l) + Q~_b^-1(:, j)
-  float th[NX];
-#pragma unroll
-  for (int r = 0; r < NX; ++r) th[r] = Q1i[r + NX * j];
-#pragma unroll
-  for (int l = 0; l < NX; ++l) {
-    const float ajl = L.A[j + NX * l];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) th[r] += L.AQ[r + NX * l] * ajl;
-  }
-#pragma unroll
-  for (int l = 0; l < NU; ++l) {
-    const float bjl = L.B[j + NX * l];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) th[r] += L.BR[r + NX * l] * bjl;
-  }
-  pin(th);
-  __syncthreads();  // every lane is done reading A
+  nb_product<true>(th, acc, arow, std::make_integer_sequence<int, NX>{});
+  nb_product<true>(th, bacc, brow, std::make_integer_sequence<int, NU>{});
   // S(b,b) = -theta, transposed into rows through A for coalesced stores
-  if (lane < NX) {
 #pragma unroll
-    for (int r = 0; r < NX; ++r) L.A[r + NX * lane] = -th[r];
-  }
-  __syncthreads();
+  for (int r = 0; r < NX; ++r) L.A[r + NX * j] = -th[r];
+  wave_sync();
   if (valid && row0) {
     // S(0,0) = -Q~_0^-1, gamma_0 = -Q~_0^-1 q_0, Pinv(0,0) = -Q~_0
     const float *Q0 = G + (size_t)G_STRIDE * row;
     for (int i = lane; i < NXX; i += GROUP) {
-      Srow[NXX + i] = -Qi[i];
+      Srow[NXX + i] = -L.AQ[i];
       Prow[NXX + i] = -(Q0[i] + ((i % NX == i / NX) ? rho : 0.f));
     }
-    if (lane < NX) {
-      float acc = 0.f;
-#pragma unroll
-      for (int l = 0; l < NX; ++l) acc += Qi[lane + NX * l] * L.qk[l];
-      gamma[(size_t)NX * row + lane] = -acc;
-    }
+    if (lane < NX) gamma[(size_t)NX * row + lane] = -a1;
     if (zero_unused)
       for (int i = lane; i < NXX; i += GROUP) {
         Srow[i] = 0.f;
@@ -229,14 +279,11 @@ __global__ void __launch_bounds__(WG) k_form_schur(Batch b, const float *__restr
     if (right)
       store_block(lane, S + (size_t)S_STRIDE * kprev + 2 * NXX, [&](int i) { return L.AQ[i / NX + NX * (i % NX)]; });
     if (lane < NX) {
-      float a1 = 0.f, a2 = 0.f, a3 = 0.f;
+      float a2 = 0.f, a3 = 0.f;
 #pragma unroll
-      for (int l = 0; l < NX; ++l) {
-        a1 += Q1i[lane + NX * l] * L.q1[l];
-        a2 += L.AQ[lane + NX * l] * L.qk[l];
-      }
+      for (int l = 0; l < NX; ++l) a2 += L.AQ[lane + NX * l] * L.qk[l];
 #pragma unroll
-      for (int l = 0; l < NU; ++l) a3 += L.BR[lane + NX * l] * L.rk[l];
+      for (int l = 0; l < NU; ++l) a3 += L.B[lane + NX * l] * L.rk[l];
       gamma[(size_t)NX * row + lane] = L.cb[lane] - (a1 - a2 - a3);
     }
     if (zero_unused) {
@@ -251,12 +298,10 @@ __global__ void __launch_bounds__(WG) k_form_schur(Batch b, const float *__restr
   // Pinv(b,b) = -theta^-1
   float x[NX];
   gj_inverse<NX>(lane, th, x);
-  __syncthreads();  // every lane is done reading S(b,b) from A
-  if (lane < NX) {
+  wave_sync();  // S(b,b) read from A
 #pragma unroll
-    for (int r = 0; r < NX; ++r) L.A[r + NX * lane] = -x[r];
-  }
-  __syncthreads();
+  for (int r = 0; r < NX; ++r) L.A[r + NX * j] = -x[r];
+  wave_sync();
   if (valid && !row0) store_block(lane, Prow + NXX, [&](int i) { return L.A[i]; });
 }
 
@@ -312,56 +357,10 @@ __device__ __forceinline__ void q_lowrank(const float *__restrict__ vq, const fl
 
 __device__ __forceinline__ double bcast_dyn16_f64(double v, int p) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const float lo = bcast_dyn16<true>(__builtin_bit_cast(float, (uint32_t)b), p);
-  const float hi = bcast_dyn16<true>(__builtin_bit_cast(float, (uint32_t)(b >> 32)), p);
+  const float lo = bcast_dyn16(__builtin_bit_cast(float, (uint32_t)b), p);
+  const float hi = bcast_dyn16(__builtin_bit_cast(float, (uint32_t)(b >> 32)), p);
   return __builtin_bit_cast(double, ((unsigned long long)__builtin_bit_cast(uint32_t, hi) << 32) |
                                         __builtin_bit_cast(uint32_t, lo));
-}
-
-// d[r] += s_l[r] * w (r < 14), s_l the s of lane l of the 16-lane group:
-// v_fmac_f32_dpp with DPP row_newbcast:l, so a block product whose left
-// factor is held by columns (lane l: column l) needs no LDS and no
-// separate broadcast instruction.  The s_nop ahead of each seven covers the
-// wait states between a VALU write of an operand (or of EXEC, Nop4) and its
-// DPP read.  The group's lanes must all be active.
-#define MPC_NBF(k) "v_fmac_f32_dpp %" #k ", %" MPC_NBS##k ", %14 row_newbcast:%15 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
-#define MPC_NBS0 "7"
-#define MPC_NBS1 "8"
-#define MPC_NBS2 "9"
-#define MPC_NBS3 "10"
-#define MPC_NBS4 "11"
-#define MPC_NBS5 "12"
-#define MPC_NBS6 "13"
-#define MPC_NB7(nop)                                                                                          \
-  asm(nop MPC_NBF(0) MPC_NBF(1) MPC_NBF(2) MPC_NBF(3) MPC_NBF(4) MPC_NBF(5) MPC_NBF(6)                          \
-      : "+v"(d[o]), "+v"(d[o + 1]), "+v"(d[o + 2]), "+v"(d[o + 3]), "+v"(d[o + 4]), "+v"(d[o + 5]), "+v"(d[o + 6]) \
-      : "v"(s[o]), "v"(s[o + 1]), "v"(s[o + 2]), "v"(s[o + 3]), "v"(s[o + 4]), "v"(s[o + 5]), "v"(s[o + 6]),       \
-        "v"(w), "i"(l))
-template <int l, bool Nop4, int o>
-__device__ __forceinline__ void nb_fma7(float (&d)[NX], const float (&s)[NX], float w) {
-  static_assert(l >= 0 && l < 16 && o + 7 <= NX, "row lane, accumulator range");
-  if constexpr (Nop4)
-    MPC_NB7("s_nop 4\n");
-  else
-    MPC_NB7("s_nop 1\n");
-}
-#undef MPC_NB7
-#undef MPC_NBF
-#undef MPC_NBS0
-#undef MPC_NBS1
-#undef MPC_NBS2
-#undef MPC_NBS3
-#undef MPC_NBS4
-#undef MPC_NBS5
-#undef MPC_NBS6
-
-// d[r] += sum_{l in Ls, in order} s_l[r] * w[l]: a block product from the
-// left factor's columns (one per lane) and the calling lane's row of the
-// right factor's transpose
-template <bool Nop4, int... Ls>
-__device__ __forceinline__ void nb_product(float (&d)[NX], const float (&s)[NX], const float *w,
-                                           std::integer_sequence<int, Ls...>) {
-  ((nb_fma7<Ls, Nop4 && Ls == 0, 0>(d, s, w[Ls]), nb_fma7<Ls, false, 7>(d, s, w[Ls])), ...);
 }
 
 __global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(4))) k_form_split(Batch b, Params p,

@@ -296,6 +296,12 @@ hipError_t launch_split_prep(const Batch &b, const float *S, const float *gamma,
 hipError_t launch_pcg_split(const Batch &b, const uint4 *items, const uint32_t *bin_off, uint32_t n_bins,
                             const float *Ps, const float *ghat, float *lambda, uint32_t max_iter, float tol,
                             const uint32_t *status, uint32_t *iters, uint32_t *flag, float *eta, hipStream_t st);
+// Of all instances (N <= pcg_split_short_knots() each), a workgroup each with
+// half the knots per 16-lane row; same results bitwise.
+hipError_t launch_pcg_split_short(const Batch &b, uint32_t n_inst, const float *Ps, const float *ghat, float *lambda,
+                                  uint32_t max_iter, float tol, const uint32_t *status, uint32_t *iters,
+                                  uint32_t *flag, float *eta, hipStream_t st);
+uint32_t pcg_split_short_knots();
 uint32_t pcg_split_max_knots();
 uint32_t pcg_split_bin_groups();
 uint32_t pcg_split_max_items();

@@ -217,7 +217,31 @@ __device__ __forceinline__ void rot_mtv3(const float (&M0)[16], float x0, const 
 #undef MPC_HORNER3
 #undef MPC_HSTEP
 
-// Four / five interleaved accumulations a_k += sum_{n=1..15} M_k[n] * ror_n(x_k),
+// two blocks of rot_mtv3
+#define MPC_HSTEP(m0, m1)                                                        \
+  "v_mul_f32 %2, %" #m0 ", %4\n"                                                 \
+  "v_mul_f32 %3, %" #m1 ", %5\n"                                                 \
+  "v_add_f32_dpp %0, %0, %2 row_ror:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+  "v_add_f32_dpp %1, %1, %3 row_ror:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define MPC_HORNER2(k0, k1, k2)                                                                        \
+  asm(MPC_HSTEP(6, 7) MPC_HSTEP(8, 9) MPC_HSTEP(10, 11)                                                  \
+      : "+v"(a0), "+v"(a1), "=&v"(t0), "=&v"(t1)                                                        \
+      : "v"(x0), "v"(x1), "v"(M0[k0]), "v"(M1[k0]), "v"(M0[k1]), "v"(M1[k1]), "v"(M0[k2]), "v"(M1[k2]))
+__device__ __forceinline__ void rot_mtv2(const float (&M0)[16], float x0, const float (&M1)[16], float x1, float &c0,
+                                         float &c1) {
+  float a0 = M0[1] * x0, a1 = M1[1] * x1, t0, t1;
+  MPC_HORNER2(2, 3, 4);
+  MPC_HORNER2(5, 6, 7);
+  MPC_HORNER2(8, 9, 10);
+  MPC_HORNER2(11, 12, 13);
+  MPC_HORNER2(14, 15, 0);
+  c0 = a0;
+  c1 = a1;
+}
+#undef MPC_HORNER2
+#undef MPC_HSTEP
+
+// Three to five interleaved accumulations a_k += sum_{n=1..15} M_k[n] * ror_n(x_k),
 // three terms per asm statement; an s_nop ahead of the first (the two wait
 // states between a VALU write of x_k and its DPP read)
 #define MPC_TERM(n, acc, x, m) \
@@ -239,6 +263,22 @@ __device__ __forceinline__ void rot_fma15x4(float &a, float xa, const float (&Ma
 }
 #undef MPC_B4
 #undef MPC_T4
+#define MPC_T3(n, m0, m1, m2) MPC_TERM(n, 0, 3, m0) MPC_TERM(n, 1, 4, m1) MPC_TERM(n, 2, 5, m2)
+#define MPC_B3(pre, n0, n1, n2)                                                                               \
+  asm(pre MPC_T3(n0, 6, 7, 8) MPC_T3(n1, 9, 10, 11) MPC_T3(n2, 12, 13, 14)                                      \
+      : "+v"(a), "+v"(b), "+v"(c)                                                                               \
+      : "v"(xa), "v"(xb), "v"(xc), "v"(Ma[n0]), "v"(Mb[n0]), "v"(Mc[n0]), "v"(Ma[n1]), "v"(Mb[n1]), "v"(Mc[n1]), \
+        "v"(Ma[n2]), "v"(Mb[n2]), "v"(Mc[n2]))
+__device__ __forceinline__ void rot_fma15x3(float &a, float xa, const float (&Ma)[16], float &b, float xb,
+                                            const float (&Mb)[16], float &c, float xc, const float (&Mc)[16]) {
+  MPC_B3("s_nop 1\n", 1, 2, 3);
+  MPC_B3("", 4, 5, 6);
+  MPC_B3("", 7, 8, 9);
+  MPC_B3("", 10, 11, 12);
+  MPC_B3("", 13, 14, 15);
+}
+#undef MPC_B3
+#undef MPC_T3
 #define MPC_T5(n, m0, m1, m2, m3, m4) \
   MPC_TERM(n, 0, 5, m0) MPC_TERM(n, 1, 6, m1) MPC_TERM(n, 2, 7, m2) MPC_TERM(n, 3, 8, m3) MPC_TERM(n, 4, 9, m4)
 #define MPC_B5(pre, n0, n1, n2)                                                                                  \
@@ -579,6 +619,250 @@ k_pcg_split(Batch b, const uint4 *__restrict__ items, const uint32_t *__restrict
   }
 }
 
+// ------------------------------------------------- short instances ----
+// A few short instances (N <= 64), a workgroup of up to four waves each: the
+// iteration above with the eight knots of a group on two 16-lane rows, four
+// each, so that twice the SIMDs share the products.  Bitwise the same, so each
+// knot keeps the form of its second product (L^_5 .. L^_7 the Horner form), and
+// a slot whose two rows differ in it takes both.  With knots 0, 1, 4, 5 on the
+// even row and 2, 3, 6, 7 on the odd one that is one slot of the four:
+//   slot  knot (even, odd row)  first product  second product
+//   0     0, 2                  rows L^_t      transposed rows L^_{t+1}
+//   1     1, 3                  rows L^_t      transposed rows L^_{t+1}
+//   2     4, 6                  rows L^_t      Horner from the rows L^_{t+1} (slot 3's)
+//   3     5, 7                  rows L^_t      even: Horner from rows, odd: transposed rows
+// All blocks are in registers, neighbours on the other row come by lane swaps,
+// and the group's sums pass from row to row in the knots' order.  The group's
+// outer neighbour is knot 8g - 1 for the even row and 8g + 8 for the odd one.
+// Iterations of N = 64 take 0.92 us against 1.17 (173 of them on a device of
+// 256 instances 238 -> 187 us), the layer's solves of 256 instances 594 -> 471
+// us on average.
+constexpr int SH_RK = 4;  // knots per row
+
+constexpr int SH_NT = 256;               // four waves
+constexpr int SH_KNOTS = 64;
+constexpr int SH_GRP = SH_KNOTS / RK;    // groups of eight knots
+
+struct ShortShared {
+  float slot[SH_NT / 16 * SLOT];         // a block per row, to transpose it
+  float zb[(SH_GRP + 2) * 2 * 16];       // staged first and last knot of group + 1, zeros at both ends
+  alignas(16) float red[2][2 * SH_GRP];  // group sums; the second half takes the writes of the even rows
+};
+
+// u of the even rows and v of the even rows | u of the odd rows and v of the
+// odd rows, in the even | odd rows
+__device__ __forceinline__ void swap16(float u, float v, float &evens, float &odds) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, u), __builtin_bit_cast(uint32_t, v),
+                                                  false, false);
+  evens = __builtin_bit_cast(float, (uint32_t)r[0]);
+  odds = __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+
+__global__ void __launch_bounds__(SH_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_pcg_split_short(Batch b, const float *__restrict__ Ps, const float *__restrict__ ghat, float *__restrict__ lambda,
+                  uint32_t max_iter, float tol, const uint32_t *__restrict__ status, uint32_t *__restrict__ iters_out,
+                  uint32_t *__restrict__ flag_out, float *__restrict__ eta_out) {
+  __shared__ ShortShared sh;
+  const uint32_t tid = threadIdx.x, inst = blockIdx.x;
+  const uint32_t i = tid & 15u, row = tid >> 4, g = tid >> 5;
+  const bool odd = row & 1u;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t d = ror_step(tid);
+  for (uint32_t k = tid; k < (SH_GRP + 2) * 2 * 16; k += SH_NT) sh.zb[k] = 0.f;
+  if (tid < 4u * SH_GRP) (&sh.red[0][0])[tid] = 0.f;
+  const uint32_t N = inst_len(b, inst), K0 = inst_first(b, inst);
+  if (status && !(status[inst] & ST_ACTIVE)) return;
+  __syncthreads();  // LDS cleared
+  if (16u * w >= N) return;  // no knots: the other waves' barriers go on without this one
+  const uint32_t cap = pcg_cap(max_iter, N);
+  const bool lane_ok = i < (uint32_t)NX;
+
+  // the slots' knots
+  const uint32_t t0 = RK * g + (odd ? 2u : 0u);
+  auto knot = [&](int t) { return t0 + (uint32_t)(t & 1) + (t & 2 ? 4u : 0u); };
+  const float *Pw = Ps + (size_t)S_STRIDE * K0;  // the instance's rows
+  const uint32_t il = lane_ok ? i : 0u;
+  auto clamped = [&](int t) { return knot(t) < N ? knot(t) : N - 1u; };
+  float lam[SH_RK], r[SH_RK], p[SH_RK], y[SH_RK];
+  bool any = false;
+#pragma unroll
+  for (int t = 0; t < SH_RK; ++t) {
+    const bool has = knot(t) < N && lane_ok;
+    const float l = lambda[(size_t)NX * (K0 + clamped(t)) + il], h = ghat[(size_t)NX * (K0 + clamped(t)) + il];
+    lam[t] = has ? l : 0.f;
+    r[t] = has ? h : 0.f;
+    any = any || lam[t] != 0.f;
+  }
+  // lambda^ = W^-1 lambda by back substitution, four knots in lockstep (above)
+  if (__builtin_amdgcn_ballot_w64(any) != 0) {
+    float wr[SH_RK][NX], den[NX], lh[SH_RK];
+    const uint32_t td = i & (SH_RK - 1);
+    const uint32_t kd = t0 + (td & 1u) + (td & 2u ? 4u : 0u);
+#pragma unroll
+    for (int k = 0; k < NX; ++k) den[k] = at(Pw, S_STRIDE * (kd < N ? kd : N - 1u) + NXX + k + NX * k);
+#pragma unroll
+    for (int t = 0; t < SH_RK; ++t) {
+      lh[t] = 0.f;
+#pragma unroll
+      for (int c = 0; c < NX; ++c) wr[t][c] = at(Pw, S_STRIDE * clamped(t) + NXX + il + NX * c);
+    }
+#pragma unroll
+    for (int k = NX - 1; k >= 0; --k) {
+      float num = 0.f;
+#pragma unroll
+      for (int t = 0; t < SH_RK; ++t) {
+        const float v = bcast_dyn16(lam[t], k);
+        num = td == (uint32_t)t ? v : num;
+      }
+      const float quo = num / den[k];
+#pragma unroll
+      for (int t = 0; t < SH_RK; ++t) {
+        const float xk = bcast_dyn16(quo, t);
+        lh[t] = (int)i == k ? xk : lh[t];
+        lam[t] -= wr[t][k] * xk;
+      }
+      pin(lh);
+      pin(lam);
+    }
+#pragma unroll
+    for (int t = 0; t < SH_RK; ++t) lam[t] = knot(t) < N && lane_ok ? lh[t] : 0.f;
+  }
+  asm volatile("" ::: "memory");  // the block reads below stay behind the rows of W
+  // the rows of L^ of the slots' knots; transposed through the row's LDS slot
+  // those of the knot after slots 0 and 1 and, odd rows, after slot 3 (even
+  // rows hold its rows there)
+  float L[SH_RK][16], K0r[16], K1r[16], Z[16];
+  uint32_t roff[16];
+  block_offsets(roff, t0, i, d);
+  auto block = [&](float (&M)[16], uint32_t dk) {  // rows of L^_{t0 + dk}, L^_0 = 0
+    load_lrows(M, lane_ok && t0 + dk < N && t0 + dk > 0u, i, d, Pw + S_STRIDE * dk, roff);
+  };
+  float *mine = sh.slot + row * SLOT;
+  auto transpose = [&](float (&M)[16], const float (&A)[16]) {
+    write_slot_t(mine, i, d, A);
+    wave_sync();
+    read_slot(M, mine, i);
+    wave_sync();
+  };
+  block(L[0], 0);
+  block(L[1], 1);
+  block(L[2], 4);
+  block(L[3], 5);
+  block(Z, 6);
+  transpose(K0r, L[1]);
+  {
+    float A[16];
+    block(A, 2);
+    transpose(K1r, A);
+    transpose(A, Z);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) Z[n] = odd ? A[n] : Z[n];
+  }
+
+  float *zs = sh.zb + (g + 1u) * 32u + (odd ? 16u : 0u) + i;
+  const float *zn_src = sh.zb + (odd ? (g + 2u) * 32u : g * 32u + 16u) + i;
+  auto smv = [&](float pn) {
+    float x0p, x1n, x2p, x3n, e, o;
+    swap16(pn, p[1], x0p, o);
+    swap16(p[0], p[2], e, o);
+    x1n = odd ? e : o;
+    swap16(p[1], p[3], e, o);
+    x2p = odd ? e : o;
+    swap16(p[2], pn, e, x3n);
+    y[0] = fmaf(L[0][0], x0p, -p[0]);
+    y[1] = fmaf(L[1][0], p[0], -p[1]);
+    y[2] = fmaf(L[2][0], x2p, -p[2]);
+    y[3] = fmaf(L[3][0], p[2], -p[3]);
+    rot_fma15x4(y[0], x0p, L[0], y[1], p[0], L[1], y[2], x2p, L[2], y[3], p[2], L[3]);
+    float yd = fmaf(Z[0], x3n, y[3]), c2, c3;
+    y[0] = fmaf(K0r[0], p[1], y[0]);
+    y[1] = fmaf(K1r[0], x1n, y[1]);
+    rot_fma15x3(y[0], p[1], K0r, y[1], x1n, K1r, yd, x3n, Z);
+    rot_mtv2(L[3], p[3], Z, x3n, c2, c3);
+    y[2] += c2;
+    c3 = y[3] + c3;
+    y[3] = odd ? yd : c3;
+  };
+  // sum over the group's eight knots of u v in their order, in the odd row
+  auto group_dot = [&](const float (&u)[SH_RK], const float (&v)[SH_RK], bool neg) {
+    auto add = [&](float s, int t) { return fmaf(neg ? -u[t] : u[t], v[t], s); };
+    float s, e, o;
+    s = add(add(0.f, 0), 1);
+    swap16(s, s, s, o);   // knots 0, 1 to the odd row
+    s = add(add(s, 0), 1);
+    swap16(s, s, e, s);   // .. 3 to the even one
+    s = add(add(s, 2), 3);
+    swap16(s, s, s, o);
+    return add(add(s, 2), 3);
+  };
+  float *red_dst = &sh.red[0][odd ? g : SH_GRP + g];
+  auto post = [&](int k, float s) { red_dst[k * 2 * SH_GRP] = row_total(s); };
+  // in the order of the kernel above: pairs, then the levels of row_total
+  // (past the eight groups it adds zeros)
+  static_assert(SH_GRP == 8, "eight group sums");
+  auto total = [&](int k) {
+    const float4 a = *reinterpret_cast<const float4 *>(&sh.red[k][0]), c = *reinterpret_cast<const float4 *>(&sh.red[k][4]);
+    return (((a.x + a.y) + (a.z + a.w)) + ((c.x + c.y) + (c.z + c.w))) + 0.f;
+  };
+  *zs = odd ? lam[3] : lam[0];
+  __syncthreads();
+  float pn = *zn_src;
+  // (the iteration as above)
+#pragma unroll
+  for (int t = 0; t < SH_RK; ++t) p[t] = lam[t];
+  uint32_t it = ~0u;  // the first pass is not counted
+  float eta = 0.f, tol_i = tol;
+  bool first = true, conv, run;
+  do {
+    smv(pn);
+    post(0, group_dot(p, y, false));
+    __syncthreads();
+    const float quo = eta / total(0), alpha = first ? 1.f : quo;
+#pragma unroll
+    for (int t = 0; t < SH_RK; ++t) r[t] -= alpha * y[t];
+    *zs = odd ? -r[3] : -r[0];
+    post(1, group_dot(r, r, true));
+    __syncthreads();
+    const float zn = *zn_src, eta_new = total(1);
+    const float alpha_l = first ? 0.f : alpha;
+#pragma unroll
+    for (int t = 0; t < SH_RK; ++t) lam[t] += alpha_l * p[t];
+    // taken in the last iteration too (p is not used after it)
+    const float quo_b = eta_new / eta, beta = first ? 0.f : quo_b;
+    eta = eta_new;
+#pragma unroll
+    for (int t = 0; t < SH_RK; ++t) p[t] = fmaf(beta, p[t], -r[t]);
+    pn = fmaf(beta, pn, zn);
+    if (first && tol < 0.f) tol_i = fmaxf(-tol * fabsf(eta), FLT_MIN);
+    ++it;
+    first = false;
+    conv = uniform(fabsf(eta) < tol_i);  // eta is the same in every lane
+    run = !conv && it < cap;
+  } while (run);
+
+  // lambda = W lambda^, two knots at a time
+  uint32_t ie = i;
+  asm volatile("" : "+v"(ie));
+  uint32_t woff[16];
+  block_offsets(woff, t0, ie, d);
+#pragma unroll
+  for (int t = 0; t < SH_RK; t += 2) {
+    float Wr[2][16], v[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      load_lrows(Wr[u], lane_ok && knot(t + u) < N, i, d, Pw + S_STRIDE * (2 * t + u) + NXX, woff);
+    rot_mv2(Wr[0], lam[t], v[0], Wr[1], lam[t + 1], v[1]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (knot(t + u) < N && lane_ok) lambda[(size_t)NX * (K0 + knot(t + u)) + i] = v[u];
+  }
+  if (tid == 0) {
+    if (iters_out) iters_out[inst] = it;
+    if (flag_out) flag_out[inst] = conv ? 0u : 1u;
+    if (eta_out) eta_out[inst] = fabsf(eta);
+  }
+}
+
 }  // namespace
 
 uint32_t pcg_split_max_knots() { return (uint32_t)KNOTS; }
@@ -610,6 +894,17 @@ hipError_t launch_pcg_split(const Batch &b, const uint4 *items, const uint32_t *
   }
   hipLaunchKernelGGL(k_pcg_split, dim3(n_bins), dim3(NT), smem, st, b, items, bin_off, Ps, ghat, lambda, max_iter,
                      tol, status, iters, flag, eta);
+  return hipGetLastError();
+}
+
+uint32_t pcg_split_short_knots() { return (uint32_t)SH_KNOTS; }
+
+hipError_t launch_pcg_split_short(const Batch &b, uint32_t n_inst, const float *Ps, const float *ghat, float *lambda,
+                                  uint32_t max_iter, float tol, const uint32_t *status, uint32_t *iters,
+                                  uint32_t *flag, float *eta, hipStream_t st) {
+  if (n_inst == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_pcg_split_short, dim3(n_inst), dim3(SH_NT), 0, st, b, Ps, ghat, lambda, max_iter, tol, status,
+                     iters, flag, eta);
   return hipGetLastError();
 }
 

@@ -61,6 +61,7 @@ struct mpc_handle {
   uint4 *split_items = nullptr;
   uint32_t *split_off = nullptr;
   uint32_t n_split_bins = 0;
+  bool split_short = false;  // launch_pcg_split_short instead of the bins
   bool split_ok = false;  // every horizon of the layout fits the split-form kernel
   float *ghat = nullptr;
   // the batched SQP in split form forms no S: each instance's rho of its last
@@ -729,6 +730,20 @@ static int build_pcg_plan(mpc_handle *h) {
   // split form: every instance in bins of the 512-lane kernel
   h->split_ok = n_inst > 0;
   for (uint32_t i = 0; i < n_inst; ++i) h->split_ok = h->split_ok && horizons[i] <= pcg_split_max_knots();
+  // Few short instances: a workgroup each of the kernel that gives each twice
+  // the waves, while there is a compute unit for each or the waves (of 16
+  // knots) are at most half the SIMDs.  Two SQP iterations of 173 PCG
+  // iterations, the bins below / that kernel: 256 of N = 64 637 / 535 us, 256 of
+  // N = 16 533 / 415, 512 of N = 8 562 / 441; past the line 512 of N = 64 735 / 747
+  // us, 512 of N = 32 628 / 636.  At N > 64 its eight waves take two per SIMD
+  // (N = 128: closed loop 5 % slower).
+  uint64_t waves = 0;
+  uint32_t longest = 0;
+  for (uint32_t i = 0; i < n_inst; ++i) {
+    waves += (horizons[i] + 15u) / 16u;
+    longest = std::max(longest, horizons[i]);
+  }
+  h->split_short = h->split_ok && longest <= pcg_split_short_knots() && (n_inst <= h->n_cu || waves <= 2u * h->n_cu);
   h->n_split_bins = 0;
   if (h->split_ok) {
     std::vector<uint32_t> all(n_inst);
@@ -1099,8 +1114,11 @@ static hipError_t pcg_batch(mpc_handle *h, float *d_lambda, const uint32_t *d_st
     // the caller formed it already), then one launch over the bins
     e = prepped ? hipSuccess : launch_split_prep(b, h->S, h->gamma, d_status, h->P, h->ghat, st);
     if (e == hipSuccess)
-      e = launch_pcg_split(b, h->split_items, h->split_off, h->n_split_bins, h->P, h->ghat, d_lambda, max_iter, tol,
-                           d_status, h->pcg_iters, h->pcg_flag, h->pcg_eta, st);
+      e = h->split_short
+              ? launch_pcg_split_short(b, h->n_inst, h->P, h->ghat, d_lambda, max_iter, tol, d_status, h->pcg_iters,
+                                       h->pcg_flag, h->pcg_eta, st)
+              : launch_pcg_split(b, h->split_items, h->split_off, h->n_split_bins, h->P, h->ghat, d_lambda, max_iter,
+                                 tol, d_status, h->pcg_iters, h->pcg_flag, h->pcg_eta, st);
     if (e == hipSuccess && mid) e = hipEventRecord(mid, st);
     return e;
   }

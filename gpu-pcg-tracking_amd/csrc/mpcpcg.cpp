@@ -42,7 +42,6 @@ struct mpc_handle {
   float *Cl = nullptr;  // [CL_STRIDE T] compact dynamics rows of the split path (G, C not written)
   float *S = nullptr, *P = nullptr, *gamma = nullptr, *dz = nullptr;
   float *knot_merits = nullptr;  // [9 T]
-  float *merits = nullptr;       // [9 B]
   float *xs = nullptr;           // [14 B]
   float *drho = nullptr, *merit0 = nullptr, *rho1 = nullptr;
   uint32_t *status_ws = nullptr, *sqp_done = nullptr, *pcg_iters = nullptr, *pcg_flag = nullptr;
@@ -284,7 +283,7 @@ const char *mpc_status_string(int s) {
 
 static void free_all(mpc_handle *h) {
   void *ptrs[] = {h->G, h->Ginv, h->gq, h->Cl, h->C, h->g, h->c, h->S, h->P, h->gamma, h->dz, h->knot_merits,
-                  h->merits, h->xs, h->drho, h->merit0, h->rho1, h->status_ws, h->sqp_done,
+                  h->xs, h->drho, h->merit0, h->rho1, h->status_ws, h->sqp_done,
                   h->pcg_iters, h->pcg_flag, h->pcg_eta, h->t0, h->knot_inst, h->inst_k0, h->bin_items,
                   h->bin_off, h->big_list, h->team_list, h->team_one, h->team_err, h->mbox, h->dir_order,
                   h->pcg_done, h->pool_ctr, h->split_items, h->split_off, h->ghat, h->rho_used,
@@ -339,7 +338,6 @@ int mpc_create(const mpc_config *cfg, mpc_handle **out) {
             alloc((void **)&h->gamma, sizeof(float) * NX * T) &&
             alloc((void **)&h->dz, sizeof(float) * NXU * T) &&
             alloc((void **)&h->knot_merits, sizeof(float) * 9 * T) &&
-            alloc((void **)&h->merits, sizeof(float) * 9 * B) &&
             alloc((void **)&h->xs, sizeof(float) * NX * B) &&
             alloc((void **)&h->drho, sizeof(float) * B) &&
             alloc((void **)&h->merit0, sizeof(float) * B) &&
@@ -587,11 +585,29 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
 
   HIP_TRY(hipMemcpyAsync(h->xs, d_xu, sizeof(float) * NX, hipMemcpyDeviceToDevice, st));
   HIP_TRY(launch_merit(b, prm, d_xu, nullptr, d_ee_ref, h->xs, nullptr, 8, 1, h->knot_merits, st));
-  HIP_TRY(launch_merit_reduce(b, h->knot_merits, 1, h->merits, st));
-  HIP_TRY(hipMemcpyAsync(h->h_merits, h->merits, sizeof(float), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
+  // what the host decides on, its kernels write to pinned host memory
+  // themselves (a copy of a few words took 3.5 us and a gap each, four of them
+  // in the first iteration: one iteration at N = 32 194 -> 186 us, 179 with the
+  // blocks ahead of the wait; three at N = 128 1159 -> 1137)
+  HIP_TRY(launch_merit_reduce(b, h->knot_merits, 1, h->h_merits, st));
+  HIP_TRY(hipEventRecord(h->ev[2], st));
+  // the blocks of the current iterate, which change nothing of the caller's:
+  // the first iteration's are formed while the host waits for the merit
+  auto form_blocks = [&](bool kkt, bool schur) {
+    hipError_t e = hipSuccess;
+    if (kkt) {
+      e = launch_form_kkt(b, prm, d_xu, d_ee_ref, h->xs, nullptr, h->G, h->C, h->g, h->c, st);
+      h->gc_compact = false;  // G and C written in full
+    }
+    if (e == hipSuccess && schur)
+      e = launch_form_schur(b, h->G, h->C, h->g, h->c, nullptr, *rho, nullptr, h->S, h->P, h->gamma, h->Ginv, 0, st);
+    return e;
+  };
+  if (cfg.sqp_max_iter > 0) HIP_TRY(form_blocks(true, true));
+  HIP_TRY(hipEventSynchronize(h->ev[2]));
   float merit0 = h->h_merits[0];
   if (!std::isfinite(merit0)) {  // nothing a line search could improve on
+    HIP_TRY(hipStreamSynchronize(st));
     s.sqp_us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
     return MPC_ERR_NONFINITE;
   }
@@ -601,18 +617,14 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
   bool not_aborted = true;
   bool time_exit = false;
   for (uint32_t it = 0; it < cfg.sqp_max_iter; ++it) {
-    HIP_TRY(launch_form_kkt(b, prm, d_xu, d_ee_ref, h->xs, nullptr, h->G, h->C, h->g, h->c, st));
-    h->gc_compact = false;  // G and C written in full
+    if (it > 0) HIP_TRY(form_blocks(true, false));
     if ((time_exit = over_budget())) break;  // toplevel.cuh:271
-    HIP_TRY(launch_form_schur(b, h->G, h->C, h->g, h->c, nullptr, *rho, nullptr, h->S, h->P, h->gamma,
-                              h->Ginv, 0, st));
+    if (it > 0) HIP_TRY(form_blocks(false, true));
     if ((time_exit = over_budget())) break;  // toplevel.cuh:283
     HIP_TRY(hipEventRecord(h->ev[0], st));
-    HIP_TRY(pcg_single(h, N, h->S, h->P, h->gamma, d_lambda, sqp_pcg_cap(cfg), cfg.pcg_exit_tol, h->pcg_iters,
-                       h->pcg_flag, st));
+    HIP_TRY(pcg_single(h, N, h->S, h->P, h->gamma, d_lambda, sqp_pcg_cap(cfg), cfg.pcg_exit_tol, h->h_pcg,
+                       h->h_pcg + 1, st));
     HIP_TRY(hipEventRecord(h->ev[1], st));
-    HIP_TRY(hipMemcpyAsync(h->h_pcg, h->pcg_iters, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(h->h_pcg + 1, h->pcg_flag, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     HIP_TRY(launch_compute_dz(b, h->Ginv, h->C, h->g, d_lambda, nullptr, h->dz, st));
     if (cfg.flags & FLAG_DIRECT_SOLVE) {
       h->h_rho[3] = *rho;
@@ -625,8 +637,7 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
                               st));
     }
     HIP_TRY(launch_merit(b, prm, d_xu, h->dz, d_ee_ref, h->xs, nullptr, 0, 8, h->knot_merits, st));
-    HIP_TRY(launch_merit_reduce(b, h->knot_merits, 8, h->merits, st));
-    HIP_TRY(hipMemcpyAsync(h->h_merits, h->merits, sizeof(float) * 8, hipMemcpyDeviceToHost, st));
+    HIP_TRY(launch_merit_reduce(b, h->knot_merits, 8, h->h_merits, st));
     HIP_TRY(hipStreamSynchronize(st));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, h->ev[0], h->ev[1]));

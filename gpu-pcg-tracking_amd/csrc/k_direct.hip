@@ -10,15 +10,19 @@
 // Solve of A x = r:
 //   forward   y_b = r_b - E_b y_{b-1},   z_b = D_b^-1 y_b
 //   backward  x_{N-1} = z_{N-1},   x_b = z_b - E_{b+1}^T x_{b+1}
-// with r = -gamma, then `refine` steps of iterative refinement: the
+// (from the other end E_b couples b to b + 1 in the same way, with B_{b+1}^T,
+// and is kept in row b + 1), with r = -gamma, then `refine` steps of iterative refinement: the
 // residual -gamma + S lambda in fp64 from the fp32 blocks, the same solve on
 // it, lambda += x.  The fp32 elimination alone is off by about cond(S) x eps
 // (1e-4..1e-2 relative on these systems); each step multiplies the error by
 // about that factor, down to the fp32 storage of lambda.
 //
-// Mapping: one wave per instance, instances longest first (few waves, one per
-// SIMD: the sweeps are bound by their dependent chains, so what counts is the
-// instructions and latencies of a step, below).  The residual is formed for
+// Mapping: one wave per instance, or with two and more refinement steps two, one
+// from each end, which meet in the middle knot (a block tridiagonal system
+// eliminates from both ends with the same operations, so the chain is half as
+// long); instances longest first (few waves, one per SIMD: the sweeps are
+// bound by their dependent chains, so what counts is the instructions and
+// latencies of a step, below).  The residual is formed for
 // all knots of all instances at once, one group per knot.
 //
 // Reference: the QDLDL path of sqpSolve (PCG_SOLVE = 0, toplevel.cuh:160-215,
@@ -36,8 +40,6 @@ constexpr int GROUP = 16;
 constexpr int GROUPS_PER_WG = 4;
 constexpr int WG = GROUP * GROUPS_PER_WG;
 
-__device__ __forceinline__ float *slot_E(float *work, size_t row) { return work + (size_t)S_STRIDE * row; }
-__device__ __forceinline__ float *slot_Dinv(float *work, size_t row) { return work + (size_t)S_STRIDE * row + NXX; }
 __device__ __forceinline__ float *slot_z(float *work, size_t row) { return work + (size_t)S_STRIDE * row + 2 * NXX; }
 
 // the instance of a wave
@@ -54,6 +56,24 @@ __device__ __forceinline__ Pick pick_instance(const Batch &b, const uint32_t *or
   p.N = inst_len(b, p.inst);
   p.live = !(status && !(status[p.inst] & ST_ACTIVE));
   return p;
+}
+
+// One side's elimination: chain positions 0 .. n are the knots from its end of
+// the instance to the meeting knot (n), side 1 counting backwards.  With one
+// side that is the last knot, and nothing meets there.
+struct Chain {
+  uint32_t side, n, N;
+  // the knot at position k
+  __device__ __forceinline__ uint32_t knot(uint32_t k) const { return side ? N - 1u - k : k; }
+  // the block row that holds the coupling of positions k - 1 and k (and, in
+  // the workspace, E of position k); row 0, with zeros, for k = 0
+  __device__ __forceinline__ uint32_t link(uint32_t k) const { return k == 0 ? 0u : side ? N - k : k; }
+};
+
+template <bool TWO>
+__device__ __forceinline__ Chain chain_of(uint32_t N, uint32_t side) {
+  const uint32_t m = TWO ? N / 2u : N - 1u;  // the meeting knot
+  return Chain{side, side ? N - 1u - m : m, N};
 }
 
 // ---- factorisation -----------------------------------------------------------
@@ -76,8 +96,14 @@ __device__ __forceinline__ Pick pick_instance(const Batch &b, const uint32_t *or
 // division on the chain, 528 clocks per pivot).
 constexpr int RS = 16;  // LDS row stride of a block (16-byte aligned rows)
 struct alignas(16) FacWaveLds {
-  float B[2][NX * RS + RS];  // B_b by rows: B(r, c) at c + RS r, knots alternating (the last RS: unused lanes' writes)
-  float Dinv[NX * RS];       // D_{b-1}^-1 by columns: (m, j) at m + RS j
+  float B[2][NX * RS + RS];  // B by rows: B(r, c) at c + RS r, knots alternating (the last RS: unused lanes' writes)
+  float Dinv[NX * RS];       // the D^-1 before by columns: (m, j) at m + RS j
+};
+template <bool TWO>
+struct alignas(16) DirectLds {
+  FacWaveLds side[TWO ? 2 : 1];
+  float meet[4][64];  // side 1's part of D at the meeting knot, by slot and lane
+  float v[16], x[16]; // in the sweeps: its part of y there; y, then x
 };
 
 __device__ __forceinline__ float lane_value(float v, uint32_t byte_addr) {
@@ -238,8 +264,10 @@ __device__ __forceinline__ float *at(float *base, uint32_t off) {
   return reinterpret_cast<float *>(reinterpret_cast<char *>(base) + 4u * off);
 }
 
-__device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restrict__ S, float *work, const Pick &p,
-                                           uint32_t lane) {
+template <bool TWO>
+__device__ __forceinline__ void factor_wave(DirectLds<TWO> &lds, const float *__restrict__ S, float *work, const Pick &p,
+                                           const Chain &ch, uint32_t lane) {
+  FacWaveLds &L = lds.side[ch.side];
   const uint32_t q = lane >> 4, jl = lane & 15u, j = jl < (uint32_t)NX ? jl : NX - 1;
   const bool tail = q < 2u;  // slot 3 holds rows 12, 13 in quarters 0, 1
   Quarters qs;
@@ -249,8 +277,10 @@ __device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restri
     qs.mask[t] = 0xFFFFull << (16 * t);
     qs.from[t] = 4u * (16u * t + jl);
     const uint32_t r = 4u * t + q, i = lane + 64u * t;
-    rr[t] = r < (uint32_t)NX ? r : 0u;                                               // clamped row
-    bl[t] = i < (uint32_t)NXX ? i / NX + RS * (i % NX) : (uint32_t)(NX * RS) + jl;   // place of element i of B
+    rr[t] = r < (uint32_t)NX ? r : 0u;  // clamped row
+    // place of element i of the block (side 1: transposed)
+    const uint32_t br = ch.side ? i / NX : i % NX, bc = ch.side ? i % NX : i / NX;
+    bl[t] = i < (uint32_t)NXX ? bc + RS * br : (uint32_t)(NX * RS) + jl;
   }
   const float *Sp = S + (size_t)S_STRIDE * p.K0;
   float *W = work + (size_t)S_STRIDE * p.K0;
@@ -259,11 +289,12 @@ __device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restri
   // past the block in its row is read with it and not used)
   float a_nxt[2][4], b_nxt[2][4];
   auto load = [&](float (&a)[4], float (&bb)[4], uint32_t k) {
-    const float *Sr = Sp + (size_t)S_STRIDE * (k < p.N ? k : p.N - 1u);
+    const uint32_t kc = k < ch.n ? k : ch.n;
+    const float *Sd = Sp + (size_t)S_STRIDE * ch.knot(kc), *Sl = Sp + (size_t)S_STRIDE * ch.link(kc);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      a[t] = at(Sr, oa)[4 * t];
-      bb[t] = at(Sr, lane)[64 * t];
+      a[t] = at(Sd, oa)[4 * t];
+      bb[t] = at(Sl, lane)[64 * t];
     }
   };
   auto put_b = [&](const float (&bb)[4], uint32_t k) {
@@ -301,15 +332,26 @@ __device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restri
 #pragma unroll
         for (int t = 0; t < 4; ++t) e[t] += br[t][m] * dv[m];
     }
+    const bool meets = k == ch.n;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) a[t] = t < 3 || tail ? -a[t] : 0.f;
+    for (int t = 0; t < 4; ++t) a[t] = (t < 3 || tail) && !(meets && ch.side) ? -a[t] : 0.f;
     // D_b(r, j) = A_b(r, j) - sum_m E(r, m) B(j, m), m in order
     if (k > 0) block_updates(a, e, bj, std::make_integer_sequence<int, NX>{});
-    float *Wk = W + (size_t)S_STRIDE * k;
+    float *Wk = W + (size_t)S_STRIDE * ch.knot(k), *Wl = W + (size_t)S_STRIDE * ch.link(k);
     // lanes 14 and 15 store what lane 13 does
 #pragma unroll
-    for (int t = 0; t < 3; ++t) at(Wk, oe)[4 * t] = e[t];
-    if (tail) at(Wk, oe)[12] = e[3];
+    for (int t = 0; t < 3; ++t) at(Wl, oe)[4 * t] = e[t];
+    if (tail) at(Wl, oe)[12] = e[3];
+    if (TWO && meets) {  // side 1's part to side 0, which inverts
+      if (ch.side) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) lds.meet[t][lane] = a[t];
+      }
+      __syncthreads();
+      if (ch.side) return;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[t] += lds.meet[t][lane];
+    }
     float keep[4], pivots = 1.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -333,11 +375,11 @@ __device__ __forceinline__ void factor_wave(FacWaveLds &L, const float *__restri
   // B of the next knot goes to LDS ahead of the step that reads it
   put_b(b_nxt[1], 1);
   step(0, a_nxt[0], b_nxt[0]);
-  for (uint32_t k = 1; k < p.N; k += 2) {
+  for (uint32_t k = 1; k <= ch.n; k += 2) {
     put_b(b_nxt[0], k + 1);
     wave_sync();
     step(k, a_nxt[1], b_nxt[1]);
-    if (k + 1 >= p.N) break;
+    if (k + 1 > ch.n) break;
     put_b(b_nxt[1], k + 2);
     wave_sync();
     step(k + 1, a_nxt[0], b_nxt[0]);
@@ -395,106 +437,124 @@ __device__ __forceinline__ void load14(float (&v)[NX], const float *p) {
   }
 }
 
-// forward and backward sweeps of one instance on the right-hand side
-// r = -gamma, or with ACCUMULATE the workspace's z slots; lambda = x, or
+// forward and backward sweeps of one side of an instance on the right-hand
+// side r = -gamma, or with ACCUMULATE the workspace's z slots; lambda = x, or
 // lambda += x with ACCUMULATE
-template <bool ACCUMULATE>
-__device__ __forceinline__ void substitute(const float *__restrict__ gamma, float *work,
-                                          float *__restrict__ lambda, const Pick &p, uint32_t lane) {
+template <bool TWO, bool ACCUMULATE>
+__device__ __forceinline__ void substitute(DirectLds<TWO> &lds, const float *__restrict__ gamma, float *work,
+                                          float *__restrict__ lambda, const Pick &p, const Chain &ch, uint32_t lane) {
   const uint32_t q = lane >> 4, i = lane & 15u, j = i < (uint32_t)NX ? i : NX - 1;
   const uint32_t turn = q ^ (q >> 1);  // rows 0, 1, 3, 2 in order
   const bool el = i < (uint32_t)NX;
-  const uint32_t last = p.N - 1u;
   float *W = work + (size_t)S_STRIDE * p.K0, *lp = lambda + (size_t)NX * p.K0;
   const float *gp = ACCUMULATE ? nullptr : gamma + (size_t)NX * p.K0;
-  // knots k0 .. k0 + 3 of the forward sweep, knot k0 + turn in the row (the
-  // last knot's data again past the end): row j of E_k (strided; E_0 = 0),
-  // row j of D_k^-1 (= column j, D^-1 symmetric) and the right-hand side
+  // positions k0 .. k0 + 3 of the forward sweep, position k0 + turn in the row
+  // (the meeting knot's data again past it): row j of E_k (strided; E_0 = 0),
+  // row j of D_k^-1 (= column j, D^-1 symmetric) and the right-hand side (the
+  // meeting knot's on side 0 alone)
   struct Fwd {
     float er[NX], dr[NX], r;
   };
   auto load_f = [&](Fwd &f, uint32_t k0) {
-    const uint32_t k = k0 + turn < last ? k0 + turn : last;
-    const float *E = at(W, S_STRIDE * k + j);
+    const uint32_t k = k0 + turn < ch.n ? k0 + turn : ch.n;
+    const float *E = at(W, S_STRIDE * ch.link(k) + j);
 #pragma unroll
     for (int m = 0; m < NX; ++m) f.er[m] = E[NX * m];
-    load14(f.dr, at(W, S_STRIDE * k + NX * j) + NXX);
-    f.r = ACCUMULATE ? E[2 * NXX] : -*at(gp, NX * k + j);
+    const uint32_t kn = ch.knot(k);
+    load14(f.dr, at(W, S_STRIDE * kn + NX * j) + NXX);
+    const float r = ACCUMULATE ? at(W, S_STRIDE * kn + j)[2 * NXX] : -*at(gp, NX * kn + j);
+    f.r = ch.side && k == ch.n ? 0.f : r;
   };
-  float y = 0.f;
+  float y = 0.f, yo = 0.f;
   auto run_f = [&](const Fwd &f, uint32_t k0) {
-    float yo, t;  // the row's own y
+    float t;  // yo: the row's own y
     t = f.r - bdot(f.er, y);
     yo = t;
     y = pass_on<0>(t);
-    if (k0 + 1 < p.N) {
+    if (k0 + 1 <= ch.n) {
       t = f.r - bdot(f.er, y);
       yo = turn == 1u ? t : yo;
       y = pass_on<1>(t);
     }
-    if (k0 + 2 < p.N) {
+    if (k0 + 2 <= ch.n) {
       t = f.r - bdot(f.er, y);
       yo = turn == 2u ? t : yo;
       y = pass_on<2>(t);
     }
-    if (k0 + 3 < p.N) {
+    if (k0 + 3 <= ch.n) {
       t = f.r - bdot(f.er, y);
       yo = turn == 3u ? t : yo;
       y = pass_on<3>(t);
     }
     const float z = bdot(f.dr, yo);
-    if (el && k0 + turn < p.N) *at(W, S_STRIDE * (k0 + turn) + 2 * NXX + i) = z;
+    if (el && k0 + turn < ch.n) *at(W, S_STRIDE * ch.knot(k0 + turn) + 2 * NXX + i) = z;
   };
   Fwd f[3];
 #pragma unroll
   for (int u = 0; u < 3; ++u) load_f(f[u], 4u * u);
-  for (uint32_t k0 = 0; k0 < p.N; k0 += 12) {
+  for (uint32_t k0 = 0; k0 <= ch.n; k0 += 12) {
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const uint32_t k = k0 + 4u * u;
-      if (k >= p.N) break;
+      if (k > ch.n) break;
       run_f(f[u], k);
       load_f(f[u], k + 12u);
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // z is read by other lanes below
-  // backward: knot top - turn in the row (knot 0 again past the start):
-  // column j of E_{k+1} (x = 0 past the last knot, whatever is read there),
-  // z_k and the value that x_k is added to
+  // the meeting knot: y = side 0's + side 1's part, x = D^-1 y
+  const uint32_t km = chain_of<TWO>(p.N, 0).n;
+  const bool owner = turn == (ch.n & 3u);  // the row whose turn it was last
+  if (ch.side && owner) lds.v[i] = yo;
+  __syncthreads();  // (z, read by other lanes below, too)
+  if (!ch.side) {
+    float dr[NX];
+    load14(dr, at(W, S_STRIDE * km + NX * j) + NXX);
+    const float l = ACCUMULATE ? *at(lp, NX * km + j) : 0.f;
+    if (owner) lds.x[i] = TWO ? yo + lds.v[i] : yo;
+    wave_sync();
+    const float xm = bdot(dr, lds.x[j]);
+    wave_sync();
+    if (q == 0) lds.x[i] = xm;
+    if (el && q == 0) *at(lp, NX * km + i) = ACCUMULATE ? l + xm : xm;
+  }
+  __syncthreads();
+  // backward: position top - turn in the row (position 0 again past the
+  // start): column j of E_{k+1}, z_k and the value that x_k is added to
   struct Bwd {
     float ec[NX], z, l;
   };
-  auto load_b = [&](Bwd &f, int top) {
+  auto load_b = [&](Bwd &g, int top) {
     const uint32_t k = top - (int)turn > 0 ? (uint32_t)(top - (int)turn) : 0u;
-    load14(f.ec, at(W, S_STRIDE * (k < last ? k + 1u : last) + NX * j));
-    f.z = *at(W, S_STRIDE * k + 2 * NXX + j);
-    f.l = ACCUMULATE ? *at(lp, NX * k + j) : 0.f;
+    load14(g.ec, at(W, S_STRIDE * ch.link(k < ch.n ? k + 1u : ch.n) + NX * j));
+    const uint32_t kn = ch.knot(k);
+    g.z = *at(W, S_STRIDE * kn + 2 * NXX + j);
+    g.l = ACCUMULATE ? *at(lp, NX * kn + j) : 0.f;
   };
-  float x = 0.f;
-  auto run_b = [&](const Bwd &f, int top) {
+  float x = lds.x[j];
+  auto run_b = [&](const Bwd &g, int top) {
     float xo, t;
-    t = f.z - bdot(f.ec, x);
+    t = g.z - bdot(g.ec, x);
     xo = t;
     x = pass_on<0>(t);
     if (top >= 1) {
-      t = f.z - bdot(f.ec, x);
+      t = g.z - bdot(g.ec, x);
       xo = turn == 1u ? t : xo;
       x = pass_on<1>(t);
     }
     if (top >= 2) {
-      t = f.z - bdot(f.ec, x);
+      t = g.z - bdot(g.ec, x);
       xo = turn == 2u ? t : xo;
       x = pass_on<2>(t);
     }
     if (top >= 3) {
-      t = f.z - bdot(f.ec, x);
+      t = g.z - bdot(g.ec, x);
       xo = turn == 3u ? t : xo;
       x = pass_on<3>(t);
     }
-    if (el && top >= (int)turn) *at(lp, NX * (uint32_t)(top - (int)turn) + i) = ACCUMULATE ? f.l + xo : xo;
+    if (el && top >= (int)turn) *at(lp, NX * ch.knot((uint32_t)(top - (int)turn)) + i) = ACCUMULATE ? g.l + xo : xo;
   };
   Bwd g[3];
-  const int n = (int)p.N;
+  const int n = (int)ch.n;
 #pragma unroll
   for (int u = 0; u < 3; ++u) load_b(g[u], n - 1 - 4 * u);
   for (int top0 = n - 1; top0 >= 0; top0 -= 12) {
@@ -508,25 +568,26 @@ __device__ __forceinline__ void substitute(const float *__restrict__ gamma, floa
   }
 }
 
-// one wave per instance: the factorisation (FACTOR; else the factors a
-// previous launch left in work), then the substitution sweeps on
-// r = -gamma, or with ACCUMULATE on the z slots, added to lambda
-template <bool FACTOR, bool ACCUMULATE>
-__global__ void __launch_bounds__(64) k_direct_wave(Batch b, const uint32_t *__restrict__ order,
-                                                   const float *__restrict__ S, const float *__restrict__ gamma,
-                                                   const uint32_t *__restrict__ status, float *work,
-                                                   float *__restrict__ lambda, uint32_t *__restrict__ iters,
-                                                   uint32_t *__restrict__ flag) {
-  __shared__ FacWaveLds lds;
-  const uint32_t lane = threadIdx.x;
+// one workgroup per instance, a wave per side: the factorisation (FACTOR;
+// else the factors a previous launch left in work), then the substitution
+// sweeps on r = -gamma, or with ACCUMULATE on the z slots, added to lambda
+template <bool TWO, bool FACTOR, bool ACCUMULATE>
+__global__ void __launch_bounds__(TWO ? 128 : 64) k_direct_wave(Batch b, const uint32_t *__restrict__ order,
+                                                    const float *__restrict__ S, const float *__restrict__ gamma,
+                                                    const uint32_t *__restrict__ status, float *work,
+                                                    float *__restrict__ lambda, uint32_t *__restrict__ iters,
+                                                    uint32_t *__restrict__ flag) {
+  __shared__ DirectLds<TWO> lds;
+  const uint32_t lane = threadIdx.x & 63u;
   const Pick p = pick_instance(b, order, status, blockIdx.x);
   if (!p.live) return;
+  const Chain ch = chain_of<TWO>(p.N, TWO ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0u);
   if constexpr (FACTOR) {
-    factor_wave(lds, S, work, p, lane);
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the factor rows written above are read below
+    factor_wave<TWO>(lds, S, work, p, ch, lane);
+    __syncthreads();  // the factor rows written above are read below
   }
-  substitute<ACCUMULATE>(gamma, work, lambda, p, lane);
-  if (!ACCUMULATE && lane == 0) {
+  substitute<TWO, ACCUMULATE>(lds, gamma, work, lambda, p, ch, lane);
+  if (!ACCUMULATE && threadIdx.x == 0) {
     if (iters) iters[p.inst] = 0;
     if (flag) flag[p.inst] = 0;
   }
@@ -558,27 +619,46 @@ __global__ void __launch_bounds__(WG) k_schur_residual(Batch b, const float *__r
 
 }  // namespace
 
-hipError_t launch_direct_solve(const Batch &b, const uint32_t *order, uint32_t n_list, const float *S,
+template <bool TWO>
+static hipError_t direct_solve(const Batch &b, const uint32_t *order, uint32_t n_list, const float *S,
                                const float *gamma, const uint32_t *status, float *work, float *lambda,
                                uint32_t refine, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
-  if (n_list == 0) return hipSuccess;
+  const dim3 grid(n_list), block(TWO ? 128 : 64);
   if (do_factor)
-    hipLaunchKernelGGL((k_direct_wave<true, false>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
-                       lambda, iters, flag);
+    hipLaunchKernelGGL((k_direct_wave<TWO, true, false>), grid, block, 0, st, b, order, S, gamma, status, work, lambda,
+                       iters, flag);
   else
-    hipLaunchKernelGGL((k_direct_wave<false, false>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
+    hipLaunchKernelGGL((k_direct_wave<TWO, false, false>), grid, block, 0, st, b, order, S, gamma, status, work,
                        lambda, iters, flag);
   hipError_t e = hipGetLastError();
-  for (uint32_t s = 0; s < refine && e == hipSuccess; ++s) {
+  const uint32_t steps = TWO ? refine + 1u : refine;
+  for (uint32_t s = 0; s < steps && e == hipSuccess; ++s) {
     hipLaunchKernelGGL(k_schur_residual, dim3((b.total_knots + GROUPS_PER_WG - 1) / GROUPS_PER_WG), dim3(WG), 0, st,
                        b, S, gamma, (const float *)lambda, work);
     e = hipGetLastError();
     if (e != hipSuccess) break;
-    hipLaunchKernelGGL((k_direct_wave<false, true>), dim3(n_list), dim3(64), 0, st, b, order, S, gamma, status, work,
-                       lambda, (uint32_t *)nullptr, (uint32_t *)nullptr);
+    hipLaunchKernelGGL((k_direct_wave<TWO, false, true>), grid, block, 0, st, b, order, S, gamma, status, work, lambda,
+                       (uint32_t *)nullptr, (uint32_t *)nullptr);
     e = hipGetLastError();
   }
   return e;
+}
+
+// Both sides at once for refine >= 2.  The two orders of elimination round
+// differently, by up to the error of an unrefined solve (5e-4 relative at N =
+// 256) or of one refined once (2e-6): either may be the closer one.  Two steps
+// are at the rounding of lambda itself (3e-8) but for ill-conditioned systems
+// (1e-5), and with the one step more that the halved sweeps pay for, both
+// sides at once are the closer in every case.  With fewer steps asked, one
+// order, that of the knots, and its bits.  (A factorisation is used again with
+// the `refine` it was made with.)
+// N = 256, refine 2: 473 -> 310 us.
+hipError_t launch_direct_solve(const Batch &b, const uint32_t *order, uint32_t n_list, const float *S,
+                               const float *gamma, const uint32_t *status, float *work, float *lambda,
+                               uint32_t refine, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
+  if (n_list == 0) return hipSuccess;
+  return refine >= 2 ? direct_solve<true>(b, order, n_list, S, gamma, status, work, lambda, refine, do_factor, iters, flag, st)
+                     : direct_solve<false>(b, order, n_list, S, gamma, status, work, lambda, refine, do_factor, iters, flag, st);
 }
 
 }  // namespace mpc

@@ -1,19 +1,19 @@
 // k_schur.hip -- Schur complement, block-Jacobi preconditioner and dz
 // recovery for gfx950.
 //
-// Two kernels, one 16-lane group per knot / block row, lane j owning
-// column j of every 14x14 block (registers), 4 groups per 64-lane workgroup:
-//   k_invert_g:   G~^-1 of every knot (Q~_k^-1, R~_k^-1) into the G^-1 buffer;
-//   k_form_schur: per block row, the products, theta, its inverse and the
-//                 outputs, reading Q~^-1 / R~^-1 from G^-1.
+// k_form_schur, one 16-lane group per block row, lane j owning column j of
+// every 14x14 block (registers): the inverses G~^-1 of the knot's blocks (to
+// their buffer, and to the next group), the products, theta, its inverse and
+// the outputs.
 // Block inverses are Gauss-Jordan eliminations on [M | I]; the pivot column
 // is broadcast within the group by DPP, and so are the left factors of the
 // block products, inside the multiply-adds.  The regularised blocks are
 // symmetric positive definite, so no pivoting is needed.
-// k_form_schur moves 5.3 KB a knot, 1.22 M knots in 1.58 ms (4.1 TB/s; a copy
-// reaches 5.1): bound by memory.  With the factors read from LDS by every
-// lane, swizzled pivot columns and the reads of a row behind its instance
-// lookup it took 2.77 ms; 128 knots 14.6 us, 8.2 now.
+// It moves 6.3 KB a knot, 1.22 M knots in 1.96 ms (3.9 TB/s; a copy reaches
+// 5.1): bound by memory, and at few knots by the chain of two inverses (128
+// knots 11.3 us).  The inverses in a kernel of their own took 2.21 ms and 13.6
+// us together; with the factors read from LDS by every lane, swizzled pivot
+// columns and the reads of a row behind its instance lookup 3.41 ms and 20.
 //
 // Math (reference: oldschur.cuh:518-963, signs as there; C stores -A, -B):
 //   Q~_k = Q_k + rho I, R~_k = R_k + rho I
@@ -40,43 +40,6 @@ namespace {
 constexpr int GROUP = 16;
 constexpr int GROUPS_PER_WG = 4;
 constexpr int WG = GROUP * GROUPS_PER_WG;
-
-// G~_k^-1 = [ (Q_k + rho I)^-1 | (R_k + rho I)^-1 ] of every knot (the
-// last knot of an instance has no R block)
-__global__ void __launch_bounds__(WG) k_invert_g(Batch b, const float *__restrict__ G,
-                                                 const float *__restrict__ rho_dev, float rho_s,
-                                                 const uint32_t *__restrict__ status, float *__restrict__ Ginv) {
-  const int lane = threadIdx.x % GROUP;
-  const uint32_t gk_raw = blockIdx.x * GROUPS_PER_WG + threadIdx.x / GROUP;
-  bool valid = gk_raw < b.total_knots;
-  const uint32_t gk = valid ? gk_raw : b.total_knots - 1;
-  const KnotRef kr = locate(b, gk);
-  if (status && !(status[kr.inst] & ST_ACTIVE)) valid = false;
-  const float rho = rho_dev ? rho_dev[kr.inst] : rho_s;
-  const float *Gk = G + (size_t)G_STRIDE * gk;
-  float *Gi = Ginv + (size_t)G_STRIDE * gk;
-  float a[NX], x[NX];
-  {
-    const int j = lane < NX ? lane : NX - 1;
-#pragma unroll
-    for (int r = 0; r < NX; ++r) a[r] = Gk[r + NX * j] + ((r == j) ? rho : 0.f);
-    gj_inverse<NX>(lane, a, x);
-    if (valid && lane < NX) {
-#pragma unroll
-      for (int r = 0; r < NX; ++r) Gi[r + NX * lane] = x[r];
-    }
-  }
-  if (kr.k + 1 < kr.N) {  // uniform over the group
-    const int j = lane < NU ? lane : NU - 1;
-#pragma unroll
-    for (int r = 0; r < NU; ++r) a[r] = Gk[NXX + r + NU * j] + ((r == j) ? rho : 0.f);
-    gj_inverse<NU>(lane, a, x);
-    if (valid && lane < NU) {
-#pragma unroll
-      for (int r = 0; r < NU; ++r) Gi[NXX + r + NU * lane] = x[r];
-    }
-  }
-}
 
 // d[r] += s_l[r] * w (r < 14), s_l the s of lane l of the 16-lane group:
 // v_fmac_f32_dpp with DPP row_newbcast:l, so a block product whose left
@@ -124,15 +87,22 @@ __device__ __forceinline__ void nb_product(float (&d)[NX], const float (&s)[NX],
   ((nb_fma7<Ls, Nop4 && Ls == 0, 0>(d, s, w[Ls]), nb_fma7<Ls, false, 7>(d, s, w[Ls])), ...);
 }
 
+// Workgroups of SG groups overlap by one row: group g of workgroup w inverts
+// the blocks of knot (SG - 1) w + g - 1, and groups g >= 1 form that block row,
+// with the inverses of the knot before from group g - 1 through LDS.
+constexpr int SG = 16;
+constexpr int SWG = GROUP * SG;
+constexpr uint32_t SSTEP = SG - 1;
+
 // 16-byte aligned blocks: AQ and A (reused for the S(b,b) and Pinv(b,b)
 // blocks on their way out) are read as float4 rows for coalesced stores
 struct alignas(16) SchurLds {
-  float AQ[NXX];  // Q~_k^-1, then Q~_b^-1, then (not for a first knot) A Q~_k^-1
-  float A[NXX];   // A_k (column-major)
-  float B[98];    // B_k, then B R~_k^-1
-  float R[49];    // R~_k^-1
+  float AQ[NXX];  // Q_b, Q~_b^-1, then (not for a first knot) A Q~_{b-1}^-1
+  float A[NXX];   // A_{b-1} (column-major)
+  float R[52];    // R_b, then R~_b^-1
+  float B[98];    // B_{b-1}, then B R~_{b-1}^-1
   float qk[16], q1[16], rk[8], cb[16];
-};  // 2384 B: sixteen workgroups' fit one CU's LDS
+};  // 2400 B: four workgroups' fit one CU's LDS
 static_assert(NXX % 4 == 0 && sizeof(float) * NXX % 16 == 0, "float4 rows of a 14 x 14 block");
 
 // a 14 x 14 block (element i at src[f(i)]) from the group's LDS to global
@@ -148,101 +118,124 @@ __device__ __forceinline__ void store_block(int lane, float *dst, F &&f) {
   }
 }
 
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) k_form_schur(Batch b, const float *__restrict__ G,
+__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(4))) k_form_schur(Batch b, const float *__restrict__ G,
                                                    const float *__restrict__ C,
                                                    const float *__restrict__ g,
                                                    const float *__restrict__ cvec,
                                                    const float *__restrict__ rho_dev, float rho_s,
                                                    const uint32_t *__restrict__ status,
                                                    float *__restrict__ S, float *__restrict__ Pinv,
-                                                   float *__restrict__ gamma, const float *__restrict__ Ginv,
+                                                   float *__restrict__ gamma, float *__restrict__ Ginv,
                                                    int out_mode) {
   const bool zero_unused = out_mode & SCHUR_ZERO_UNUSED, right = out_mode & SCHUR_RIGHT_BLOCK;
-  __shared__ SchurLds lds[GROUPS_PER_WG];
+  __shared__ SchurLds lds[SG];
   const int grp = threadIdx.x / GROUP, lane = threadIdx.x % GROUP;
-  const uint32_t gk_raw = blockIdx.x * GROUPS_PER_WG + grp;
-  bool valid = gk_raw < b.total_knots;
-  const uint32_t gk = valid ? gk_raw : b.total_knots - 1;
+  const int64_t row_raw = (int64_t)blockIdx.x * SSTEP + grp - 1;
+  const bool in_range = row_raw >= 0 && row_raw < (int64_t)b.total_knots;
+  const uint32_t gk = in_range ? (uint32_t)row_raw : (row_raw < 0 ? 0u : b.total_knots - 1);
   SchurLds &L = lds[grp];
   // The block row's reads are issued before the instance lookup, all of them
   // together: the previous knot's (for an instance's first knot another's
   // last; what is formed from them is not stored there) and this knot's.
-  const size_t row = gk, kprev = gk > 0 ? gk - 1 : 0;  // block row b >= 1: k = b - 1
+  const size_t row = gk, kprev = gk > 0 ? gk - 1 : 0;
   const float *Ck = C + (size_t)C_STRIDE * kprev;
-  const float *Qi = Ginv + (size_t)G_STRIDE * kprev;  // Q~_k^-1, then R~_k^-1
-  const float *Q1i = Ginv + (size_t)G_STRIDE * row;   // Q~_b^-1
+  const float *Gb = G + (size_t)G_STRIDE * row;
   const int j = lane < NX ? lane : NX - 1, ju = lane < NU ? lane : NU - 1;
-  float acol[NX], arow[NX], bcol[NX], brow[NU], qi[NX], ri[NU], th[NX];
+  // element lane + 16 k of a block of n, past its end the last one (which
+  // then goes to its place again)
+  auto at = [&](int k, int n) { return lane + GROUP * k < n ? lane + GROUP * k : n - 1; };
+  constexpr int NA = (NXX + GROUP - 1) / GROUP, NB = (98 + GROUP - 1) / GROUP, NR = (49 + GROUP - 1) / GROUP;
+  float th[NX];
   float a1 = 0.f;  // (Q~_b^-1 q_b)_j
+  bool valid = grp > 0 && in_range, row0, last;
+  float rho;
   {
-    constexpr int NA = (NXX + GROUP - 1) / GROUP, NB = (98 + GROUP - 1) / GROUP, NR = (49 + GROUP - 1) / GROUP;
-    float va[NA], vb[NB], vq[NA], vr[NR], v1[NA];
-    // element lane + 16 k of a block of n, past its end the last one
-    auto at = [&](int k, int n) { return lane + GROUP * k < n ? lane + GROUP * k : n - 1; };
+    float vg[NA], vr[NR], va[NA], vb[NB];
+#pragma unroll
+    for (int k = 0; k < NA; ++k) vg[k] = Gb[at(k, NXX)];
+    // (the caller's G ends with the Q of the last knot)
+#pragma unroll
+    for (int k = 0; k < NR; ++k) vr[k] = gk + 1 < b.total_knots ? Gb[NXX + at(k, 49)] : 1.f;
 #pragma unroll
     for (int k = 0; k < NA; ++k) va[k] = Ck[at(k, NXX)];
 #pragma unroll
     for (int k = 0; k < NB; ++k) vb[k] = Ck[NXX + at(k, 98)];
-#pragma unroll
-    for (int k = 0; k < NA; ++k) vq[k] = Qi[at(k, NXX)];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) vr[k] = Qi[NXX + at(k, 49)];
-#pragma unroll
-    for (int k = 0; k < NA; ++k) v1[k] = Q1i[at(k, NXX)];
     const float vk = g[(size_t)NXU * kprev + j], vu = g[(size_t)NXU * kprev + NX + ju],
-                vg = g[(size_t)NXU * row + j], vc = cvec ? cvec[(size_t)NX * row + j] : 0.f;  // no c: c = 0
-    // (past the end the last element again, to its place)
+                v1 = g[(size_t)NXU * row + j], vc = cvec ? cvec[(size_t)NX * row + j] : 0.f;  // no c: c = 0
+    const KnotEnds ke = knot_ends(b, gk);
+    row0 = ke.first;
+    last = !ke.has_next;
+    valid = valid && !(status && !(status[ke.inst] & ST_ACTIVE));
+    rho = rho_dev ? rho_dev[ke.inst] : rho_s;
+#pragma unroll
+    for (int k = 0; k < NA; ++k) L.AQ[at(k, NXX)] = vg[k];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) L.R[at(k, 49)] = vr[k];
 #pragma unroll
     for (int k = 0; k < NA; ++k) L.A[at(k, NXX)] = -va[k];
 #pragma unroll
     for (int k = 0; k < NB; ++k) L.B[at(k, 98)] = -vb[k];
-#pragma unroll
-    for (int k = 0; k < NA; ++k) L.AQ[at(k, NXX)] = vq[k];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) L.R[at(k, 49)] = vr[k];
     L.qk[j] = vk;
     L.rk[ju] = vu;
-    L.q1[j] = vg;
+    L.q1[j] = v1;
     L.cb[j] = vc;
-    wave_sync();  // (a workgroup is one wave)
-    // columns j of A, Q~_k^-1, Q~_b^-1 and (j < 7) of B, R~_k^-1; rows j of A, B
-#pragma unroll
-    for (int l = 0; l < NX; ++l) {
-      acol[l] = L.A[l + NX * j];
-      arow[l] = L.A[j + NX * l];
-      bcol[l] = L.B[l + NX * ju];
-      qi[l] = L.AQ[l + NX * j];
-    }
-#pragma unroll
-    for (int l = 0; l < NU; ++l) {
-      brow[l] = L.B[j + NX * l];
-      ri[l] = L.R[l + NU * ju];
-    }
-    wave_sync();
-#pragma unroll
-    for (int k = 0; k < NA; ++k) L.AQ[at(k, NXX)] = v1[k];
-    wave_sync();
-#pragma unroll
-    for (int l = 0; l < NX; ++l) {
-      th[l] = L.AQ[l + NX * j];
-      a1 += L.AQ[j + NX * l] * L.q1[l];
-    }
-    wave_sync();
+    wave_sync();  // (a group is inside one wave)
   }
-  const KnotRef kr = locate(b, gk);
-  if (status && !(status[kr.inst] & ST_ACTIVE)) valid = false;
-  const float rho = rho_dev ? rho_dev[kr.inst] : rho_s;
-  const uint32_t bk = kr.k;
-  float *Srow = S + (size_t)S_STRIDE * row;
-  float *Prow = Pinv + (size_t)S_STRIDE * row;
-  const bool row0 = bk == 0;
-  // AQ = A Q~_k^-1 (column j), BR = B R~_k^-1 (column j < 7): the left
+  // Q~_b^-1, R~_b^-1: by columns, to LDS, and to G^-1 (the last knot of an
+  // instance has no R block)
+  {
+    float a[NX], x[NX];
+#pragma unroll
+    for (int r = 0; r < NX; ++r) a[r] = L.AQ[r + NX * j] + ((r == j) ? rho : 0.f);
+    gj_inverse<NX>(lane, a, th);
+#pragma unroll
+    for (int r = 0; r < NU; ++r) a[r] = L.R[r + NU * ju] + ((r == ju) ? rho : 0.f);
+    gj_inverse<NU>(lane, a, x);
+    wave_sync();
+#pragma unroll
+    for (int r = 0; r < NX; ++r) L.AQ[r + NX * j] = th[r];
+#pragma unroll
+    for (int r = 0; r < NU; ++r) L.R[r + NU * ju] = x[r];
+  }
+  __syncthreads();  // the inverses to the next group
+  if (valid) {
+    float *Gi = Ginv + (size_t)G_STRIDE * row;
+    for (int i = lane; i < NXX; i += GROUP) Gi[i] = L.AQ[i];
+    if (!last)
+      for (int i = lane; i < 49; i += GROUP) Gi[NXX + i] = L.R[i];
+  }
+  // AQ = A Q~_{b-1}^-1 (column j), BR = B R~_{b-1}^-1 (column j < 7): the left
   // factor's columns from their lanes by DPP
-  float acc[NX], bacc[NX];
+  const SchurLds &Lp = lds[grp > 0 ? grp - 1 : 0];
+  float acc[NX], bacc[NX], arow[NX], brow[NU];
 #pragma unroll
   for (int r = 0; r < NX; ++r) acc[r] = bacc[r] = 0.f;
-  nb_product<true>(acc, acol, qi, std::make_integer_sequence<int, NX>{});
-  nb_product<true>(bacc, bcol, ri, std::make_integer_sequence<int, NU>{});
+  {
+    float col[NX], w[NX];
+#pragma unroll
+    for (int l = 0; l < NX; ++l) {
+      col[l] = L.A[l + NX * j];
+      w[l] = Lp.AQ[l + NX * j];
+      a1 += L.AQ[j + NX * l] * L.q1[l];
+    }
+    nb_product<true>(acc, col, w, std::make_integer_sequence<int, NX>{});
+  }
+  {
+    float col[NX], w[NU];
+#pragma unroll
+    for (int l = 0; l < NX; ++l) col[l] = L.B[l + NX * ju];
+#pragma unroll
+    for (int l = 0; l < NU; ++l) w[l] = Lp.R[l + NU * ju];
+    nb_product<true>(bacc, col, w, std::make_integer_sequence<int, NU>{});
+  }
+  // rows j of A and of B (the right factors of theta, transposed)
+#pragma unroll
+  for (int l = 0; l < NX; ++l) arow[l] = L.A[j + NX * l];
+#pragma unroll
+  for (int l = 0; l < NU; ++l) brow[l] = L.B[j + NX * l];
+  float *Srow = S + (size_t)S_STRIDE * row;
+  float *Prow = Pinv + (size_t)S_STRIDE * row;
+  __syncthreads();  // the inverses read by the next group
   if (!row0) {  // the same for the whole group
 #pragma unroll
     for (int r = 0; r < NX; ++r) L.AQ[r + NX * j] = acc[r];
@@ -287,7 +280,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) k_
       gamma[(size_t)NX * row + lane] = L.cb[lane] - (a1 - a2 - a3);
     }
     if (zero_unused) {
-      if (bk + 1 == kr.N && right)
+      if (last && right)
         for (int i = lane; i < NXX; i += GROUP) Srow[2 * NXX + i] = 0.f;
       for (int i = lane; i < NXX; i += GROUP) {
         Prow[i] = 0.f;
@@ -328,9 +321,6 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) k_
 // through LDS and write their row (each row from exactly one group).  That
 // hand-over is the one workgroup barrier; every other LDS exchange stays
 // inside a group, so inside one wave (wave_sync).
-constexpr int SG = 16;
-constexpr int SWG = GROUP * SG;
-constexpr uint32_t SSTEP = SG - 1;
 
 struct alignas(16) SplitRowLds {
   float AQ[NXX];   // A Q~_{b-1}^-1 = S(b, b-1)
@@ -680,12 +670,8 @@ hipError_t launch_form_schur(const Batch &b, const float *G, const float *C, con
                              float *S, float *Pinv, float *gamma, float *Ginv, int out_mode,
                              hipStream_t st) {
   if (b.total_knots == 0) return hipSuccess;
-  const dim3 grid((b.total_knots + GROUPS_PER_WG - 1) / GROUPS_PER_WG);
-  hipLaunchKernelGGL(k_invert_g, grid, dim3(WG), 0, st, b, G, rho_dev, rho, status, Ginv);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_form_schur, grid, dim3(WG), 0, st, b, G, C, g, c, rho_dev, rho, status, S, Pinv, gamma,
-                     (const float *)Ginv, out_mode);
+  hipLaunchKernelGGL(k_form_schur, dim3((b.total_knots + SSTEP - 1) / SSTEP), dim3(SWG), 0, st, b, G, C, g, c, rho_dev,
+                     rho, status, S, Pinv, gamma, Ginv, out_mode);
   return hipGetLastError();
 }
 

@@ -274,6 +274,20 @@ __device__ __forceinline__ void rnea_dir(int dir, const float *s, const float *c
                                          const float *bxa, float *dtau) {
   const int jq = dir < NQ ? dir : -1;
   const int jd = dir >= NQ ? dir - NQ : -1;
+  // X v, X a or (for a velocity) v, and f of the direction's own link, read
+  // ahead (two components are not used by S x .): in the branch that uses
+  // them each wave waited for the reads of every link.  The terms stay in
+  // branches: as selects the sums round otherwise.
+  const int jl = dir < NQ ? dir : dir - NQ;
+  const float *own = dir < NQ ? bxa : bv;
+  float xv[6] = {}, xo[6] = {}, fi[6] = {};
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    if (k == 2) continue;
+    xv[k] = bxv[6 * jl + k];
+    xo[k] = own[6 * jl + k];
+    fi[k] = bf[6 * jl + k];
+  }
   float df[NQ][6];
   float dvp[6] = {0, 0, 0, 0, 0, 0}, dap[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -282,10 +296,11 @@ __device__ __forceinline__ void rnea_dir(int dir, const float *s, const float *c
     X_mv(i, s[i], c[i], dvp, dv);
     X_mv(i, s[i], c[i], dap, da);
     if (i == jq) {
-      crm_z(bxv + 6 * i, t);
+      asm volatile("");  // a branch: no select
+      crm_z(xv, t);
 #pragma unroll
       for (int k = 0; k < 6; ++k) dv[k] -= t[k];
-      crm_z(bxa + 6 * i, t);
+      crm_z(xo, t);
 #pragma unroll
       for (int k = 0; k < 6; ++k) da[k] -= t[k];
     }
@@ -295,8 +310,9 @@ __device__ __forceinline__ void rnea_dir(int dir, const float *s, const float *c
 #pragma unroll
     for (int k = 0; k < 6; ++k) da[k] += t[k];
     if (i == jd) {
+      asm volatile("");  // a branch: no select
       // v_i x S  = -(S x v_i)
-      crm_z(bv + 6 * i, t);
+      crm_z(xo, t);
 #pragma unroll
       for (int k = 0; k < 6; ++k) da[k] -= t[k];
     }
@@ -326,7 +342,7 @@ __device__ __forceinline__ void rnea_dir(int dir, const float *s, const float *c
       for (int k = 0; k < 6; ++k) df[i - 1][k] += t[k];
       if (i == jq) {
         // (dX_i/dq_i)^T f_i = X_i^T (S x* f_i)
-        const float *fi = bf + 6 * i;
+        asm volatile("");  // a branch: no select
         const float sf[6] = {-fi[1], fi[0], 0.f, -fi[4], fi[3], 0.f};
         XT_fv(i, s[i], c[i], sf, t);
 #pragma unroll

@@ -158,8 +158,6 @@ static uint32_t sqp_pcg_cap(const mpc_config &c) {
   return (c.flags & FLAG_PCG_CAP_BY_N) ? PCG_CAP_BY_N : c.pcg_max_iter;
 }
 
-
-
 // PCG of one instance: the one-workgroup kernel for a lone instance (stair:
 // the resident kernel) when its Schur system fits one workgroup, a team of
 // two or four up to four times that, streaming otherwise.
@@ -764,9 +762,9 @@ static int build_pcg_plan(mpc_handle *h) {
     // with one, 215 with four, 327 with eight).  So while the bins fit the
     // device at once they are kept as empty as that allows: 4, 8 or 16 groups
     // instead of 32 per bin (instances of more groups have their own).
-    // Every packing is the same solve, bitwise.  256 instances of N = 64 (256
-    // bins instead of 64): layer and adjoint 5.9 -> 4.3 ms; 16 of N = 5..97:
-    // two SQP iterations 765 -> 533 us.
+    // Every packing is the same solve, bitwise.  256 instances of N = 64 in 256
+    // bins instead of 64 (they take the kernel above now): layer and adjoint
+    // 5.9 -> 4.3 ms; 16 of N = 5..97: two SQP iterations 765 -> 533 us.
     std::vector<BinB> sb;
     for (uint32_t cap = 4; cap <= pcg_split_bin_groups(); cap *= 2) {
       double fill = 0.0;  // a lower bound on the bins, before packing them

@@ -198,7 +198,8 @@ int mpc_pcg_solve(mpc_handle *h, uint32_t N, const float *d_S, const float *d_Pi
 
 /* Direct solve of S lambda = gamma (one instance of N knots) by block LDL^T
  * of -S on the GPU, then refine_steps (<= 16) steps of iterative refinement
- * with an fp64 residual; d_work: 588 N floats of scratch (the layout of S:
+ * with an fp64 residual (asked for two or more, it eliminates from both ends
+ * and takes one step more); d_work: 588 N floats of scratch (the layout of S:
  * the elimination factors and a vector per block row).  GPU counterpart of
  * the reference's QDLDL solve (qdldl_helper.cuh:62-180, toplevel.cuh:314-335);
  * the SQP drivers use 2 refinement steps. */
@@ -354,7 +355,7 @@ int mpc_batch_pcg_exit(mpc_handle *h, uint32_t *d_iters, uint32_t *d_flags, floa
 
 /* The Schur systems of the last batched SQP iteration (the workspace's S
  * and gamma) solved directly, block LDL^T of -S with refine_steps (<= 16)
- * steps of fp64-residual refinement, into d_lambda_out (14 per knot, the
+ * steps of fp64-residual refinement as in mpc_direct_solve, into d_lambda_out (14 per knot, the
  * batch's lambda layout): the accuracy reference for the PCG multipliers
  * that solve returned (the reference's QDLDL solve of the same system,
  * toplevel.cuh:314-335).  After a split-form solve (mpc_pcg_plan.split),

@@ -276,8 +276,9 @@ __device__ __forceinline__ void rnea_dir(int dir, const float *s, const float *c
   const int jd = dir >= NQ ? dir - NQ : -1;
   // X v, X a or (for a velocity) v, and f of the direction's own link, read
   // ahead (two components are not used by S x .): in the branch that uses
-  // them each wave waited for the reads of every link.  The terms stay in
-  // branches: as selects the sums round otherwise.
+  // them each wave waited for the reads of every link (k_form_kkt, bound by
+  // this chain: 127 k knots 143 -> 134 us, 32 knots 18.5 -> 17.4).  The terms
+  // stay in branches: as selects the sums round otherwise.
   const int jl = dir < NQ ? dir : dir - NQ;
   const float *own = dir < NQ ? bxa : bv;
   float xv[6] = {}, xo[6] = {}, fi[6] = {};

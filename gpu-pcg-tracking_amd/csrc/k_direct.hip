@@ -122,19 +122,35 @@ __device__ __forceinline__ bool mid_range(float v) {
 #define MPC_NB " row_newbcast:%c[l] row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
 // One slot of a pivot step: x -= column * xp, a -= column * ap, the column's
 // element by DPP from lane l of the row; then the next pivot from lane pl of
-// a.  A DPP read needs two wait states after the write of what it reads: a was
-// written in the step before, at least the two products ap and xp ago.
-template <int l, int pl>
+// a.  A DPP read needs two wait states after the write of what it reads.  From
+// step 1 on they are there: a was written in the step before, at least the two
+// products ap and xp ago.  In step 0 the compiler's copies and negations of
+// the block may stand right before the asm (it does not see the read inside),
+// so it begins with an s_nop, as does pivot_rest's.  Reading the pivot takes two
+// wait states after the v_readlane: pivot_rest has three instructions ahead of
+// it, but DIV divides by it at once.  (tests/test_wait_states.py checks the
+// listing.)
+#define MPC_PIVOT_FIRST(before, behind)           \
+  asm(before                                      \
+      "v_fmac_f32_dpp %[x], %[a], -%[xp]" MPC_NB  \
+      "v_fmac_f32_dpp %[a], %[a], -%[ap]" MPC_NB  \
+      "s_nop 0\n"                                 \
+      "v_readlane_b32 %[p], %[a], %[pl]\n"        \
+      behind                                      \
+      : [x] "+v"(x), [a] "+v"(a), [p] "=s"(piv)   \
+      : [xp] "v"(xp), [ap] "v"(ap), [l] "i"(l), [pl] "i"(pl))
+template <bool DIV, int l, int pl>
 __device__ __forceinline__ float pivot_first(float &x, float &a, float xp, float ap) {
   float piv;
-  asm("v_fmac_f32_dpp %[x], %[a], -%[xp]" MPC_NB
-      "v_fmac_f32_dpp %[a], %[a], -%[ap]" MPC_NB
-      "s_nop 0\n"
-      "v_readlane_b32 %[p], %[a], %[pl]\n"
-      : [x] "+v"(x), [a] "+v"(a), [p] "=s"(piv)
-      : [xp] "v"(xp), [ap] "v"(ap), [l] "i"(l), [pl] "i"(pl));
+  if constexpr (DIV)
+    MPC_PIVOT_FIRST("s_nop 1\n", "s_nop 1\n");
+  else if constexpr (l == 0)
+    MPC_PIVOT_FIRST("s_nop 1\n", "");
+  else
+    MPC_PIVOT_FIRST("", "");
   return piv;
 }
+#undef MPC_PIVOT_FIRST
 
 // The other three slots of the step, with the next pivot's inverse between
 // them: v_rcp_f32, one refinement and two residual steps, which is the
@@ -156,22 +172,30 @@ __device__ __forceinline__ float pivot_first(float &x, float &a, float xp, float
   "v_fma_f32 %[i], %[t], %[r], %[r]\n"          \
   "v_fma_f32 %[t], -%[p], %[i], 1.0\n"          \
   "v_fma_f32 %[i], %[t], %[r], %[i]\n"
+#define MPC_PIVOT_REST_OTHER(before)                                                                                \
+  asm(before MPC_PIVOT_REST                                                                                         \
+      "v_cndmask_b32_e64 %[ac], %[ac], %[ap], %[m]\n"                                                               \
+      "v_cndmask_b32_e64 %[xc], %[xc], %[xp], %[m]\n"                                                               \
+      : [x0] "+v"(x0), [a0] "+v"(a0), [x1] "+v"(x1), [a1] "+v"(a1), [x2] "+v"(x2), [a2] "+v"(a2), [xc] "+v"(xc),     \
+        [ac] "+v"(ac), [i] "=&v"(inv), [r] "=&v"(r), [t] "=&v"(t)                                                   \
+      : [xp] "v"(xp), [ap] "v"(ap), [p] "s"(piv), [m] "s"(mask), [l] "i"(l))
 template <int l>
 __device__ __forceinline__ float pivot_rest(float &x0, float &a0, float &x1, float &a1, float &x2, float &a2, float xp,
                                             float ap, float piv, float &xc, float &ac, uint64_t mask) {
   float inv, r, t;
-  asm(MPC_PIVOT_REST
-      "v_cndmask_b32_e64 %[ac], %[ac], %[ap], %[m]\n"
-      "v_cndmask_b32_e64 %[xc], %[xc], %[xp], %[m]\n"
-      : [x0] "+v"(x0), [a0] "+v"(a0), [x1] "+v"(x1), [a1] "+v"(a1), [x2] "+v"(x2), [a2] "+v"(a2), [xc] "+v"(xc),
-        [ac] "+v"(ac), [i] "=&v"(inv), [r] "=&v"(r), [t] "=&v"(t)
-      : [xp] "v"(xp), [ap] "v"(ap), [p] "s"(piv), [m] "s"(mask), [l] "i"(l));
+  if constexpr (l == 0)
+    MPC_PIVOT_REST_OTHER("s_nop 1\n");
+  else
+    MPC_PIVOT_REST_OTHER("");
   return inv;
 }
-// row P in the first of the three slots
+#undef MPC_PIVOT_REST_OTHER
+// row P in the first of the three slots (not in step 0, whose row 0 and row 1
+// are in one slot)
 template <int l>
 __device__ __forceinline__ float pivot_rest(float &x0, float &a0, float &x1, float &a1, float &x2, float &a2, float xp,
                                             float ap, float piv, uint64_t mask) {
+  static_assert(l > 0, "no wait states ahead of the first DPP read");
   float inv, r, t;
   asm(MPC_PIVOT_REST
       "v_cndmask_b32_e64 %[a0], %[a0], %[ap], %[m]\n"
@@ -237,7 +261,7 @@ __device__ __forceinline__ void gj_wave_steps(const Quarters &qs, float (&a)[4],
   const float ap = rowa * inv, xp = rowx * inv;
   if constexpr (P + 1 < NX) {
     constexpr int Q1 = (P + 1) & 3, T1 = (P + 1) >> 2;  // and of row P + 1
-    const float next = pivot_first<P, 16 * Q1 + P + 1>(x[T1], a[T1], xp, ap);
+    const float next = pivot_first<DIV, P, 16 * Q1 + P + 1>(x[T1], a[T1], xp, ap);
     const float ra = lane_value(a[T1], qs.from[Q1]), rx = lane_value(x[T1], qs.from[Q1]);
     float ni;
     if constexpr (T1 == TP) {

@@ -243,7 +243,8 @@ __device__ __forceinline__ void rot_mtv2(const float (&M0)[16], float x0, const 
 
 // Three to five interleaved accumulations a_k += sum_{n=1..15} M_k[n] * ror_n(x_k),
 // three terms per asm statement; an s_nop ahead of the first (the two wait
-// states between a VALU write of x_k and its DPP read)
+// states between a VALU write of x_k and its DPP read; that no copy of x_k lands
+// right ahead of a later one is checked by tests/test_wait_states.py)
 #define MPC_TERM(n, acc, x, m) \
   "v_fmac_f32_dpp %" #acc ", %" #x ", %" #m " row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
 #define MPC_T4(n, m0, m1, m2, m3) MPC_TERM(n, 0, 4, m0) MPC_TERM(n, 1, 5, m1) MPC_TERM(n, 2, 6, m2) MPC_TERM(n, 3, 7, m3)

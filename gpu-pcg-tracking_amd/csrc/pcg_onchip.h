@@ -137,7 +137,9 @@ struct Rows {
 // even and an odd sum, m_0 + ror_2(m_2) of the even one a multiply-add; all
 // four taken together step by step.  A pair of steps n, n + 1 (n odd): the products
 // of the contributions come first, so that each DPP read is at least two
-// instructions behind the write of what it reads.
+// instructions behind the write of what it reads.  (Of x and xl only the first
+// statement makes sure itself; a copy of them that the compiler put right ahead
+// of a later one would be found by tests/test_wait_states.py.)
 #define MPC_DPPM " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
 #define MPC_PAIR(n, n1)                                                                                       \
   asm("v_mul_f32 %4, %13, %8\n"                                                                               \

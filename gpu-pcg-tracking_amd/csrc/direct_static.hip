@@ -56,8 +56,9 @@ extern "C" int mpc_direct_solve_static(uint32_t N, const float *d_S, const float
   float *work = scratch_on_current_device();
   if (!work) return MPC_ERR_HIP;
   const mpc::Batch b{nullptr, nullptr, 1u, N};
-  if (mpc::launch_direct_solve(b, nullptr, 1, d_S, d_gamma, nullptr, work, d_lambda, refine_steps, true, nullptr,
-                               nullptr, (hipStream_t)stream) != hipSuccess)
+  if (mpc::launch_direct_solve(b, nullptr, 1, d_S, d_gamma, nullptr, work, d_lambda, refine_steps,
+                               mpc::direct_both_ends(1, N, N, refine_steps), true, nullptr, nullptr,
+                               (hipStream_t)stream) != hipSuccess)
     return MPC_ERR_HIP;
   return MPC_OK;
 }

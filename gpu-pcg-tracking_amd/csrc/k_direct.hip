@@ -17,10 +17,9 @@
 // (1e-4..1e-2 relative on these systems); each step multiplies the error by
 // about that factor, down to the fp32 storage of lambda.
 //
-// Mapping: one wave per instance, or with two and more refinement steps two, one
-// from each end, which meet in the middle knot (a block tridiagonal system
-// eliminates from both ends with the same operations, so the chain is half as
-// long); instances longest first (few waves, one per SIMD: the sweeps are
+// Mapping: one wave per instance, or (direct_both_ends) two, one from each end,
+// which meet in the middle knot (a block tridiagonal system eliminates from both
+// ends with the same operations, so the chain is half as long); instances longest first (few waves, one per SIMD: the sweeps are
 // bound by their dependent chains, so what counts is the instructions and
 // latencies of a step, below).  The residual is formed for
 // all knots of all instances at once, one group per knot.
@@ -646,7 +645,7 @@ __global__ void __launch_bounds__(WG) k_schur_residual(Batch b, const float *__r
 template <bool TWO>
 static hipError_t direct_solve(const Batch &b, const uint32_t *order, uint32_t n_list, const float *S,
                                const float *gamma, const uint32_t *status, float *work, float *lambda,
-                               uint32_t refine, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
+                               uint32_t steps, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
   const dim3 grid(n_list), block(TWO ? 128 : 64);
   if (do_factor)
     hipLaunchKernelGGL((k_direct_wave<TWO, true, false>), grid, block, 0, st, b, order, S, gamma, status, work, lambda,
@@ -655,7 +654,6 @@ static hipError_t direct_solve(const Batch &b, const uint32_t *order, uint32_t n
     hipLaunchKernelGGL((k_direct_wave<TWO, false, false>), grid, block, 0, st, b, order, S, gamma, status, work,
                        lambda, iters, flag);
   hipError_t e = hipGetLastError();
-  const uint32_t steps = TWO ? refine + 1u : refine;
   for (uint32_t s = 0; s < steps && e == hipSuccess; ++s) {
     hipLaunchKernelGGL(k_schur_residual, dim3((b.total_knots + GROUPS_PER_WG - 1) / GROUPS_PER_WG), dim3(WG), 0, st,
                        b, S, gamma, (const float *)lambda, work);
@@ -668,21 +666,36 @@ static hipError_t direct_solve(const Batch &b, const uint32_t *order, uint32_t n
   return e;
 }
 
-// Both sides at once for refine >= 2.  The two orders of elimination round
-// differently, by up to the error of an unrefined solve (5e-4 relative at N =
-// 256) or of one refined once (2e-6): either may be the closer one.  Two steps
-// are at the rounding of lambda itself (3e-8) but for ill-conditioned systems
-// (1e-5), and with the one step more that the halved sweeps pay for, both
-// sides at once are the closer in every case.  With fewer steps asked, one
-// order, that of the knots, and its bits.  (A factorisation is used again with
-// the `refine` it was made with.)
-// N = 256, refine 2: 473 -> 310 us.
+// Both ends at once take one refinement step more than asked.  The two orders
+// of elimination round differently, by up to the error of an unrefined solve
+// (5e-4 relative at N = 256) or of one refined twice (1e-6; 3e-8, the rounding
+// of lambda itself, on well-conditioned systems): after the same number of
+// steps either may be the closer one (over 324 systems, N = 2 .. 512, R =
+// 1e-2 .. 1e-6, rho 1e-3 and 1, two steps: by up to 20 and 14 times).  With the
+// step more that the halved chains pay for, both ends at once were at least as
+// close on every one.  So the caller must have asked for two steps; with fewer
+// it is one order, that of the knots, and its bits.
+// It pays while the longest chain lasts longer than the work of all knots spread
+// over half the device's SIMDs (for equal horizons: two instances per compute
+// unit, a SIMD for each of their waves).  Two refinement steps from one end /
+// from both, us: N = 64, 1 instance 139 / 101, 256 158 / 129, 512 185 / 181, past the
+// line 1024 272 / 286, 4096 878 / 1116; N = 256, 1 490 / 322, 256 564 / 420, 512 714 /
+// 710, 1024 1145 / 1261, 2048 2022 / 2461; N = 16, 51 / 48, 54 / 53, 62 / 66, 90 / 92, 4096
+// 216 / 271; N = 32 .. 512 mixed, 512 instances 1149 / 879, 1024 1349 / 1250, past
+// the line (from 1187 on) 1280 1456 / 1450, 2048 1850 / 2122.
+bool direct_both_ends(uint32_t n_cu, uint32_t total_knots, uint32_t longest, uint32_t refine) {
+  return refine >= 2 && total_knots <= 2ull * n_cu * longest;
+}
+
 hipError_t launch_direct_solve(const Batch &b, const uint32_t *order, uint32_t n_list, const float *S,
                                const float *gamma, const uint32_t *status, float *work, float *lambda,
-                               uint32_t refine, bool do_factor, uint32_t *iters, uint32_t *flag, hipStream_t st) {
+                               uint32_t refine, bool both_ends, bool do_factor, uint32_t *iters, uint32_t *flag,
+                               hipStream_t st) {
   if (n_list == 0) return hipSuccess;
-  return refine >= 2 ? direct_solve<true>(b, order, n_list, S, gamma, status, work, lambda, refine, do_factor, iters, flag, st)
-                     : direct_solve<false>(b, order, n_list, S, gamma, status, work, lambda, refine, do_factor, iters, flag, st);
+  return both_ends ? direct_solve<true>(b, order, n_list, S, gamma, status, work, lambda, refine + 1u, do_factor,
+                                        iters, flag, st)
+                   : direct_solve<false>(b, order, n_list, S, gamma, status, work, lambda, refine, do_factor, iters,
+                                         flag, st);
 }
 
 }  // namespace mpc

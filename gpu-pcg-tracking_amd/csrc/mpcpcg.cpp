@@ -158,6 +158,15 @@ static uint32_t sqp_pcg_cap(const mpc_config &c) {
   return (c.flags & FLAG_PCG_CAP_BY_N) ? PCG_CAP_BY_N : c.pcg_max_iter;
 }
 
+// whether direct solves of one instance, or of the batch, eliminate from both
+// ends (the factors that a solve leaves and one on them reads must agree in it)
+static bool one_both_ends(const mpc_handle *h, uint32_t N, uint32_t refine) {
+  return direct_both_ends(h->n_cu, N, N, refine);
+}
+static bool batch_both_ends(const mpc_handle *h, uint32_t refine) {
+  return direct_both_ends(h->n_cu, h->total, h->max_n, refine);
+}
+
 // PCG of one instance: the one-workgroup kernel for a lone instance (stair:
 // the resident kernel) when its Schur system fits one workgroup, a team of
 // two or four up to four times that, streaming otherwise.
@@ -167,7 +176,7 @@ static hipError_t pcg_single(mpc_handle *h, uint32_t N, const float *S, const fl
   const uint32_t flags = h->cfg.flags;
   if (flags & FLAG_DIRECT_SOLVE)
     return launch_direct_solve(single(N), nullptr, 1, S, gamma, nullptr, const_cast<float *>(P), lambda,
-                               h->cfg.direct_refine, true, iters, flag, st);
+                               h->cfg.direct_refine, one_both_ends(h, N, h->cfg.direct_refine), true, iters, flag, st);
   const bool stair = flags & FLAG_PCG_STAIR;
   if (!(flags & FLAG_PCG_STREAM)) {
     if (N <= pcg_lone_max_knots() && !stair)
@@ -228,7 +237,9 @@ static hipError_t refine_kkt(mpc_handle *h, const float *d_rho, const float *g, 
                          [&](float *l, float tol) {
                            if (h->cfg.flags & FLAG_DIRECT_SOLVE)
                              return launch_direct_solve(batch_of(h), h->dir_order, h->n_inst, h->S, h->gamma, nullptr,
-                                                        h->P, l, h->cfg.direct_refine, false, nullptr, nullptr, st);
+                                                        h->P, l, h->cfg.direct_refine,
+                                                        batch_both_ends(h, h->cfg.direct_refine), false, nullptr,
+                                                        nullptr, st);
                            return pcg_batch(h, l, nullptr, h->cfg.pcg_max_iter, tol, nullptr, st);
                          },
                          st);
@@ -524,8 +535,8 @@ int mpc_pcg_solve(mpc_handle *h, uint32_t N, const float *d_S, const float *d_Pi
 int mpc_direct_solve(mpc_handle *h, uint32_t N, const float *d_S, const float *d_gamma, float *d_lambda,
                      uint32_t refine_steps, float *d_work, mpc_stream_t stream) {
   if (!h || !n_ok(h, N) || !d_S || !d_gamma || !d_lambda || !d_work || refine_steps > 16) return MPC_ERR_ARG;
-  HIP_TRY(launch_direct_solve(single(N), nullptr, 1, d_S, d_gamma, nullptr, d_work, d_lambda, refine_steps, true,
-                              nullptr, nullptr, (hipStream_t)stream));
+  HIP_TRY(launch_direct_solve(single(N), nullptr, 1, d_S, d_gamma, nullptr, d_work, d_lambda, refine_steps,
+                              one_both_ends(h, N, refine_steps), true, nullptr, nullptr, (hipStream_t)stream));
   return MPC_OK;
 }
 
@@ -630,7 +641,9 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
       HIP_TRY(refine_kkt_with(h, b, N, h->rho_one, h->g, h->c, h->dz, d_lambda, h->cfg.direct_kkt_refine, 0.f,
                               [&](float *l, float) {
                                 return launch_direct_solve(b, nullptr, 1, h->S, h->gamma, nullptr, h->P, l,
-                                                           h->cfg.direct_refine, false, nullptr, nullptr, st);
+                                                           h->cfg.direct_refine,
+                                                           one_both_ends(h, N, h->cfg.direct_refine), false, nullptr,
+                                                           nullptr, st);
                               },
                               st));
     }
@@ -1098,7 +1111,8 @@ int mpc_batch_direct_resolve(mpc_handle *h, float *d_lambda_out, uint32_t refine
     HIP_TRY(launch_form_schur(batch_of(h), h->G, h->C, h->g, h->c, h->rho_used, 0.f, nullptr, h->S, h->P, h->gamma,
                               h->Ginv, 0, (hipStream_t)stream));
   HIP_TRY(launch_direct_solve(batch_of(h), h->dir_order, h->n_inst, h->S, h->gamma, nullptr, h->P, d_lambda_out,
-                              refine_steps, true, nullptr, nullptr, (hipStream_t)stream));
+                              refine_steps, batch_both_ends(h, refine_steps), true, nullptr, nullptr,
+                              (hipStream_t)stream));
   return MPC_OK;
 }
 
@@ -1133,7 +1147,7 @@ static hipError_t pcg_batch(mpc_handle *h, float *d_lambda, const uint32_t *d_st
   }
   if (h->cfg.flags & FLAG_DIRECT_SOLVE) {
     e = launch_direct_solve(b, h->dir_order, h->n_inst, h->S, h->gamma, d_status, h->P, d_lambda, h->cfg.direct_refine,
-                            true, h->pcg_iters, h->pcg_flag, st);
+                            batch_both_ends(h, h->cfg.direct_refine), true, h->pcg_iters, h->pcg_flag, st);
     if (e == hipSuccess && mid) e = hipEventRecord(mid, st);
     return e;
   }

@@ -202,7 +202,7 @@ int mpc_pcg_solve(mpc_handle *h, uint32_t N, const float *d_S, const float *d_Pi
  * and takes one step more); d_work: 588 N floats of scratch (the layout of S:
  * the elimination factors and a vector per block row).  GPU counterpart of
  * the reference's QDLDL solve (qdldl_helper.cuh:62-180, toplevel.cuh:314-335);
- * the SQP drivers use 2 refinement steps. */
+ * the SQP drivers take mpc_config's direct_refine steps (default 0). */
 int mpc_direct_solve(mpc_handle *h, uint32_t N, const float *d_S, const float *d_gamma, float *d_lambda,
                      uint32_t refine_steps, float *d_work, mpc_stream_t stream);
 
@@ -355,8 +355,9 @@ int mpc_batch_pcg_exit(mpc_handle *h, uint32_t *d_iters, uint32_t *d_flags, floa
 
 /* The Schur systems of the last batched SQP iteration (the workspace's S
  * and gamma) solved directly, block LDL^T of -S with refine_steps (<= 16)
- * steps of fp64-residual refinement as in mpc_direct_solve, into d_lambda_out (14 per knot, the
- * batch's lambda layout): the accuracy reference for the PCG multipliers
+ * steps of fp64-residual refinement as in mpc_direct_solve (a batch of more
+ * knots than the longest horizon times twice the device's compute units from
+ * one end always, with the steps asked for), into d_lambda_out (14 per knot, the batch's lambda layout): the accuracy reference for the PCG multipliers
  * that solve returned (the reference's QDLDL solve of the same system,
  * toplevel.cuh:314-335).  After a split-form solve (mpc_pcg_plan.split),
  * which forms no S, S and gamma are first formed from the last iteration's

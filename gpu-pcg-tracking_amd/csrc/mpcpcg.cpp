@@ -60,7 +60,7 @@ struct mpc_handle {
   uint4 *split_items = nullptr;
   uint32_t *split_off = nullptr;
   uint32_t n_split_bins = 0;
-  bool split_short = false;  // launch_pcg_split_short instead of the bins
+  bool split_short = false;  // launch_pcg_split_short instead: a bin per instance
   bool split_ok = false;  // every horizon of the layout fits the split-form kernel
   float *ghat = nullptr;
   // the batched SQP in split form forms no S: each instance's rho of its last
@@ -766,8 +766,8 @@ static int build_pcg_plan(mpc_handle *h) {
     longest = std::max(longest, horizons[i]);
   }
   h->split_short = h->split_ok && longest <= pcg_split_short_knots() && (n_inst <= h->n_cu || waves <= 2u * h->n_cu);
-  h->n_split_bins = 0;
-  if (h->split_ok) {
+  h->n_split_bins = h->split_short ? n_inst : 0;  // a workgroup each, no table
+  if (h->split_ok && !h->split_short) {
     std::vector<uint32_t> all(n_inst);
     for (uint32_t i = 0; i < n_inst; ++i) all[i] = i;
     // A bin runs as long as its longest instance, and an iteration of a
@@ -1015,6 +1015,7 @@ int mpc_batch_autotune(mpc_handle *h, uint32_t iters, uint32_t reps, mpc_pcg_pla
   const bool split_cand = h->split_ok && !(h->cfg.flags & FLAG_PCG_STAIR);
   if (split_cand)
     for (uint32_t mi : {8u, 4u, 2u}) {
+      if (mi != 8 && h->split_short) continue;  // an instance per workgroup under each of them
       PcgPlan c;
       c.max_items = mi;
       c.split = true;

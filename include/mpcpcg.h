@@ -283,7 +283,8 @@ int mpc_batch_set_timing(mpc_handle *h, int enable);
  * Not used while timing is enabled.  No counterpart in the reference (its
  * SQP loop decides on the host between launches, toplevel.cuh:254-446). */
 int mpc_batch_set_graph(mpc_handle *h, int enable);
-/* PCG packing of the batch layout: out4 = {resident-kernel bins, teams
+/* PCG packing of the batch layout: out4 = {bins (workgroups) of the resident
+ * kernel or, in split form, of the split-form kernel, teams
  * (two workgroups for N <= 256, four for N <= 512), instances on the
  * streaming kernel, cooperative launches per PCG phase before the first
  * non-cooperative one (four-workgroup team launches, then the pool or the
@@ -314,7 +315,9 @@ int mpc_batch_pcg_launch_map(const mpc_handle *h, uint32_t *launch_of_inst);
  * arithmetic per instance (bins and teams: bitwise), only the packing and
  * the schedule change.  split = 1 (block Jacobi, every N <= 256): all
  * instances instead run on the split-form kernel, bins of up to max_items
- * instances on 512-lane workgroups (256 knots, one per CU); block-Jacobi
+ * instances on 512-lane workgroups (256 knots, one per CU; while the bins fit
+ * the device at once they are kept as empty as that allows), or, where every
+ * N <= 64 and the instances are few, a workgroup each; block-Jacobi
  * PCG there is CG on W^T S W (W = chol(-S(b,b))^-1 blockwise, formed with
  * the Schur block rows; in mpc_batch_sqp the regularised cost blocks are
  * inverted in closed form, Q~ being diagonal plus rank one), the same

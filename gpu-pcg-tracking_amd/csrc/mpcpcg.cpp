@@ -108,6 +108,9 @@ struct mpc_handle {
   // pinned staging for the host round trips of the plain driver
   float *h_merits = nullptr;
   uint32_t *h_pcg = nullptr;
+  // the last PCG was a plain solve's: its iterations and flag are in h_pcg, and
+  // go to pcg_iters and pcg_flag when mpc_batch_pcg_exit asks for them
+  bool plain_exit = false;
   float *h_rho = nullptr;
   // batch layout
   std::vector<uint32_t> horizons, k0;
@@ -633,6 +636,7 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
     HIP_TRY(hipEventRecord(h->ev[0], st));
     HIP_TRY(pcg_single(h, N, h->S, h->P, h->gamma, d_lambda, sqp_pcg_cap(cfg), cfg.pcg_exit_tol, h->h_pcg,
                        h->h_pcg + 1, st));
+    h->plain_exit = true;
     HIP_TRY(hipEventRecord(h->ev[1], st));
     HIP_TRY(launch_compute_dz(b, h->Ginv, h->C, h->g, d_lambda, nullptr, h->dz, st));
     if (cfg.flags & FLAG_DIRECT_SOLVE) {
@@ -1097,6 +1101,11 @@ int mpc_batch_pcg_exit(mpc_handle *h, uint32_t *d_iters, uint32_t *d_flags, floa
   if (!h->batch_ready) return MPC_ERR_NOT_READY;
   hipStream_t st = (hipStream_t)stream;
   const size_t n = h->n_inst;
+  if (h->plain_exit) {
+    HIP_TRY(hipMemcpyAsync(h->pcg_iters, h->h_pcg, sizeof(uint32_t), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(h->pcg_flag, h->h_pcg + 1, sizeof(uint32_t), hipMemcpyHostToDevice, st));
+    h->plain_exit = false;
+  }
   if (d_iters) HIP_TRY(hipMemcpyAsync(d_iters, h->pcg_iters, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
   if (d_flags) HIP_TRY(hipMemcpyAsync(d_flags, h->pcg_flag, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
   if (d_eta) HIP_TRY(hipMemcpyAsync(d_eta, h->pcg_eta, sizeof(float) * n, hipMemcpyDeviceToDevice, st));
@@ -1132,6 +1141,7 @@ int mpc_batch_phase_times(mpc_handle *h, double *us7) {
 static hipError_t pcg_batch(mpc_handle *h, float *d_lambda, const uint32_t *d_status, uint32_t max_iter, float tol,
                             hipEvent_t mid, hipStream_t st, bool prepped) {
   const Batch b = batch_of(h);
+  h->plain_exit = false;
   hipError_t e;
   if (split_active(h)) {
     // block Jacobi in split form: the split system from S and gamma (unless
@@ -1271,6 +1281,7 @@ int mpc_batch_sqp(mpc_handle *h, float *d_xu, float *d_lambda, const float *d_ee
   if (sqp_iters > MPC_MAX_SQP_ITERS) return MPC_ERR_ARG;
   for (double &v : h->phase_us) v = 0;
   if (h->graph_on && !h->timing) {
+    h->plain_exit = false;  // (a replay does not come by pcg_batch)
     mpc_handle::GraphKey k;
     k.epoch = h->graph_epoch;
     k.sqp_iters = sqp_iters;

@@ -68,6 +68,7 @@ struct mpc_handle {
   float *rho_used = nullptr;
   bool schur_formed = true;  // the last batched solve left S and gamma in the workspace
   bool gc_compact = false;   // its linearisation left G and C in the compact form (gq, Cl)
+  bool batch_blocks = false;  // the workspace's blocks are a batched solve's
   // PCG teams: two workgroups for 128 < N <= 256, four for 256 < N <= 512
   uint32_t *team_list = nullptr, *team_one = nullptr, *team_err = nullptr;
   uint32_t *pcg_done = nullptr;       // [B] parts that finished each team solve
@@ -604,18 +605,21 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
   HIP_TRY(launch_merit_reduce(b, h->knot_merits, 1, h->h_merits, st));
   HIP_TRY(hipEventRecord(h->ev[2], st));
   // the blocks of the current iterate, which change nothing of the caller's:
-  // the first iteration's are formed while the host waits for the merit
+  // the first iteration's are formed while the host waits for the merit (not
+  // over those of a batched solve, which a solve that ends here leaves to
+  // mpc_batch_direct_resolve)
   auto form_blocks = [&](bool kkt, bool schur) {
     hipError_t e = hipSuccess;
     if (kkt) {
       e = launch_form_kkt(b, prm, d_xu, d_ee_ref, h->xs, nullptr, h->G, h->C, h->g, h->c, st);
-      h->gc_compact = false;  // G and C written in full
+      h->gc_compact = h->batch_blocks = false;  // G and C written in full
     }
     if (e == hipSuccess && schur)
       e = launch_form_schur(b, h->G, h->C, h->g, h->c, nullptr, *rho, nullptr, h->S, h->P, h->gamma, h->Ginv, 0, st);
     return e;
   };
-  if (cfg.sqp_max_iter > 0) HIP_TRY(form_blocks(true, true));
+  const bool ahead = cfg.sqp_max_iter > 0 && !h->batch_blocks;
+  if (ahead) HIP_TRY(form_blocks(true, true));
   HIP_TRY(hipEventSynchronize(h->ev[2]));
   float merit0 = h->h_merits[0];
   if (!std::isfinite(merit0)) {  // nothing a line search could improve on
@@ -629,9 +633,9 @@ int mpc_sqp_solve(mpc_handle *h, uint32_t N, const float *d_ee_ref, float *d_lam
   bool not_aborted = true;
   bool time_exit = false;
   for (uint32_t it = 0; it < cfg.sqp_max_iter; ++it) {
-    if (it > 0) HIP_TRY(form_blocks(true, false));
+    if (it > 0 || !ahead) HIP_TRY(form_blocks(true, false));
     if ((time_exit = over_budget())) break;  // toplevel.cuh:271
-    if (it > 0) HIP_TRY(form_blocks(false, true));
+    if (it > 0 || !ahead) HIP_TRY(form_blocks(false, true));
     if ((time_exit = over_budget())) break;  // toplevel.cuh:283
     HIP_TRY(hipEventRecord(h->ev[0], st));
     HIP_TRY(pcg_single(h, N, h->S, h->P, h->gamma, d_lambda, sqp_pcg_cap(cfg), cfg.pcg_exit_tol, h->h_pcg,
@@ -1142,6 +1146,7 @@ static hipError_t pcg_batch(mpc_handle *h, float *d_lambda, const uint32_t *d_st
                             hipEvent_t mid, hipStream_t st, bool prepped) {
   const Batch b = batch_of(h);
   h->plain_exit = false;
+  h->batch_blocks = true;
   hipError_t e;
   if (split_active(h)) {
     // block Jacobi in split form: the split system from S and gamma (unless
@@ -1282,6 +1287,7 @@ int mpc_batch_sqp(mpc_handle *h, float *d_xu, float *d_lambda, const float *d_ee
   for (double &v : h->phase_us) v = 0;
   if (h->graph_on && !h->timing) {
     h->plain_exit = false;  // (a replay does not come by pcg_batch)
+    h->batch_blocks = true;
     mpc_handle::GraphKey k;
     k.epoch = h->graph_epoch;
     k.sqp_iters = sqp_iters;

@@ -58,3 +58,30 @@ def test_exit_state_is_the_last_solves(pkg, orc, graph):
         assert all(np.array_equal(a, b) for a, b in zip(before, last))
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("split", [0, 1])
+def test_failed_plain_solve_leaves_the_batch_systems(pkg, orc, split):
+    """A plain solve that ends at its first merit (a reference that is not
+    finite) has solved nothing: the last batch's systems are still there."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    horizons = [64, 32]
+    s = pkg.Solver(pkg.default_config(max_knots=64, max_instances=2, max_total_knots=128, sqp_max_iter=2))
+    try:
+        s.batch_set_plan(split=split)
+        _, ee, xu = helpers.make_instance(orc, 5700, 64)
+        s.sqp_solve(64, _dev(ee), torch.zeros(14 * 64, device="cuda"), _dev(xu), 1e-3)
+        _batch_sqp(pkg, orc, s, horizons, 5800, 2)
+        lam = [torch.zeros(14 * sum(horizons), device="cuda") for _ in range(3)]
+        s.batch_direct_resolve(lam[0], refine=2)
+        bad = torch.full((6 * 64,), float("nan"), device="cuda")
+        for k in (1, 2):
+            with pytest.raises(pkg.MpcError):
+                s.sqp_solve(64, bad, torch.zeros(14 * 64, device="cuda"), _dev(xu), 1e-3)
+            s.batch_direct_resolve(lam[k], refine=2)
+        torch.cuda.synchronize()
+        assert torch.isfinite(lam[0]).all() and lam[0].any()
+        assert torch.equal(lam[0], lam[1]) and torch.equal(lam[0], lam[2])
+    finally:
+        s.close()

@@ -212,9 +212,10 @@ k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pi
     run = !conv && it < cap;
   } while (run);
 
+  // (without an iteration lambda is as it was; 0 * p made NaN of an infinity)
 #pragma unroll
   for (int t = 0; t < KR; ++t)
-    if (b0 + t < N && lane_ok) lambda[NX * (b0 + t) + i] = lam[t];
+    if (it > 0 && b0 + t < N && lane_ok) lambda[NX * (b0 + t) + i] = lam[t];
   if (tid == 0) {
     if (iters_out) *iters_out = it;
     if (flag_out) *flag_out = conv ? 0u : 1u;

@@ -107,7 +107,6 @@ __device__ __forceinline__ float lane_of(float v, int l) {
 
 typedef __attribute__((address_space(1))) unsigned long long MailWord;  // in global memory
 
-// tag_xor: 0, or a bit pattern that makes the tag wrong (the poison hook)
 // buffer of epoch e in the set `set` (0 or 1) of the mailbox
 __device__ __forceinline__ uint32_t mb_buf(uint32_t set, uint32_t e) { return (set << 2) | (e & 3u); }
 
@@ -157,7 +156,7 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
   static_assert(Q == 2 || Q == 4, "teams of 2 or 4 workgroups");
   const uint32_t inst = team_inst[team];
   if (status && !(status[inst] & ST_ACTIVE)) return true;  // same decision on every part
-  const uint32_t tag_xor = poison == part + 1u ? 0x80000000u : 0u;
+  const uint32_t tag_xor = poison == part + 1u ? 0x80000000u : 0u;  // makes the tags wrong (the poison hook)
   const bool lane_ok = i < (uint32_t)NX;
   const uint32_t N = inst_len(b, inst), K0 = inst_first(b, inst);
   const uint32_t chunk = (((N + Q - 1) / Q) + 3u) & ~3u;  // <= 128 for N <= 128 Q
@@ -366,10 +365,13 @@ __device__ __forceinline__ bool team_solve(uint32_t tid, uint32_t part, uint32_t
     if (lane64 == 0) atomicOr(err, 1u);
     return false;  // this part is not counted in `done`: the instance gets PCG_FLAG_FAULT
   }
+  // (without an iteration lambda is as it was; 0 * p made NaN of an infinity)
+  if (it > 0) {
 #pragma unroll
-  for (int t = 0; t < RK; ++t) {
-    const uint32_t lk = b0 + (uint32_t)t;
-    if (lk < n_own && lane_ok) lambda[(size_t)NX * (K0 + kb + lk) + i] = lam[t * 16];
+    for (int t = 0; t < RK; ++t) {
+      const uint32_t lk = b0 + (uint32_t)t;
+      if (lk < n_own && lane_ok) lambda[(size_t)NX * (K0 + kb + lk) + i] = lam[t * 16];
+    }
   }
   if (tid == 0) {
     if (part == 0) {

@@ -254,9 +254,10 @@ __device__ __forceinline__ void body(uint32_t tid, uint32_t bin, unsigned char *
   }
 
   if (!live) return;
+  // (without an iteration lambda is as it was; 0 * p made NaN of an infinity)
 #pragma unroll
   for (int t = 0; t < RK; ++t)
-    if (b0 + t < N && lane_ok) lambda[(size_t)NX * (K0 + b0 + t) + i] = lam[t];
+    if (it > 0 && b0 + t < N && lane_ok) lambda[(size_t)NX * (K0 + b0 + t) + i] = lam[t];
   if (lg == 0 && i == 0) {
     if (iters_out) iters_out[inst] = it;
     if (flag_out) flag_out[inst] = conv ? 0u : 1u;

@@ -1,12 +1,14 @@
-"""CPU: the assembly of every kernel keeps the wait states that gfx950 leaves
-to software.  The compiler keeps them for its own instructions, but does not
+"""CPU: checks of the assembly of every kernel, for what no result shows
+reliably: the wait states that gfx950 leaves to software, and spills.
+
+Wait states.  The compiler keeps them for its own instructions, but does not
 see those inside an asm statement, and may put its copies right before or
 behind one; so the whole listing is checked, along every path.
 
 Rules (wait states between the two; an instruction in between counts one, s_nop
 n counts n + 1; AMD CDNA3 ISA guide, required software wait states, and LLVM's
 GCNHazardRecognizer for gfx940 and later):
-  VALU writes a VGPR            -> DPP reads it                          2
+  VALU writes a VGPR            -> DPP or v_permlane reads it            2
                                 -> v_readlane / v_readfirstlane reads it 1
   transcendental writes a VGPR  -> other VALU reads it                   1
   VALU writes an SGPR or VCC    -> VALU reads it                         2
@@ -95,6 +97,8 @@ class Inst:
             for r in vector:
                 if self.op.startswith(("v_readlane", "v_readfirstlane")):
                     yield r, 1, False
+                if self.op.startswith("v_permlane"):
+                    yield r, 2, False
                 if not self.trans:
                     yield r, 1, True
         for r in self.mem_reads:
@@ -206,6 +210,7 @@ def _listing(src):
     ("v_readlane_b32 s4, v1, 3\n v_mov_b32_e32 v9, v8\n v_mul_f32_e32 v2, s4, v3", 1),
     ("v_readlane_b32 s4, v1, 3\n s_nop 1\n v_mul_f32_e32 v2, s4, v3", 0),
     ("v_mov_b32_e32 v1, v2\n v_readlane_b32 s4, v1, 3", 1),
+    ("v_mov_b32_e32 v1, v2\n s_nop 0\n v_permlane16_swap_b32 v3, v1", 1),
     ("v_rcp_f32_e32 v1, v2\n v_mul_f32_e32 v3, v1, v1", 1),
     ("v_rcp_f32_e32 v1, v2\n s_nop 0\n v_mul_f32_e32 v3, v1, v1", 0),
     # the write at the loop's end, the read at its start
@@ -216,15 +221,45 @@ def test_the_check_itself(code, count):
     assert len(hazards(f".type f,@function\nf:\n {code}\n s_endpgm\n")) == count
 
 
-def test_kernels_keep_the_wait_states():
+@pytest.fixture(scope="module")
+def listings():
     srcs = [s for s in recipe.sources() if s.endswith(".hip")]
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
-        listings = list(ex.map(_listing, srcs))
-    kernels, found = 0, []
-    for src, text in zip(srcs, listings):
-        kernels += text.count("\ts_endpgm")
-        found += [(os.path.basename(src), *h) for h in hazards(text)]
-    assert kernels > 30
+        out = dict(zip(map(os.path.basename, srcs), ex.map(_listing, srcs)))
+    assert sum(text.count("\ts_endpgm") for text in out.values()) > 30
+    return out
+
+
+def test_kernels_keep_the_wait_states(listings):
+    found = [(name, *h) for name, text in listings.items() for h in hazards(text)]
     for h in found[:40]:
         print(h)
     assert not found, f"{len(found)} reads too close to a write"
+
+
+def narrow_spills(text):
+    """[(line, text)] of register spills ahead of the s_or_b64 exec of their block,
+    which store the lanes of the branch that ends there and no others."""
+    found, block = [], []
+    for no, line in enumerate(text.splitlines(), 1):
+        if re.match(r"[\w.$]+:|; %bb\.", line):
+            block = []
+        if "Folded Spill" in line or ("Reload Reuse" in line and "v_accvgpr_write" in line):
+            block.append((no, line.strip()))
+        if re.match(r"\s*s_or_b64 exec, exec,", line):
+            found += block
+            block = []
+    return found
+
+
+def test_spills_store_every_lane(listings):
+    """The compiler has put the spill of a value for all lanes ahead of the end
+    of a branch that only some had taken; reloaded for the others it was
+    whatever the slot held (a team kernel then stored knots of lambda in wrong
+    places)."""
+    assert narrow_spills("; %bb.1:\n\tscratch_store_dword off, v1, off ; 4-byte Folded Spill\n"
+                         "\ts_or_b64 exec, exec, s[0:1]\n") != []
+    assert narrow_spills("; %bb.1:\n\ts_or_b64 exec, exec, s[0:1]\n"
+                         "\tscratch_store_dword off, v1, off ; 4-byte Folded Spill\n") == []
+    found = [(name, *f) for name, text in listings.items() for f in narrow_spills(text)]
+    assert not found, found

@@ -253,8 +253,8 @@ hipError_t launch_pcg_res(const Batch &b, const uint4 *items, const uint32_t *bi
                           uint32_t max_iter, float tol, const uint32_t *status, uint32_t *iters,
                           uint32_t *flag, float *eta, bool stair, hipStream_t st);
 // Block-Jacobi PCG of one instance (N <= pcg_lone_max_knots()) on one
-// workgroup laid out for latency (k_pcg_lone.hip); bitwise the results of
-// launch_pcg_res.
+// workgroup laid out for latency (k_pcg_lone.hip), tol >= 0; bitwise the
+// results of launch_pcg_res.
 hipError_t launch_pcg_lone(uint32_t N, const float *S, const float *Pinv, const float *gamma, float *lambda,
                            uint32_t max_iter, float tol, uint32_t *iters, uint32_t *flag, float *eta, hipStream_t st);
 uint32_t pcg_lone_max_knots();

@@ -49,15 +49,6 @@ struct LoneShared {
   alignas(16) float red[2][MAX_GROUPS + 4];
 };
 
-// the 16 lanes of a row, in the order of wave_sum
-__device__ __forceinline__ float row_total(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  v += dpp_f<0x140>(v);  // row_mirror
-  return v;
-}
-
 // v of rows 0 and 2 in rows 1 and 3 (which = 0), or of rows 1 and 3 in rows 0
 // and 2 (1)
 template <int which>
@@ -177,7 +168,7 @@ k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pi
 #pragma unroll
   for (int t = 0; t < KR; ++t) p[t] = lam[t];
   uint32_t it = ~0u;  // the first pass is not counted
-  float eta = 0.f, tol_i = tol;
+  float eta = 0.f;
   bool first = true, conv, run;
   do {
     group_smv<KR>(R, p, pm, pp, y);
@@ -204,18 +195,18 @@ k_pcg_lone(uint32_t N, const float *__restrict__ S, const float *__restrict__ Pi
     for (int t = 0; t < KR; ++t) p[t] = fmaf(beta, p[t], z[t]);
     pm = fmaf(beta, pm, zm);
     pp = fmaf(beta, pp, zp);
-    // tol < 0: exit relative to the first residual, |eta| < -tol |eta_0|
-    if (first && tol < 0.f) tol_i = fmaxf(-tol * fabsf(eta), FLT_MIN);
     ++it;
     first = false;
-    conv = __builtin_amdgcn_ballot_w64(fabsf(eta) < tol_i) != 0;  // eta is the same in every lane
+    conv = uniform(fabsf(eta) < tol);  // eta is the same in every lane
     run = !conv && it < cap;
   } while (run);
 
   // (without an iteration lambda is as it was; 0 * p made NaN of an infinity)
+  if (it > 0) {
 #pragma unroll
-  for (int t = 0; t < KR; ++t)
-    if (it > 0 && b0 + t < N && lane_ok) lambda[NX * (b0 + t) + i] = lam[t];
+    for (int t = 0; t < KR; ++t)
+      if (b0 + t < N && lane_ok) lambda[NX * (b0 + t) + i] = lam[t];
+  }
   if (tid == 0) {
     if (iters_out) *iters_out = it;
     if (flag_out) *flag_out = conv ? 0u : 1u;

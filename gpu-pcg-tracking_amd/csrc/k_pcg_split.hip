@@ -171,16 +171,6 @@ __device__ __forceinline__ void read_slot(float (&M)[16], const float *Sl, uint3
   }
 }
 
-// total of the 16 lanes of each row, in every lane of the row (fixed order;
-// each step adds two values in either order, so the lanes agree bitwise)
-__device__ __forceinline__ float row_total(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  v += dpp_f<0x140>(v);  // row_mirror
-  return v;
-}
-
 // (M_k^T x_k)_i for three blocks with rotated rows M_k: sum_n ror_n(m_n),
 // m_n = M[(16 - n) & 15] x, in Horner form m_0 + ror_1(m_1 + ror_1(m_2 + ...
 // + ror_1(m_15))): 16 products and 15 row_ror:1 additions per block, the

@@ -68,18 +68,25 @@ __device__ __forceinline__ void rot_mv2(const float (&Ma)[16], float xa, float &
   rot_fma15x2(ya, xa, Ma, yb, xb, Mb);
 }
 
-// wave64 sum, identical in every lane, in a fixed order: quads, eights and
-// rows by DPP, then (row0 + row1) + (row2 + row3)
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+// total of the 16 lanes of each row, in every lane of the row (fixed order;
+// each step adds two values in either order, so the lanes agree bitwise)
+__device__ __forceinline__ float row_total(float v) {
   v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
   v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
   v += dpp_f<0x141>(v);  // row_half_mirror
   v += dpp_f<0x140>(v);  // row_mirror
+  return v;
+}
+
+// wave64 sum, identical in every lane, in a fixed order: the rows, then
+// (row0 + row1) + (row2 + row3)
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row_total(v);
   const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
   const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
   const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
